@@ -3,6 +3,8 @@
 // (reactions.jl:311-460) and the pivoted dense solve (reactions.jl:463-503).
 #pragma once
 
+#include <utility>
+
 #include "f3d_internal.h"
 
 namespace f3d {
@@ -19,10 +21,10 @@ namespace f3d {
 // relative) in Horner form with fma; 2^k by ldexp.  log: x = m 2^e with m in
 // [sqrt(1/2), sqrt(2)), log m = 2 atanh(s), s = (m - 1)/(m + 1) (|s| <= 0.172),
 // by its series to s^21 (remainder < 1e-18).
+// The special cases (NaN, overflow, underflow, zero, negative, infinite
+// arguments) are selects on the result, not branches: a wave carries one
+// straight line of arithmetic through the rate evaluation.
 __device__ inline double f3d_exp(double x) {
-  if (x != x) return x;
-  if (x > 709.782712893384) return __builtin_inf();
-  if (x < -745.1332191019412) return 0.0;
   const double kd = floor(x * 1.4426950408889634 + 0.5);
   const double r = (x - kd * 6.93147180369123816490e-01) - kd * 1.90821492927058770002e-10;
   double p = 1.0 / 6227020800.0;  // 1/13!
@@ -39,18 +41,17 @@ __device__ inline double f3d_exp(double x) {
   p = fma(p, r, 0.5);
   p = fma(p, r, 1.0);
   p = fma(p, r, 1.0);
-  return ldexp(p, (int)kd);
+  p = ldexp(p, (int)kd);
+  p = x > 709.782712893384 ? __builtin_inf() : p;
+  return x < -745.1332191019412 ? 0.0 : p;
 }
 
 __device__ inline double f3d_log(double x) {
-  if (!(x > 0.0)) return x == 0.0 ? -__builtin_inf() : __builtin_nan("");
-  if (x == __builtin_inf()) return x;
   int e = 0;
   double m = frexp(x, &e);  // x = m 2^e, m in [0.5, 1)
-  if (m < 0.70710678118654752440) {
-    m = m * 2.0;
-    e -= 1;
-  }
+  const bool low = m < 0.70710678118654752440;
+  m = low ? m * 2.0 : m;
+  e = low ? e - 1 : e;
   const double s = (m - 1.0) / (m + 1.0);
   const double z = s * s;
   double p = 1.0 / 21.0;
@@ -65,7 +66,9 @@ __device__ inline double f3d_log(double x) {
   p = fma(p, z, 1.0 / 3.0);
   p = fma(p, z, 1.0);
   const double ed = (double)e;
-  return ed * 6.93147180369123816490e-01 + (ed * 1.90821492927058770002e-10 + (2.0 * s) * p);
+  double v = ed * 6.93147180369123816490e-01 + (ed * 1.90821492927058770002e-10 + (2.0 * s) * p);
+  v = x == __builtin_inf() ? x : v;
+  return x > 0.0 ? v : (x == 0.0 ? -__builtin_inf() : __builtin_nan(""));
 }
 
 __device__ inline double f3d_log10(double x) { return f3d_log(x) * 0.43429448190325182765; }
@@ -119,11 +122,13 @@ struct KinRT {
   __device__ double ef(int n, int m) const { return P->ef[n][m]; }
   __device__ double loP(int n, int k) const { return P->loP[n][k]; }
   __device__ double Troe(int n, int k) const { return P->Troe[n][k]; }
+  __device__ static constexpr bool inert(int) { return false; }  // not known at compile time
 };
 template <class T>
 struct KinCT {
   __device__ explicit constexpr KinCT(const DevParams*) {}
   static constexpr bool kConst = true;
+  static constexpr int kNr = T::NR;
   __device__ constexpr int nr() const { return T::NR; }
   __device__ constexpr int rtype(int n) const { return T::rtype[n]; }
   __device__ constexpr int sgm(int n) const { return T::sgm[n]; }
@@ -133,19 +138,28 @@ struct KinCT {
   __device__ constexpr double ef(int n, int m) const { return T::ef[n][m]; }
   __device__ constexpr double loP(int n, int k) const { return T::loP[n][k]; }
   __device__ constexpr double Troe(int n, int k) const { return T::Troe[n][k]; }
+  // species m is produced and consumed by no reaction
+  __device__ static constexpr bool inert(int m) {
+    for (int n = 0; n < T::NR; ++n)
+      if (T::vf[n][m] != T::vr[n][m]) return false;
+    return true;
+  }
 };
 
-// for (n = 0; n < K.nr(); ++n) body(n): unrolled for compile-time tables
+// body(n) for every reaction n, in order.  With compile-time tables n is an
+// integral constant, one instantiation of the body per reaction: an unroll
+// pragma gives up on a body of this size and leaves a run-time loop that reads
+// and tests the stoichiometry.
+template <class K, class F, int... N>
+__device__ __forceinline__ void for_reactions_ct(F&& body, std::integer_sequence<int, N...>) {
+  // one reaction at a time: interleaving the unrolled reactions would hold
+  // several reactions' temporaries next to the Jacobian
+  ((body(std::integral_constant<int, N>{}), __builtin_amdgcn_sched_barrier(0)), ...);
+}
 template <class K, class F>
 __device__ __forceinline__ void for_reactions(const K& Kp, F&& body) {
   if constexpr (K::kConst) {
-#pragma unroll
-    for (int n = 0; n < Kp.nr(); ++n) {
-      body(n);
-      // one reaction at a time: interleaving the unrolled reactions would
-      // hold several reactions' temporaries next to the Jacobian
-      __builtin_amdgcn_sched_barrier(0);
-    }
+    for_reactions_ct<K>(body, std::make_integer_sequence<int, K::kNr>{});
   } else {
     const int Nr = Kp.nr();
     for (int n = 0; n < Nr; ++n) body(n);
@@ -198,7 +212,7 @@ __device__ inline void production_rate(const DevParams* __restrict__ P, const do
       for (int l = 0; l < NS; ++l) A[l][m] = 0.0;
     }
   }
-  for_reactions(Kp, [&](const int n) {
+  for_reactions(Kp, [&](const auto n) __attribute__((always_inline)) {
     const double kf = Kp.Arr(n, 0) * f3d_exp(Kp.Arr(n, 1) * lgT - Kp.Arr(n, 2) * invT);
     double dg = 0;
 #pragma unroll
@@ -372,7 +386,7 @@ __device__ inline void production_rate_block3(const DevParams* __restrict__ P, c
 #pragma unroll
     for (int i = 0; i < 3; ++i) M[i][j] = 0.0;
   }
-  for_reactions(Kp, [&](const int n) {
+  for_reactions(Kp, [&](const auto n) __attribute__((always_inline)) {
     const double kf = Kp.Arr(n, 0) * f3d_exp(Kp.Arr(n, 1) * lgT - Kp.Arr(n, 2) * invT);
     double dg = 0;
 #pragma unroll
@@ -472,29 +486,35 @@ __device__ inline void production_rate_block3(const DevParams* __restrict__ P, c
 }
 
 // solve, reactions.jl:463-503 (partial pivoting; row exchanges done with
-// selects so the matrix stays in registers, skipped for a column where no
-// lane of the wave exchanges rows).  Only the columns >= k that the back
-// substitution reads are eliminated; they are bit-identical to the
-// reference's full-row update.  RCP (Newton mode): each row's factor is
+// selects so the matrix stays in registers; the exchange with a row is
+// skipped where no lane of the wave picks that row).  Only the columns >= k
+// that the back substitution reads are eliminated; they are bit-identical to
+// the reference's full-row update.  RCP (Newton mode): each row's factor is
 // -a[i][k] times 1/a[k][k], formed once per column, instead of divided.
-template <int N, bool RCP = false>
+// UNIT (Newton mode, an inert last species, whose row of the system is a
+// unit vector): row N-2 is known to be e_{N-2}, so up to its own column it is
+// never a pivot and its elimination factors are zero; both are left out.
+template <int N, bool RCP = false, bool UNIT = false>
 __device__ inline void gauss_solve(double (&a)[N][N], double (&b)[N], double (&x)[N]) {
+  constexpr int U = UNIT ? N - 2 : -1;
 #pragma unroll
   for (int k = 0; k < N - 1; ++k) {
     double fmax_ = fabs(a[k][k]);
     int kk = k;
 #pragma unroll
     for (int i = k + 1; i < N; ++i) {
+      if (i == U) continue;
       const double absa = fabs(a[i][k]);
       if (absa > fmax_) {
         fmax_ = absa;
         kk = i;
       }
     }
-    if (__any(kk != k)) {
 #pragma unroll
-      for (int i = k + 1; i < N; ++i) {
-        const bool sw = (kk == i);
+    for (int i = k + 1; i < N; ++i) {
+      if (i == U) continue;
+      const bool sw = (kk == i);
+      if (__any(sw)) {
 #pragma unroll
         for (int j = k; j < N; ++j) {
           const double t = a[k][j];
@@ -509,6 +529,7 @@ __device__ inline void gauss_solve(double (&a)[N][N], double (&b)[N], double (&x
     const double inv = RCP ? 1.0 / a[k][k] : 0.0;
 #pragma unroll
     for (int i = k + 1; i < N; ++i) {
+      if (i == U) continue;
       const double f = RCP ? -a[i][k] * inv : -a[i][k] / a[k][k];
 #pragma unroll
       for (int j = k + 1; j < N; ++j) a[i][j] += f * a[k][j];
