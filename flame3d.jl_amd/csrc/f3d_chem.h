@@ -87,21 +87,47 @@ __device__ inline double ipow(double x, int n) {
   return r;
 }
 
-// gibbs, thermo.jl:163-191 (g/RT)
-template <int NS>
-__device__ inline void gibbs(const DevParams* __restrict__ P, double T, double lgT, double invT,
-                             double* gi) {
-  const double mlogT = 1 - lgT;
-  const double T1 = 0.5 * T;
-  const double T2 = 1.0 / 6.0 * T * T;
-  const double T3 = T1 * T2;
-  const double T4 = 1.8 * T2 * T2;
-#pragma unroll
-  for (int n = 0; n < NS; ++n) {
-    const double* c = (T < P->sep[n]) ? P->lo[n] : P->hi[n];
-    gi[n] = c[0] * mlogT - c[1] * T1 - c[2] * T2 - c[3] * T3 - c[4] * T4 + c[5] * invT - c[6];
+// g/RT (gibbs, thermo.jl:163-191) and h/RT of a species at T (NASA-7)
+struct GibbsT {
+  double mlogT, T1, T2, T3, T4, invT;
+  __device__ GibbsT(double T, double lgT, double iT) {
+    mlogT = 1 - lgT;
+    T1 = 0.5 * T;
+    T2 = 1.0 / 6.0 * T * T;
+    T3 = T1 * T2;
+    T4 = 1.8 * T2 * T2;
+    invT = iT;
   }
-}
+  __device__ double g(const NasaSet& q) const {
+    return q.c0 * mlogT - q.c1 * T1 - q.c2 * T2 - q.c3 * T3 - q.c4 * T4 + q.c5 * invT - q.c6;
+  }
+};
+struct EnthalpyT {
+  double T1, T2, T3, T4, invT;
+  __device__ EnthalpyT(double T, double iT) {
+    T1 = 0.5 * T;
+    T2 = 1.0 / 3.0 * T * T;
+    T3 = 0.25 * T * T * T;
+    T4 = 0.2 * T * T * T * T;
+    invT = iT;
+  }
+  __device__ double h(const NasaSet& q) const {
+    return q.c0 + q.c1 * T1 + q.c2 * T2 + q.c3 * T3 + q.c4 * T4 + q.c5 * invT;
+  }
+};
+// the species' g/RT in registers (no h/RT: for rates without the T column)
+template <int NS>
+struct GibbsReg {
+  double v[NS];
+  __device__ GibbsReg(const NasaTab<NS>& N, const DevParams* __restrict__ P, double T, double lgT,
+                      double invT) {
+    const GibbsT G(T, lgT, invT);
+#pragma unroll
+    for (int n = 0; n < NS; ++n) v[n] = G.g(N.at(n, T, P->sep[n]));
+  }
+  __device__ double g(int m) const { return v[m]; }
+  __device__ double h(int) const { return 0.0; }
+};
 
 // Reaction parameters of the rate evaluation.  KinRT reads them from the
 // uniform parameter block (any mechanism: scalar loads and wave-uniform
@@ -179,26 +205,14 @@ __device__ __forceinline__ void for_reactions(const K& Kp, F&& body) {
 // and of F through Fcent(T) and Pr(T).
 // RCP (Newton mode): the reverse rate constant as kf (RsT)^-sgm exp(-dg)
 // with 1/RsT formed once, instead of kf / Kc per reaction.
+// th: the species' g/RT and (TDER) h/RT at T.
 template <int NS, bool JAC, bool FULL = false, int NA = NS, bool TDER = false, bool RCP = false,
-          class K = KinRT>
+          class K = KinRT, class TH>
 __device__ inline void production_rate(const DevParams* __restrict__ P, const double* sc, double T,
-                                       double (&A)[NA][NA], double* wdot) {
+                                       double lgT, double invT, const TH& th, double (&A)[NA][NA],
+                                       double* wdot) {
   const K Kp(P);
-  const double lgT = f3d_log(T);
-  const double invT = 1.0 / T;
-  double gi[NS];
-  gibbs<NS>(P, T, lgT, invT, gi);
-  double hRT[TDER ? NS : 1];  // h/RT of each species (NASA-7), for d ln Kc / dT
   if (TDER) {
-    const double T1 = 0.5 * T;
-    const double T2 = 1.0 / 3.0 * T * T;
-    const double T3 = 0.25 * T * T * T;
-    const double T4 = 0.2 * T * T * T * T;
-#pragma unroll
-    for (int n = 0; n < NS; ++n) {
-      const double* c = (T < P->sep[n]) ? P->lo[n] : P->hi[n];
-      hRT[n] = c[0] + c[1] * T1 + c[2] * T2 + c[3] * T3 + c[4] * T4 + c[5] * invT;
-    }
 #pragma unroll
     for (int l = 0; l < NS; ++l) A[l][NA - 1] = 0.0;
   }
@@ -216,7 +230,8 @@ __device__ inline void production_rate(const DevParams* __restrict__ P, const do
     const double kf = Kp.Arr(n, 0) * f3d_exp(Kp.Arr(n, 1) * lgT - Kp.Arr(n, 2) * invT);
     double dg = 0;
 #pragma unroll
-    for (int m = 0; m < NS; ++m) dg += gi[m] * (double)(Kp.vf(n, m) - Kp.vr(n, m));
+    for (int m = 0; m < NS; ++m)
+      if (!K::kConst || Kp.vf(n, m) != Kp.vr(n, m)) dg += th.g(m) * (double)(Kp.vf(n, m) - Kp.vr(n, m));
     double kr;  // reverse rate constant kf / Kc, Kc = (RsT)^sgm exp(dg)
     if (RCP) {
       const int sg = Kp.sgm(n);
@@ -330,7 +345,8 @@ __device__ inline void production_rate(const DevParams* __restrict__ P, const do
     if (TDER) {
       double dgs = 0.0;  // sum_m (nu_f - nu_r)_m d(g_m/RT)/dT = -sum_m nu_m h_m/RT / T
 #pragma unroll
-      for (int m = 0; m < NS; ++m) dgs += hRT[m] * (double)(Kp.vf(n, m) - Kp.vr(n, m));
+      for (int m = 0; m < NS; ++m)
+        if (!K::kConst || Kp.vf(n, m) != Kp.vr(n, m)) dgs += th.h(m) * (double)(Kp.vf(n, m) - Kp.vr(n, m));
       const double dlnkf = Kp.Arr(n, 1) * invT + Kp.Arr(n, 2) * invT * invT;
       const double dlnKc = (double)Kp.sgm(n) * invT - dgs * invT;
       const double dqT = q_f * (dlnkf + dlnfac) - q_r * (dlnkf - dlnKc + dlnfac);
@@ -358,6 +374,17 @@ __device__ inline void production_rate(const DevParams* __restrict__ P, const do
   });
 }
 
+// the same with the species' g/RT evaluated here, in registers
+template <int NS, bool JAC, class K = KinRT>
+__device__ inline void production_rate_at(const NasaTab<NS>& N, const DevParams* __restrict__ P,
+                                          const double* sc, double T, double (&A)[NS][NS],
+                                          double* wdot) {
+  const double lgT = f3d_log(T);
+  const double invT = 1.0 / T;
+  const GibbsReg<NS> th(N, P, T, lgT, invT);
+  production_rate<NS, JAC, false, NS, false, false, K>(P, sc, T, lgT, invT, th, A, wdot);
+}
+
 // Production rates (as production_rate without the Jacobian) together with
 // the 3x3 block M[i][j] = d wdot_{ci} / d c_{cj} over three chosen species
 // (ci < 0: unused row/column, left zero): exact mass-action derivatives
@@ -365,14 +392,15 @@ __device__ inline void production_rate(const DevParams* __restrict__ P, const do
 // falloff rates with the falloff factor held fixed (the Lindemann part).
 // One pass over the reactions: the transcendentals are shared with wdot.
 template <int NS, class K = KinRT>
-__device__ inline void production_rate_block3(const DevParams* __restrict__ P, const double* sc,
+__device__ inline void production_rate_block3(const NasaTab<NS>& N,
+                                              const DevParams* __restrict__ P, const double* sc,
                                               double T, const int (&ci)[3], double* wdot,
                                               double (&M)[3][3]) {
   const K Kp(P);
   const double lgT = f3d_log(T);
   const double invT = 1.0 / T;
-  double gi[NS], cc[3];
-  gibbs<NS>(P, T, lgT, invT, gi);
+  double cc[3];
+  const GibbsReg<NS> th(N, P, T, lgT, invT);
   const double RsT = P->Ru / P->atm * 1e6 * T;
   const double iRsT = 1.0 / RsT;
 #pragma unroll
@@ -390,7 +418,8 @@ __device__ inline void production_rate_block3(const DevParams* __restrict__ P, c
     const double kf = Kp.Arr(n, 0) * f3d_exp(Kp.Arr(n, 1) * lgT - Kp.Arr(n, 2) * invT);
     double dg = 0;
 #pragma unroll
-    for (int m = 0; m < NS; ++m) dg += gi[m] * (double)(Kp.vf(n, m) - Kp.vr(n, m));
+    for (int m = 0; m < NS; ++m)
+      if (!K::kConst || Kp.vf(n, m) != Kp.vr(n, m)) dg += th.g(m) * (double)(Kp.vf(n, m) - Kp.vr(n, m));
     const int sg = Kp.sgm(n);  // kr = kf / Kc, Kc = (RsT)^sgm exp(dg), with 1/RsT formed once
     const double kr = kf * ((sg > 0 ? ipow(iRsT, sg) : ipow(RsT, -sg)) * f3d_exp(-dg));
     // q_f, q_r: the full mass-action products (same order as production_rate,

@@ -197,77 +197,164 @@ __device__ inline void h_specs(const DevParams* P, R T, R* h) {
   }
 }
 
-// ei_specs, thermo.jl:136-160 and InternalEnergy, thermo.jl:219-228 (FP64).
-// RCP: rho_k e_k times 1/W_k instead of divided by W_k (one rounding
-// differs; the Newton chemistry and the warm-started e -> T use it).
+// NASA-7 fits of the species, staged in LDS by each block that evaluates
+// energies or heat capacities per lane.  A lane reads the set of its side of
+// the breakpoint at its own offset: two distinct addresses per wave, 80 bytes
+// apart, so both are read without bank conflicts, as 16-byte reads.  (From the
+// parameter block the set is either two branches of scalar loads per species,
+// each waited for, or a per-lane pointer into global memory.)  Entries that
+// are functions of the parameters alone are formed once per block, with the
+// operations the per-cell formulas had.  With div_const below: point-implicit
+// air step 150x75x50 119.8 -> 90.4 us, three FP32 stage ends 256x192x128 2.62
+// -> 2.11 ms, surrogate step 192x128x128 3.93 -> 3.52 ms.
+struct NasaSet {
+  double c0m1, c1, c2, c3, c4;  // a1 - 1, a2 .. a5
+  double d5;                    // 0 below the breakpoint, a6(high) - a6(low) above
+  double c0, c5, c6, pad;       // a1, a6, a7
+};
+template <int NS>
+struct NasaTab {
+  NasaSet s[NS][2];         // [species][0 below, 1 above the breakpoint]
+  double emin[NS], emax[NS];  // e_k W_k / Ru at min_temp, max_temp
+  double as[NS];            // (a1(low) - 1) Ru / W_k
+
+  // by every thread of the block, before any of them leaves the kernel
+  __device__ void fill(const DevParams* __restrict__ P) {
+    for (int i = threadIdx.x; i < 2 * NS; i += blockDim.x) {
+      const int n = i >> 1;
+      const double* c = (i & 1) ? P->hi[n] : P->lo[n];
+      NasaSet& q = s[n][i & 1];
+      q.c0m1 = c[0] - 1;
+      q.c1 = c[1];
+      q.c2 = c[2];
+      q.c3 = c[3];
+      q.c4 = c[4];
+      q.d5 = (i & 1) ? c[5] - P->lo[n][5] : 0.0;
+      q.c0 = c[0];
+      q.c5 = c[5];
+      q.c6 = c[6];
+    }
+    __syncthreads();
+    for (int n = threadIdx.x; n < NS; n += blockDim.x) {
+      emin[n] = energy_poly(n, P->min_temp, P->sep[n]);
+      emax[n] = energy_poly(n, P->max_temp, P->sep[n]);
+      as[n] = s[n][0].c0m1 * P->Ru / P->mw[n];
+    }
+    __syncthreads();
+  }
+  __device__ const NasaSet& at(int n, double T, double sep) const { return s[n][T < sep ? 0 : 1]; }
+  // ei_specs, thermo.jl:136-160: e W / Ru of species n
+  __device__ double energy_poly(int n, double T, double sep) const {
+    const double T2 = 0.5 * T * T;
+    const double T3 = 2.0 / 3.0 * T2 * T;
+    const double T4 = T2 * T2;
+    const double T5 = 0.8 * T4 * T;
+    const NasaSet& q = at(n, T, sep);
+    return q.c0m1 * T + q.c1 * T2 + q.c2 * T3 + q.c3 * T4 + q.c4 * T5 + q.d5;
+  }
+};
+
+// a / b for a constant b > 0 of the parameter block with rb = 1 / b rounded:
+// one Newton correction of a rb by its exact remainder, four instructions of
+// full rate instead of a division's eleven.  The result is the rounded
+// quotient unless that lies within 2^-51 ulp of a rounding boundary (or a is
+// so small that the remainder is subnormal).
+__device__ __forceinline__ double div_const(double a, double b, double rb) {
+  const double q = a * rb;
+  return fma(fma(-q, b, a), rb, q);
+}
+
+// InternalEnergy, thermo.jl:219-228, and CV, thermo.jl:194-203 (FP64), at the
+// same temperature.  RCP: rho_k e_k times 1/W_k instead of divided by W_k (one
+// rounding differs; the Newton chemistry and the warm-started e -> T use it).
 template <int NS, bool RCP = false>
-__device__ inline double internal_energy(const DevParams* P, double T, const double* rhoi) {
+__device__ inline void energy_cv(const NasaTab<NS>& N, const DevParams* P, double T,
+                                 const double* rhoi, double& e_out, double& cv_out) {
   const double T2 = 0.5 * T * T;
   const double T3 = 2.0 / 3.0 * T2 * T;
   const double T4 = T2 * T2;
   const double T5 = 0.8 * T4 * T;
-  double result = 0;
+  const double S2 = T * T;
+  const double S3 = S2 * T;
+  const double S4 = S2 * S2;
+  double es = 0, cs = 0;
 #pragma unroll
   for (int n = 0; n < NS; ++n) {
-    const double* lo = P->lo[n];
-    const double* hc = P->hi[n];
-    double e;
-    if (T < P->sep[n]) {
-      e = (lo[0] - 1) * T + lo[1] * T2 + lo[2] * T3 + lo[3] * T4 + lo[4] * T5;
-    } else {
-      e = (hc[0] - 1) * T + hc[1] * T2 + hc[2] * T3 + hc[3] * T4 + hc[4] * T5 + (hc[5] - lo[5]);
-    }
-    result += RCP ? rhoi[n] * e * P->rmw[n] : rhoi[n] * e / P->mw[n];
+    const NasaSet& q = N.at(n, T, P->sep[n]);
+    const double e = q.c0m1 * T + q.c1 * T2 + q.c2 * T3 + q.c3 * T4 + q.c4 * T5 + q.d5;
+    const double cp = q.c0 + q.c1 * T + q.c2 * S2 + q.c3 * S3 + q.c4 * S4;
+    es += RCP ? rhoi[n] * e * P->rmw[n] : div_const(rhoi[n] * e, P->mw[n], P->rmw[n]);
+    cs += RCP ? (cp - 1) * rhoi[n] * P->rmw[n]
+              : div_const((cp - 1) * rhoi[n], P->mw[n], P->rmw[n]);
   }
-  return result * P->Ru;
+  e_out = es * P->Ru;
+  cv_out = cs * P->Ru;
 }
-
-// CV, thermo.jl:194-203 (FP64); RCP as internal_energy
 template <int NS, bool RCP = false>
-__device__ inline double cv_mix(const DevParams* P, double T, const double* rhoi) {
-  const double T2 = T * T;
-  const double T3 = T2 * T;
-  const double T4 = T2 * T2;
-  double result = 0;
-#pragma unroll
-  for (int n = 0; n < NS; ++n) {
-    const double* c = (T < P->sep[n]) ? P->lo[n] : P->hi[n];
-    const double cp = c[0] + c[1] * T + c[2] * T2 + c[3] * T3 + c[4] * T4;
-    result += RCP ? (cp - 1) * rhoi[n] * P->rmw[n] : (cp - 1) * rhoi[n] / P->mw[n];
-  }
-  return result * P->Ru;
+__device__ inline double cv_mix(const NasaTab<NS>& N, const DevParams* P, double T,
+                                const double* rhoi) {
+  double e, cv;
+  energy_cv<NS, RCP>(N, P, T, rhoi, e, cv);
+  return cv;
+}
+template <int NS, bool RCP = false>
+__device__ inline double internal_energy(const NasaTab<NS>& N, const DevParams* P, double T,
+                                         const double* rhoi) {
+  double e, cv;
+  energy_cv<NS, RCP>(N, P, T, rhoi, e, cv);
+  return e;
 }
 
-// Pmixture, thermo.jl:20-26; RCP as internal_energy
+// Pmixture, thermo.jl:20-26; RCP as energy_cv
 template <int NS, bool RCP = false>
 __device__ inline double pmixture(const DevParams* P, double T, const double* rhoi) {
   double YOW = 0;
 #pragma unroll
-  for (int n = 0; n < NS; ++n) YOW += RCP ? rhoi[n] * P->rmw[n] : rhoi[n] / P->mw[n];
+  for (int n = 0; n < NS; ++n)
+    YOW += RCP ? rhoi[n] * P->rmw[n] : div_const(rhoi[n], P->mw[n], P->rmw[n]);
   return P->Ru * T * YOW;
+}
+
+// Where GetT starts: the energies at the ends of the fits' range, the result
+// outside it (linear extrapolation), and e / A_s inside it.
+template <int NS>
+__device__ inline bool get_T_start(const NasaTab<NS>& N, const DevParams* P, double ein,
+                                   const double* rhoi, double& t1) {
+  const double tmin = P->min_temp, tmax = P->max_temp;
+  double emin = 0, emax = 0, As = 0;
+#pragma unroll
+  for (int n = 0; n < NS; ++n) {
+    emin += div_const(rhoi[n] * N.emin[n], P->mw[n], P->rmw[n]);
+    emax += div_const(rhoi[n] * N.emax[n], P->mw[n], P->rmw[n]);
+    As += N.as[n] * rhoi[n];
+  }
+  emin *= P->Ru;
+  emax *= P->Ru;
+  if (ein < emin) {
+    t1 = tmin - (emin - ein) / cv_mix<NS>(N, P, tmin, rhoi);
+    return false;
+  }
+  if (ein > emax) {
+    t1 = tmax - (emax - ein) / cv_mix<NS>(N, P, tmax, rhoi);
+    return false;
+  }
+  t1 = ein / As;
+  if (t1 < tmin || t1 > tmax) t1 = tmin + (tmax - tmin) / (emax - emin) * (ein - emin);
+  return true;
 }
 
 // GetT, thermo.jl:231-282 (FP64 Newton e -> T; tol 1e-3 K, <= 30 updates,
 // +-100 K step clamp, linear extrapolation outside [min_temp, max_temp]).
 template <int NS>
-__device__ inline double get_T(const DevParams* P, double ein, const double* rhoi, int* iters) {
+__device__ inline double get_T(const NasaTab<NS>& N, const DevParams* P, double ein,
+                               const double* rhoi) {
   const double tol = 1e-3;
-  const double tmin = P->min_temp, tmax = P->max_temp;
-  const double emin = internal_energy<NS>(P, tmin, rhoi);
-  const double emax = internal_energy<NS>(P, tmax, rhoi);
-  if (iters) *iters = 0;
-  if (ein < emin) return tmin - (emin - ein) / cv_mix<NS>(P, tmin, rhoi);
-  if (ein > emax) return tmax - (emax - ein) / cv_mix<NS>(P, tmax, rhoi);
-  double As = 0;
-#pragma unroll
-  for (int n = 0; n < NS; ++n) As += (P->lo[n][0] - 1) * P->Ru / P->mw[n] * rhoi[n];
-  double t1 = ein / As;
-  if (t1 < tmin || t1 > tmax) t1 = tmin + (tmax - tmin) / (emax - emin) * (ein - emin);
-  int it = 0;
+  double t1;
+  if (!get_T_start<NS>(N, P, ein, rhoi, t1)) return t1;
   double x1 = 0.0, x2 = 0.0;  // t1 one and two updates ago
   for (int m = 0; m < 30; ++m) {
-    const double e1 = internal_energy<NS>(P, t1, rhoi);
-    const double cv = cv_mix<NS>(P, t1, rhoi);
+    double e1, cv;
+    energy_cv<NS>(N, P, t1, rhoi, e1, cv);
     double dt = (ein - e1) / cv;
     if (dt > 100.0) {
       dt = 100.0;
@@ -283,16 +370,11 @@ __device__ inline double get_T(const DevParams* P, double ein, const double* rho
     // fits at a breakpoint, where the updates alternate across it) the rest
     // cycles with period two and the point the 30 updates end on is known:
     // the same result, bit for bit, without the remaining updates.
-    if (m >= 2 && t1 == x2) {
-      if (iters) *iters = 30;
-      return ((30 - m) % 2 == 0) ? t1 : x1;
-    }
+    if (m >= 2 && t1 == x2) return ((30 - m) % 2 == 0) ? t1 : x1;
     x2 = x1;
     x1 = t1;
     t1 += dt;
-    ++it;
   }
-  if (iters) *iters = it;
   return t1;
 }
 
@@ -309,22 +391,15 @@ __device__ inline double get_T(const DevParams* P, double ein, const double* rho
 // rounding each differs from get_T's; the cycle point it returns agrees with
 // get_T's to that rounding).
 template <int NS>
-__device__ inline double get_T_gap(const DevParams* P, double ein, const double* rhoi) {
+__device__ inline double get_T_gap(const NasaTab<NS>& N, const DevParams* P, double ein,
+                                   const double* rhoi) {
   const double tol = 1e-3;
-  const double tmin = P->min_temp, tmax = P->max_temp;
-  const double emin = internal_energy<NS>(P, tmin, rhoi);
-  const double emax = internal_energy<NS>(P, tmax, rhoi);
-  if (ein < emin) return tmin - (emin - ein) / cv_mix<NS>(P, tmin, rhoi);
-  if (ein > emax) return tmax - (emax - ein) / cv_mix<NS>(P, tmax, rhoi);
-  double As = 0;
-#pragma unroll
-  for (int n = 0; n < NS; ++n) As += (P->lo[n][0] - 1) * P->Ru / P->mw[n] * rhoi[n];
-  double t1 = ein / As;
-  if (t1 < tmin || t1 > tmax) t1 = tmin + (tmax - tmin) / (emax - emin) * (ein - emin);
+  double t1;
+  if (!get_T_start<NS>(N, P, ein, rhoi, t1)) return t1;
   double x1 = 0.0, x2 = 0.0;  // t1 one and two updates ago
   for (int m = 0; m < 30; ++m) {
-    const double e1 = internal_energy<NS, true>(P, t1, rhoi);
-    const double cv = cv_mix<NS, true>(P, t1, rhoi);
+    double e1, cv;
+    energy_cv<NS, true>(N, P, t1, rhoi, e1, cv);
     double dt = (ein - e1) / cv;
     if (dt > 100.0) {
       dt = 100.0;
@@ -357,17 +432,17 @@ __device__ inline double get_T_gap(const DevParams* P, double ein, const double*
 // of a breakpoint, the result is get_T's own end point (get_T_gap).  The
 // warm updates evaluate the energy and c_v with the reciprocal molar masses.
 template <int NS>
-__device__ inline double get_T_from(const DevParams* P, double ein, const double* rhoi,
-                                    double T_guess) {
+__device__ inline double get_T_from(const NasaTab<NS>& N, const DevParams* P, double ein,
+                                    const double* rhoi, double T_guess) {
   const double tol = 1e-3;
   const double tmin = P->min_temp, tmax = P->max_temp;
-  if (!(T_guess >= tmin && T_guess <= tmax)) return get_T<NS>(P, ein, rhoi, nullptr);
+  if (!(T_guess >= tmin && T_guess <= tmax)) return get_T<NS>(N, P, ein, rhoi);
   double t1 = T_guess;
   bool done = false;
   double dt_prev = 0.0;
   for (int m = 0; m < 30; ++m) {
-    const double e1 = internal_energy<NS, true>(P, t1, rhoi);
-    const double cv = cv_mix<NS, true>(P, t1, rhoi);
+    double e1, cv;
+    energy_cv<NS, true>(N, P, t1, rhoi, e1, cv);
     double dt = (ein - e1) / cv;
     if (dt > 100.0) {
       dt = 100.0;
@@ -382,24 +457,25 @@ __device__ inline double get_T_from(const DevParams* P, double ein, const double
     } else if (dt * dt_prev < 0.0 && fabs(dt) >= 0.5 * fabs(dt_prev)) {
       // the update flips sign without shrinking: the energy sits in the
       // jump of the NASA-7 fits at their breakpoint (no exact root)
-      return get_T_gap<NS>(P, ein, rhoi);
+      return get_T_gap<NS>(N, P, ein, rhoi);
     }
     dt_prev = dt;
     t1 += dt;
   }
-  if (!done || !(t1 >= tmin && t1 <= tmax)) return get_T<NS>(P, ein, rhoi, nullptr);
+  if (!done || !(t1 >= tmin && t1 <= tmax)) return get_T<NS>(N, P, ein, rhoi);
   // within 0.5 K of a breakpoint (the jumps of the fits are <= 0.2 K wide):
   // where the jump is narrower than the tolerance, or the fits overlap (two
   // roots), the start decides where the update stops; take get_T's end point
 #pragma unroll
   for (int n = 0; n < NS; ++n)
-    if (fabs(t1 - P->sep[n]) <= 0.5) return get_T_gap<NS>(P, ein, rhoi);
+    if (fabs(t1 - P->sep[n]) <= 0.5) return get_T_gap<NS>(N, P, ein, rhoi);
   return t1;
 }
 
 // common epilogue of eval_gpu / eval_gpu_stiff (reactions.jl:209-229, :286-306)
 template <int NS>
-__device__ inline void chem_epilogue(const DevParams* __restrict__ P, double* __restrict__ U,
+__device__ inline void chem_epilogue(const NasaTab<NS>& N, const DevParams* __restrict__ P,
+                                     double* __restrict__ U,
                                      double* __restrict__ Q, double* __restrict__ rhoi, long p,
                                      long NP, double* r, double dei) {
   U[p + 4 * NP] += dei;
@@ -414,7 +490,7 @@ __device__ inline void chem_epilogue(const DevParams* __restrict__ P, double* __
   for (int n = 0; n < NS; ++n) r[n] *= rho / sr;
   double ein = Q[p + 6 * NP];
   ein += dei;
-  const double T = fmax(get_T<NS>(P, ein, r, nullptr), kEps);
+  const double T = fmax(get_T<NS>(N, P, ein, r), kEps);
   const double pr = fmax(pmixture<NS>(P, T, r), kEps);
   Q[p + 4 * NP] = pr;
   Q[p + 5 * NP] = T;

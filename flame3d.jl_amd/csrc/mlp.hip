@@ -544,6 +544,8 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3))
               const DevParams* __restrict__ P, const NNDev* __restrict__ C, Geom g,
               const float* __restrict__ out, double* __restrict__ cand,
               int8_t* __restrict__ status) {
+  __shared__ NasaTab<NS> N;
+  N.fill(P);
   const long ncell = (long)g.Nx * g.Ny * g.Nz;
   const long id = gid();
   if (id >= ncell) return;
@@ -623,7 +625,7 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3))
     double esum = 0.0;
 #pragma unroll
     for (int n = 0; n < NS; ++n) esum += fabs(P->hfm[n] * dY[n]);
-    if (!(esum * rho <= (double)C->dT_max * cv_mix<NS, true>(P, T, r))) code = 5;
+    if (!(esum * rho <= (double)C->dT_max * cv_mix<NS, true>(N, P, T, r))) code = 5;
   }
   if (code == 1) {
     double rn[NS], dei = 0.0, sr = 0.0;
@@ -639,7 +641,7 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3))
 #pragma unroll
     for (int n = 0; n < NS; ++n) rn[n] *= rhoc / sr;
     const double ein = Q[p + 6 * NP] + dei;
-    const double Tn = fmax(get_T_from<NS>(P, ein, rn, T), kEps);
+    const double Tn = fmax(get_T_from<NS>(N, P, ein, rn, T), kEps);
 #pragma unroll
     for (int n = 0; n < NS; ++n) cand[(long)n * ncell + id] = rn[n];
     cand[(long)NS * ncell + id] = Tn;
@@ -655,6 +657,8 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))
               const DevParams* __restrict__ P, const NNDev* __restrict__ C, Geom g, double dt,
               const double* __restrict__ cand, int32_t* __restrict__ tile_count,
               int8_t* __restrict__ status) {
+  __shared__ NasaTab<NS> N;
+  N.fill(P);
   const long ncell = (long)g.Nx * g.Ny * g.Nz;
   const long id = gid();  // a wave holds the 64 cells of one tile
   const long NP = g.NP;
@@ -678,11 +682,11 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))
       for (int n = 0; n < NS; ++n) sc[n] = rn[n] * P->cmw[n];
       if (C->chain_max > 0.0f) {
         const int cidx[3] = {C->chain_idx[0], C->chain_idx[1], C->chain_idx[2]};
-        production_rate_block3<NS, K>(P, sc, Tn, cidx, wdot, Mc);
+        production_rate_block3<NS, K>(N, P, sc, Tn, cidx, wdot, Mc);
       } else {
-        production_rate<NS, false>(P, sc, Tn, Adum, wdot);
+        production_rate_at<NS, false>(N, P, sc, Tn, Adum, wdot);
       }
-      const double cvn = cv_mix<NS, true>(P, Tn, rn);
+      const double cvn = cv_mix<NS, true>(N, P, Tn, rn);
       if (res_on) {
         double rmax = 0.0, esum = 0.0;
 #pragma unroll
@@ -698,7 +702,7 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))
       if (code == 1 && C->chi_max > 0.0f) {
         double w2[NS];
         const double hT = 1e-4 * Tn;
-        production_rate<NS, false>(P, sc, Tn + hT, Adum, w2);
+        production_rate_at<NS, false>(N, P, sc, Tn + hT, Adum, w2);
         double dq = 0.0;
 #pragma unroll
         for (int n = 0; n < NS; ++n)

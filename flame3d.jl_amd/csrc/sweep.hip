@@ -954,6 +954,8 @@ __global__ void __launch_bounds__(kBlock)
                    double* __restrict__ Q, const float* __restrict__ rhs, double dt,
                    const double* __restrict__ J, const DevParams* __restrict__ P, Geom g,
                    int lin, double la, double lb) {
+  __shared__ NasaTab<NS> N;
+  N.fill(P);
   const long NC = (long)g.Nx * g.Ny * g.Nz;
   const long id = gid();
   if (id >= NC) return;
@@ -990,7 +992,7 @@ __global__ void __launch_bounds__(kBlock)
   const double vv = u[2] * rinv;
   const double ww = u[3] * rinv;
   const double ei = fmax(u[4] - 0.5 * rho * (uu * uu + vv * vv + ww * ww), kEps);
-  const double T = fmax(get_T_from<NS>(P, ei, r, Q[p + 5 * NP]), kEps);
+  const double T = fmax(get_T_from<NS>(N, P, ei, r, Q[p + 5 * NP]), kEps);
   const double pr = fmax(pmixture<NS, true>(P, T, r), kEps);
 #pragma unroll
   for (int n = 0; n < NS; ++n) rhoi[p + n * NP] = r[n];

@@ -231,6 +231,8 @@ template <int NS, bool WARM>
 __global__ void __launch_bounds__(kBlock)
     k_c2prim(double* __restrict__ U, double* __restrict__ Q, double* __restrict__ rhoi,
              const int64_t* __restrict__ tag, const DevParams* __restrict__ P, Geom g) {
+  __shared__ NasaTab<NS> N;
+  N.fill(P);
   const long id = gid();
   if (id >= (long)g.Nx * g.Ny * g.Nz) return;
   int a, b, c;
@@ -253,7 +255,7 @@ __global__ void __launch_bounds__(kBlock)
   const double v = U[p + 2 * NP] * rinv;
   const double w = U[p + 3 * NP] * rinv;
   const double ei = fmax(U[p + 4 * NP] - 0.5 * rho * (u * u + v * v + w * w), kEps);
-  const double T = fmax(WARM ? get_T_from<NS>(P, ei, r, Q[p + 5 * NP]) : get_T<NS>(P, ei, r, nullptr),
+  const double T = fmax(WARM ? get_T_from<NS>(N, P, ei, r, Q[p + 5 * NP]) : get_T<NS>(N, P, ei, r),
                        kEps);
   const double pr = fmax(pmixture<NS>(P, T, r), kEps);
 #pragma unroll
@@ -375,6 +377,8 @@ __global__ void __launch_bounds__(kBlock)
                 const R* __restrict__ Fdy, const R* __restrict__ Fdz, double dt,
                 const double* __restrict__ J, const int64_t* __restrict__ tag,
                 const DevParams* __restrict__ P, Geom g, int lin, double la, double lb) {
+  __shared__ NasaTab<NS> N;
+  N.fill(P);
   const long id = gid();
   if (id >= (long)g.Nx * g.Ny * g.Nz) return;
   int a, b, c;
@@ -443,7 +447,7 @@ __global__ void __launch_bounds__(kBlock)
   const double vv = u[2] * rinv;
   const double ww = u[3] * rinv;
   const double ei = fmax(u[4] - 0.5 * rho * (uu * uu + vv * vv + ww * ww), kEps);
-  const double T = fmax(WARM ? get_T_from<NS>(P, ei, r, Q[p + 5 * NP]) : get_T<NS>(P, ei, r, nullptr),
+  const double T = fmax(WARM ? get_T_from<NS>(N, P, ei, r, Q[p + 5 * NP]) : get_T<NS>(N, P, ei, r),
                        kEps);
   const double pr = fmax(pmixture<NS>(P, T, r), kEps);
 #pragma unroll
