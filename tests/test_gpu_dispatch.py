@@ -1,0 +1,75 @@
+"""Branches of the launch rules at the sizes where they can go wrong, against
+the FP64 oracle: boundary fills whose two faces share a launch or run in turn,
+and the marches' segment counts on blocks too small to fill the chip."""
+import numpy as np
+import pytest
+import torch
+
+from helpers import rel_err, to_np, to_torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _state(shape, m, seed=3):
+    import flame3d_amd.cases as cases
+    grid = cases.skewed_grid(*shape)
+    Q, rhoi = cases.random_state(grid, m, seed=seed, shock=True)
+    return grid, Q, rhoi
+
+
+@pytest.mark.parametrize("mech", ["air5", "h2_lidryer"])
+@pytest.mark.parametrize("kinds", [(1, 2, 2, 1, 1, 3), (3, 1, 1, 3, 2, 3), (2, 1, 0, 1, 3, 3),
+                                   (1, 1, 2, 2, 0, 0)])
+def test_fill_pairs_of_faces(mech, kinds):
+    """Every pairing of fill kinds on the smallest block (N = 4, where copy
+    sources and periodic sources are nearest the nodes the other face
+    writes); copies of values: equal bit for bit."""
+    import flame3d_amd.abi as abi
+    import flame3d_amd.mech as mm
+    from oracle import Oracle
+    m = mm.load(mech)
+    shape = (4, 5, 4)
+    grid, Q, rhoi = _state(shape, m)
+    orc, ctx = Oracle(*shape, m), abi.Context(*shape, m, "fp64")
+    inQ = [1.2, 300.0, 1.0, -2.0, 1.0e5, 310.0, 2.0e5]
+    inr = list(np.linspace(0.1, 0.2, m.Ns))
+    Qo, ro = to_np(Q), to_np(rhoi)
+    Uo = orc.prim2c(Qo)
+    Qg, rg, Ug = Q.cuda(), rhoi.cuda(), to_torch(Uo)
+    orc.fill(kinds, Qo, Uo, ro, inQ, inr)
+    ctx.set_boundary(kinds, inQ, inr)
+    ctx.fill(Qg, Ug, rg)
+    torch.cuda.synchronize()
+    for got, ref in ((Qg, Qo), (Ug, Uo), (rg, ro)):
+        assert np.array_equal(to_np(got), ref)
+    ctx.close()
+
+
+@pytest.mark.parametrize("shape", [(4, 4, 4), (65, 7, 5), (9, 33, 34), (70, 66, 9)])
+@pytest.mark.parametrize("mech", ["air5", "h2_lidryer"])
+def test_stage_on_small_and_ragged_blocks(mech, shape):
+    """One FP64 stage on blocks of one short segment, several, a remainder
+    segment and a partial wave: 1e-12 normwise per field, the FP64 path's
+    parity bar."""
+    import flame3d_amd.abi as abi
+    import flame3d_amd.cases as cases
+    import flame3d_amd.mech as mm
+    from oracle import Oracle
+    m = mm.load(mech)
+    grid, Q, rhoi = _state(shape, m, seed=8)
+    dt = cases.cfl_dt(grid, Q, 0.3)
+    kinds = (2, 2, 2, 2, 1, 1)
+    orc = Oracle(*shape, m)
+    Qo, ro = to_np(Q), to_np(rhoi)
+    U = orc.prim2c(Qo)
+    M, J = [to_np(x) for x in grid.metrics], to_np(grid.J)
+    ctx = abi.Context(*shape, m, "fp64")
+    ctx.set_metrics([x.cuda() for x in grid.metrics], grid.J.cuda())
+    ctx.set_boundary(kinds)
+    Qg, rg, Ug = Q.cuda(), rhoi.cuda(), to_torch(U)
+    orc.rk3_stage(1, U, orc.zeros(5), ro, orc.zeros(m.Ns), Qo, orc.workspace(), M, J, dt, kinds)
+    ctx.rk3_stage(1, Ug, ctx.zeros(5), rg, ctx.zeros(m.Ns), Qg, dt)
+    torch.cuda.synchronize()
+    for got, ref in ((Qg, Qo), (Ug, U), (rg, ro)):
+        assert rel_err(to_np(got), ref) < 1e-12
+    ctx.close()
