@@ -64,7 +64,8 @@ struct f3d_ctx {
   int sensor_kind = 0;  // F3D_SENSOR_PRESSURE / F3D_SENSOR_DUCROS
   int stage_kind = 0;   // F3D_STAGE_FUSED / F3D_STAGE_GRANULAR (F3D_FP32 contexts)
   int kin_table = 0;    // F3D_KIN_*: the chemistry kernels' reaction-parameter source
-  long spec_waves = 0;  // species-diffusion march waves resident on the device (0: not queried)
+  // resident blocks of the march kernels on the device (0: not queried)
+  long spec_waves = 0, visc_waves = 0, conv_blocks = 0, weno_waves = 0;
   f3d::DevParams host_params;
   f3d::DevParams* dparams = nullptr;
   // boundary fills
@@ -119,6 +120,38 @@ int hip_check(hipError_t e, const char* what);
 constexpr int kBlock = 256;
 
 inline unsigned nblocks(long n, int block = kBlock) { return (unsigned)((n + block - 1) / block); }
+
+// Segments per line of a march over nd cells or faces: n0, or more where a
+// launch of n0 `lines` blocks leaves half of the device's resident block slots
+// (cap) empty.  A march is a chain of dependent steps, so on a block too small
+// to fill the chip its time is the longest chain, and shorter segments (4 at
+// least, below which the priming rows are most of the work) run side by side
+// instead: the FP32 right-hand side of 97x61x43 cells 603 -> 265 us.  Up to
+// half full the longer segments' fewer priming rows win (256^3 viscous sweep,
+// 5 instead of 4 segments: 1 % slower).
+inline int fill_segments(int n0, long cap, long lines, int nd) {
+  const long n = cap / (lines < 1 ? 1 : lines);
+  const int most = nd / 4 < 1 ? 1 : nd / 4;
+  const int want = n > most ? most : (int)n;
+  return want >= 2 * n0 ? want : n0;
+}
+// Resident blocks of a kernel on the current device (queried once per context
+// and kernel; *slot keeps it).
+template <class K>
+inline long resident_blocks(K kernel, int threads, long* slot) {
+  if (*slot == 0) {
+    int nb = 0, ncu = 0, dev = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, reinterpret_cast<const void*>(kernel),
+                                                     threads, 0) != hipSuccess || nb < 1)
+      nb = 1;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+        ncu < 1)
+      ncu = 1;
+    *slot = (long)nb * ncu;
+  }
+  return *slot;
+}
 
 // Bijective remap of hardware block b of nb so that consecutive logical
 // blocks run on the same XCD (workgroups are dealt round-robin over the 8

@@ -333,7 +333,11 @@ int launch_weno(f3d_ctx* c, int dir, void* F, const void* phi, const void* Fp, c
   const long nf = (long)(g.Nx + (dir == 0)) * (g.Ny + (dir == 1)) * (g.Nz + (dir == 2));
   if (dir != 0) {
     const int nd = (dir == 1 ? g.Ny : g.Nz) + 1;
-    const int nseg = (nd + kMarchSeg - 1) / kMarchSeg;
+    const long cap = c->precision == F3D_FP64
+                         ? resident_blocks(&k_weno_march<double>, 64, &c->weno_waves)
+                         : resident_blocks(&k_weno_march<float>, 64, &c->weno_waves);
+    const long lines = (long)((g.Nx + 63) / 64) * (dir == 1 ? g.Nz : g.Ny) * NV;
+    const int nseg = fill_segments((nd + kMarchSeg - 1) / kMarchSeg, cap, lines, nd);
     const int seg = (nd + nseg - 1) / nseg;  // <= kMarchSeg: the branch codes fit 64 bits
     const dim3 grid((g.Nx + 63) / 64, dir == 1 ? g.Nz : g.Ny, nseg * NV);
     if (c->precision == F3D_FP64)

@@ -1019,9 +1019,11 @@ static void conv_ns(f3d_ctx* c, int dir, float* rhs, const double* Q, const doub
                        A[0], A[1], A[2], phi, c->dparams, g, acc);
   } else {
     const int nd = dir == 1 ? g.Ny : g.Nz;
-    const int nseg = (nd + kConvSeg - 1) / kConvSeg;
+    const unsigned nl = (g.Nx + 63) / 64, nt = dir == 1 ? g.Nz : g.Ny;
+    const long cap = resident_blocks(&k_sw_conv_m<NS>, 64 * (1 + (NS + 2) / 3), &c->conv_blocks);
+    const int nseg = fill_segments((nd + kConvSeg - 1) / kConvSeg, cap, (long)nl * nt, nd);
     const int seg = (nd + nseg - 1) / nseg;
-    const dim3 grid((g.Nx + 63) / 64, dir == 1 ? g.Nz : g.Ny, nseg);
+    const dim3 grid(nl, nt, (nd + seg - 1) / seg);
     hipLaunchKernelGGL((k_sw_conv_m<NS>), grid, dim3(64, 1 + (NS + 2) / 3), 0, s, rhs, Q, rhoi,
                        A[0], A[1], A[2], phi, c->dparams, g, dir, seg, acc);
   }
@@ -1034,18 +1036,7 @@ static void conv_ns(f3d_ctx* c, int dir, float* rhs, const double* Q, const doub
 // on 256 CUs) instead of 4 (4096 waves, a second round of 1024).
 template <int NS>
 static int spec_segments(f3d_ctx* c, int nd, long lines) {
-  if (c->spec_waves == 0) {
-    int nb = 0, ncu = 0, dev = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
-            &nb, reinterpret_cast<const void*>(&k_sw_spec_m<NS>), 64, 0) != hipSuccess || nb < 1)
-      nb = 1;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-        ncu < 1)
-      ncu = 1;
-    c->spec_waves = (long)nb * ncu;
-  }
-  const long cap = c->spec_waves;
+  const long cap = resident_blocks(&k_sw_spec_m<NS>, 64, &c->spec_waves);
   int best = 1;
   long bc = -1;
   for (int n = 1; n <= max(1, nd / 16); ++n) {
@@ -1056,7 +1047,7 @@ static int spec_segments(f3d_ctx* c, int nd, long lines) {
       best = n;
     }
   }
-  return best;
+  return fill_segments(best, cap, lines, nd);
 }
 
 template <int NS>
@@ -1073,8 +1064,10 @@ static void diff_ns(f3d_ctx* c, int dir, float* rhs, const double* Q, const floa
                        J, D, c->dparams, g);
   } else {
     const int nd = dir == 1 ? g.Ny : g.Nz;
-    const int nsv = (nd + kViscSeg - 1) / kViscSeg, sv = (nd + nsv - 1) / nsv;
     const unsigned nl = (g.Nx + 63) / 64, nt = dir == 1 ? g.Nz : g.Ny;
+    const long cap = resident_blocks(&k_sw_visc_m, 64, &c->visc_waves);
+    const int nsv = fill_segments((nd + kViscSeg - 1) / kViscSeg, cap, (long)nl * nt, nd);
+    const int sv = (nd + nsv - 1) / nsv;
     const int nss = spec_segments<NS>(c, nd, (long)nl * nt), ss = (nd + nss - 1) / nss;
     hipLaunchKernelGGL(k_sw_visc_m, dim3(nl, nt, nsv), dim3(64), 0, s, rhs, Q, M, J, lam, mu, g,
                        dir, sv);
