@@ -96,9 +96,12 @@ static int fill_params(DevParams& P, const f3d_dims* d, const f3d_thermo* th,
   for (int n = 0; n < d->Ns; ++n)
     for (int l = 0; l < d->Ns; ++l) {
       const double wr = P.mw[l] / P.mw[n];
-      P.wr4_f[n][l] = (float)std::sqrt(std::sqrt(wr));
-      P.c8_f[n][l] = (float)(1.0 / std::sqrt(8.0 + 8.0 / wr));
-      P.iwr_f[n][l] = (float)(1.0 / wr);
+      P.wr4[n][l] = std::sqrt(std::sqrt(wr));
+      P.c8[n][l] = 1.0 / std::sqrt(8.0 + 8.0 / wr);
+      P.iwr[n][l] = 1.0 / wr;
+      P.wr4_f[n][l] = (float)P.wr4[n][l];
+      P.c8_f[n][l] = (float)P.c8[n][l];
+      P.iwr_f[n][l] = (float)P.iwr[n][l];
     }
   for (int n = 0; n < d->Ns; ++n) {
     P.rmw[n] = 1.0 / P.mw[n];

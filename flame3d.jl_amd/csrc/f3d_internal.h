@@ -42,9 +42,10 @@ struct DevParams {
   float visc_f[MAXNS][5], cond_f[MAXNS][5], bdiff_f[MAXNS][MAXNS][5];
   float Ru_f, WENOeps_f, phi1_f, phi2_f, SWeps2_f, UP7_f[7];
   float Rmw_f[MAXNS];  // Ru / W_n rounded to float
-  // Wilke's species-pair constants for the FP32 mixture rule (W_l / W_n)^(1/4),
+  // Wilke's species-pair constants for the mixture rule: (W_l / W_n)^(1/4),
   // 1 / sqrt(8 (1 + W_n / W_l)) and W_n / W_l
   float wr4_f[MAXNS][MAXNS], c8_f[MAXNS][MAXNS], iwr_f[MAXNS][MAXNS];
+  double wr4[MAXNS][MAXNS], c8[MAXNS][MAXNS], iwr[MAXNS][MAXNS];  // the same, FP64
 };
 
 // Padded-block geometry (0-based).  Point p = i + Nxt*(j + Nyt*k); variable
@@ -186,6 +187,9 @@ struct PT<double> {
   __device__ static double sweps2(const DevParams* P) { return P->SWeps2; }
   __device__ static const double* up7(const DevParams* P) { return P->UP7; }
   __device__ static double eps() { return kEps; }
+  __device__ static double wr4(const DevParams* P, int n, int l) { return P->wr4[n][l]; }
+  __device__ static double c8(const DevParams* P, int n, int l) { return P->c8[n][l]; }
+  __device__ static double iwr(const DevParams* P, int n, int l) { return P->iwr[n][l]; }
 };
 template <>
 struct PT<float> {
@@ -205,6 +209,9 @@ struct PT<float> {
   __device__ static const float* up7(const DevParams* P) { return P->UP7_f; }
   // eps(Float64) is used as a floor in the reference; kept as the same value
   __device__ static float eps() { return (float)kEps; }
+  __device__ static float wr4(const DevParams* P, int n, int l) { return P->wr4_f[n][l]; }
+  __device__ static float c8(const DevParams* P, int n, int l) { return P->c8_f[n][l]; }
+  __device__ static float iwr(const DevParams* P, int n, int l) { return P->iwr_f[n][l]; }
 };
 
 // ---- thermo device functions (thermo.jl) -----------------------------------

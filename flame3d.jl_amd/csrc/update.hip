@@ -115,83 +115,67 @@ __device__ inline void mixture_props(const DevParams* __restrict__ P, R T, R Pr,
     mui[n] = sq * sq;
     sqi[n] = fabs(sq);
   }
-  // Wilke, Phi[n][l] (thermo.jl:321-334)
-  R phi[NS][NS];
-  if constexpr (sizeof(R) == 4) {
-    // FP32: sqrt(mu_n / mu_l) = |sq_n| / |sq_l| (mu = sq^2) and the species-pair
-    // factors precomputed, so no division or square root per pair
+  // Wilke (thermo.jl:321-334): den_n = sum_l X_l Phi[n][l] with sqrt(mu_n /
+  // mu_l) = |sq_n| / |sq_l| (mu = sq^2) and the species-pair factors
+  // precomputed, so no division or square root per pair.  Each pair adds to
+  // both species' sums as it is formed (every sum still runs over l in order),
+  // so the Ns x Ns matrix is never held.
+  R den[NS];
+  {
     R isq[NS];
 #pragma unroll
     for (int n = 0; n < NS; ++n) isq[n] = qdiv(R(1), sqi[n]);
 #pragma unroll
     for (int n = 0; n < NS; ++n) {
+      den[n] = R(0);
 #pragma unroll
       for (int l = 0; l < n; ++l) {
         const R rs = sqi[n] * isq[l];  // sqrt(vr)
-        const R f1 = R(1) + rs * P->wr4_f[n][l];
-        const R tmp = f1 * f1 * P->c8_f[n][l];
-        phi[n][l] = tmp;
+        const R f1 = R(1) + rs * PT<R>::wr4(P, n, l);
+        const R tmp = f1 * f1 * PT<R>::c8(P, n, l);
+        den[n] += X[l] * tmp;
         const R ir = sqi[l] * isq[n];  // 1 / sqrt(vr)
-        phi[l][n] = tmp * (ir * ir) * P->iwr_f[n][l];
+        den[l] += X[n] * (tmp * (ir * ir) * PT<R>::iwr(P, n, l));
       }
-      phi[n][n] = R(1);
-    }
-  } else {
+      den[n] += X[n];
+      // one species' pairs at a time (the scheduler would otherwise hold the
+      // constants and terms of many)
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int n = 0; n < NS; ++n) {
-      const R tmp1 = R(1) / PT<R>::mw(P, n);
-      const R tmp2 = mui[n];
-#pragma unroll
-      for (int l = 0; l <= n; ++l) {
-        const R wr = PT<R>::mw(P, l) * tmp1;
-        const R vr = tmp2 / mui[l];
-        const R f1 = R(1) + sqrt(vr * sqrt(wr));
-        const R tmp = f1 * f1 / sqrt(R(8) + R(8) / wr);
-        phi[n][l] = tmp;
-        phi[l][n] = tmp / (vr * wr);
-      }
-      phi[n][n] = R(1);
+      for (int l = 0; l <= n; ++l) asm volatile("" : "+v"(den[l]));
     }
   }
   R m = 0;
 #pragma unroll
-  for (int n = 0; n < NS; ++n) {
-    R tmp = 0;
-#pragma unroll
-    for (int l = 0; l < NS; ++l) tmp += X[l] * phi[n][l];
-    m += qdiv(X[n] * mui[n], tmp);
-  }
+  for (int n = 0; n < NS; ++n) m += qdiv(X[n] * mui[n], den[n]);
   mu = m;
   // binary diffusion, D_kl P = T^1.5 poly (thermo.jl:349-367)
-  const R T15 = T * sqT;
-#pragma unroll
-  for (int n = 0; n < NS; ++n) {
-#pragma unroll
-    for (int nn = n; nn < NS; ++nn) {
-      const R* p = PT<R>::bdiff(P, n, nn);
-      const R tmp = T15 * (p[0] + lgT * p[1] + lgT2 * p[2] + lgT3 * p[3] + lgT4 * p[4]);
-      // FP32: the pair's reciprocal once (the sums below multiply by it)
-      const R v = (sizeof(R) == 4) ? qdiv(R(1), tmp) : tmp;
-      phi[nn][n] = v;
-      phi[n][nn] = v;
-    }
-  }
   // D_k = (1 - X_k) / (P sum_{l!=k} X_l / D_kl + eps) with 1 - X_k taken as
   // sum_{l!=k} X_l (equal since sum X = 1): the difference 1 - X_k cancels
   // catastrophically in nearly pure cells, where the sum stays exact (a
   // binary mixture then gives D_1 = D_12 / P for any composition)
+  const R T15 = T * sqT;
+  R sd[NS], sx[NS];
+#pragma unroll
+  for (int n = 0; n < NS; ++n) sd[n] = sx[n] = R(0);
 #pragma unroll
   for (int n = 0; n < NS; ++n) {
-    R s = 0, sx = 0;
 #pragma unroll
-    for (int nn = 0; nn < NS; ++nn) {
-      if (nn == n) continue;
-      s += (sizeof(R) == 4) ? X[nn] * phi[n][nn] : X[nn] / phi[n][nn];
-      sx += X[nn];
+    for (int nn = n + 1; nn < NS; ++nn) {
+      const R* p = PT<R>::bdiff(P, n, nn);
+      const R tmp = T15 * (p[0] + lgT * p[1] + lgT2 * p[2] + lgT3 * p[3] + lgT4 * p[4]);
+      const R v = qdiv(R(1), tmp);  // the pair's reciprocal, for both sums
+      sd[n] += X[nn] * v;
+      sx[n] += X[nn];
+      sd[nn] += X[n] * v;
+      sx[nn] += X[n];
     }
-    s *= Pr;
-    Diff[n] = qdiv(sx, s + PT<R>::eps());
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int nn = 0; nn < NS; ++nn) asm volatile("" : "+v"(sd[nn]), "+v"(sx[nn]));
   }
+#pragma unroll
+  for (int n = 0; n < NS; ++n) Diff[n] = qdiv(sx[n], sd[n] * Pr + PT<R>::eps());
 }
 
 // mixture, thermo.jl:371-403 (every padded point)
@@ -212,11 +196,15 @@ __global__ void __launch_bounds__(kBlock)
   for (int n = 0; n < NS; ++n) {
     Y[n] = fmax((R)rhoi[p + (long)n * NP] * rinv, R(0));
     Yi[p + (long)n * NP] = Y[n];
-    YOW += Y[n] / PT<R>::mw(P, n);
+    if constexpr (sizeof(R) == 8)
+      X[n] = div_const(Y[n], P->mw[n], P->rmw[n]);
+    else
+      X[n] = Y[n] / PT<R>::mw(P, n);
+    YOW += X[n];
   }
   const R YOWINV = R(1) / YOW;
 #pragma unroll
-  for (int n = 0; n < NS; ++n) X[n] = Y[n] / PT<R>::mw(P, n) * YOWINV;
+  for (int n = 0; n < NS; ++n) X[n] *= YOWINV;
   R l, m;
   mixture_props<NS, R>(P, T, Pr, X, Df, l, m);
 #pragma unroll
