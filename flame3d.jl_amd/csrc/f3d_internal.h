@@ -163,6 +163,20 @@ __device__ inline unsigned xcd_remap(unsigned b, unsigned nb) {
   return base + k;
 }
 
+// Line t of an ny x nz cross-section in an order that keeps its y and z
+// neighbours close in time: slabs of kSlab z planes, y by y, z fastest inside
+// a slab.  With y fastest over a whole plane a stencil's z neighbours come
+// round again after ny lines of every field, more than an XCD's 4 MB of L2
+// holds; here after kSlab (two planes per slab edge are read twice).
+constexpr int kSlab = 16;
+__device__ inline void slab_line(int t, int ny, int nz, int& b, int& c) {
+  const int per = ny * kSlab;
+  const int sl = t / per, r = t - sl * per;
+  const int h = min(kSlab, nz - sl * kSlab);
+  b = r / h;
+  c = sl * kSlab + (r - b * h);
+}
+
 __device__ inline unsigned xcd_block() { return xcd_remap(blockIdx.x, gridDim.x); }
 
 __device__ inline long gid() { return (long)xcd_block() * blockDim.x + threadIdx.x; }
@@ -216,15 +230,17 @@ struct PT<float> {
 
 // ---- thermo device functions (thermo.jl) -----------------------------------
 
-// h_specs, thermo.jl:107-133 (J/kg)
-template <int NS, typename R>
-__device__ inline void h_specs(const DevParams* P, R T, R* h) {
-  const R T2 = R(0.5) * T * T;
-  const R T3 = R(2.0 / 3.0) * T2 * T;
-  const R T4 = T2 * T2;
-  const R T5 = R(0.8) * T4 * T;
-#pragma unroll
-  for (int n = 0; n < NS; ++n) {
+// h_specs, thermo.jl:107-133 (J/kg), species by species
+template <typename R>
+struct SpecEnthalpy {
+  R T, T2, T3, T4, T5;
+  __device__ explicit SpecEnthalpy(R t) : T(t) {
+    T2 = R(0.5) * T * T;
+    T3 = R(2.0 / 3.0) * T2 * T;
+    T4 = T2 * T2;
+    T5 = R(0.8) * T4 * T;
+  }
+  __device__ R h(const DevParams* P, int n) const {
     const R* lo = PT<R>::lo(P, n);
     const R* hc = PT<R>::hi(P, n);
     R v;
@@ -233,8 +249,14 @@ __device__ inline void h_specs(const DevParams* P, R T, R* h) {
     } else {
       v = hc[0] * T + hc[1] * T2 + hc[2] * T3 + hc[3] * T4 + hc[4] * T5 + (hc[5] - lo[5]);
     }
-    h[n] = v * PT<R>::Rmw(P, n);  // Ru / W_n (the same quotient, rounded once on the host)
+    return v * PT<R>::Rmw(P, n);  // Ru / W_n (the same quotient, rounded once on the host)
   }
+};
+template <int NS, typename R>
+__device__ inline void h_specs(const DevParams* P, R T, R* h) {
+  const SpecEnthalpy<R> H(T);
+#pragma unroll
+  for (int n = 0; n < NS; ++n) h[n] = H.h(P, n);
 }
 
 // NASA-7 fits of the species, staged in LDS by each block that evaluates

@@ -389,8 +389,9 @@ __global__ void __launch_bounds__(kBlock)
   N.fill(P);
   const long id = gid();
   if (id >= (long)g.Nx * g.Ny * g.Nz) return;
-  int a, b, c;
-  interior_idx(id, g, a, b, c);
+  const int a = (int)(id % g.Nx);
+  int b, c;
+  slab_line((int)(id / g.Nx), g.Ny, g.Nz, b, c);
   const long p = (a + NG) + (long)g.Nxt * ((b + NG) + (long)g.Nyt * (c + NG));
   if (tag && tag[p] != 0) return;
   const long NP = g.NP;

@@ -34,18 +34,25 @@ struct Metrics {
 };
 
 // viscousFlux_x/y/z, viscous.jl:1-428 (LES branches off, run.jl:7-8)
-template <typename R, typename MT>
+// Bound by the latency of its 66 stencil loads.  FP64: registers for two waves
+// per SIMD, so that the scheduler issues the loads together (with three to five
+// waves it saves registers and waits in between): 128^3, 153-168 us per launch
+// to 132-150 us, and 13.8 to 4.9 us on a 24x16x12 block.
+template <typename R, typename MT, int dir>
 __global__ void __launch_bounds__(kBlock)
+    __attribute__((amdgpu_waves_per_eu(sizeof(R) == 8 ? 2 : 1, sizeof(R) == 8 ? 2 : 8)))
     k_viscous(R* __restrict__ Fv, const double* __restrict__ Q, Metrics<MT> M,
               const MT* __restrict__ J, const R* __restrict__ lam, const R* __restrict__ mu,
-              const R* __restrict__ Fh, const int64_t* __restrict__ tag, Geom g, int dir) {
+              const R* __restrict__ Fh, const int64_t* __restrict__ tag, Geom g) {
   const int nx = g.Nx + (dir == 0), ny = g.Ny + (dir == 1), nz = g.Nz + (dir == 2);
   const long nf = (long)nx * ny * nz;
-  const long f = gid();
-  if (f >= nf) return;
-  const int a = (int)(f % nx);
-  const int tt = (int)(f / nx);
-  const int b = tt % ny, c = tt / ny;
+  const long id = gid();
+  if (id >= nf) return;
+  const int a = (int)(id % nx);
+  const int tt = (int)(id / nx);
+  int b, c;
+  slab_line(tt, ny, nz, b, c);
+  const long f = a + (long)nx * (b + (long)ny * c);
   const long ic = (a + NG) + (long)g.Nxt * ((b + NG) + (long)g.Nyt * (c + NG));
   if (tag && tag[ic] == 1) return;
   const long st[3] = {1, (long)g.Nxt, (long)g.Nxt * g.Nyt};
@@ -64,8 +71,12 @@ __global__ void __launch_bounds__(kBlock)
   for (int q = 0; q < 4; ++q) {
     const double* fq = Q + qv[q] * NP;
 #pragma unroll
-    for (int t = 0; t < 3; ++t)
-      dq[q][t] = (t == dir) ? d_normal<R>(fq, ic, s) : d_cross4<R>(fq, ic, s, st[t]);
+    for (int t = 0; t < 3; ++t) {
+      if (t == dir)
+        dq[q][t] = d_normal<R>(fq, ic, s);
+      else
+        dq[q][t] = d_cross4<R>(fq, ic, s, st[t]);
+    }
   }
   const R u = ((R)Q[im + NP] + (R)Q[ic + NP]) * R(0.5);
   const R v = ((R)Q[im + 2 * NP] + (R)Q[ic + 2 * NP]) * R(0.5);
@@ -96,23 +107,32 @@ __global__ void __launch_bounds__(kBlock)
 
 // specViscousFlux_x/y/z, viscous.jl:430-665: rho D_k = (D_{i-1} + D_i) rho_face
 // (no 1/2, viscous.jl:473), correction velocity, enthalpy flux Fh.
-template <int NS, typename R, typename MT>
+// Bound by the latency of its 14 loads per species, so by how many waves are
+// resident: the corrected velocity V_k - Y_k sum V enters the fluxes linearly,
+// so of a species only V_k . n, Y_k and two running sums (V h, Y h) are kept,
+// not its three velocity components, its enthalpy and its mass fraction until
+// the sum is known (174 VGPRs, two waves per SIMD).  128^3, 9 species, FP64:
+// 357 -> 195 us (x), 240 us (y, z: 72 % of the L1's access rate), of which the
+// slab order of the lines took the fetched bytes from 1.08 to 0.60 GB.
+template <int NS, typename R, typename MT, int DIR>
 __global__ void __launch_bounds__(kBlock)
     k_spec_viscous(R* __restrict__ Fd, const double* __restrict__ Q, const R* __restrict__ Yi,
                    Metrics<MT> M, const MT* __restrict__ J, const R* __restrict__ D,
                    R* __restrict__ Fh, const int64_t* __restrict__ tag,
-                   const DevParams* __restrict__ P, Geom g, int dir) {
-  const int nx = g.Nx + (dir == 0), ny = g.Ny + (dir == 1), nz = g.Nz + (dir == 2);
+                   const DevParams* __restrict__ P, Geom g) {
+  const int nx = g.Nx + (DIR == 0), ny = g.Ny + (DIR == 1), nz = g.Nz + (DIR == 2);
   const long nf = (long)nx * ny * nz;
-  const long f = gid();
-  if (f >= nf) return;
-  const int a = (int)(f % nx);
-  const int tt = (int)(f / nx);
-  const int b = tt % ny, c = tt / ny;
+  const long id = gid();
+  if (id >= nf) return;
+  const int a = (int)(id % nx);
+  const int tt = (int)(id / nx);
+  int b, c;
+  slab_line(tt, ny, nz, b, c);
+  const long f = a + (long)nx * (b + (long)ny * c);
   const long ic = (a + NG) + (long)g.Nxt * ((b + NG) + (long)g.Nyt * (c + NG));
   if (tag && tag[ic] == 1) return;
   const long st[3] = {1, (long)g.Nxt, (long)g.Nxt * g.Nyt};
-  const long s = st[dir];
+  const long s = st[DIR];
   const long im = ic - s;
   const long NP = g.NP;
   R m[9];
@@ -121,42 +141,53 @@ __global__ void __launch_bounds__(kBlock)
   const R Jac = ((R)J[im] + (R)J[ic]) * R(0.5);
   const R rho = ((R)Q[im] + (R)Q[ic]) * R(0.5);
   const R T = ((R)Q[im + 5 * NP] + (R)Q[ic + 5 * NP]) * R(0.5);
-  R hi[NS], Vk1[NS], Vk2[NS], Vk3[NS];
-  h_specs<NS, R>(P, T, hi);
-  R sum1 = 0, sum2 = 0, sum3 = 0;
+  const R n0 = m[3 * DIR], n1 = m[3 * DIR + 1], n2 = m[3 * DIR + 2];
+  R Vn[NS], Yn[NS];
+  R sum1 = 0, sum2 = 0, sum3 = 0;  // sum_k V_k
+  R fh1 = 0, fh2 = 0, fh3 = 0;     // sum_k V_k h_k
+  R yh = 0;                        // sum_k Y_k h_k
+  const SpecEnthalpy<R> H(T);
 #pragma unroll
   for (int n = 0; n < NS; ++n) {
     const R* y = Yi + (long)n * NP;
     const R rhoDi = (D[im + (long)n * NP] + D[ic + (long)n * NP]) * rho;
     R dY[3];
 #pragma unroll
-    for (int t = 0; t < 3; ++t) dY[t] = (t == dir) ? y_normal<R>(y, ic, s) : y_cross2<R>(y, ic, s, st[t]);
+    for (int t = 0; t < 3; ++t) {
+      if (t == DIR)
+        dY[t] = y_normal<R>(y, ic, s);
+      else
+        dY[t] = y_cross2<R>(y, ic, s, st[t]);
+    }
     const R Vx = (dY[0] * m[0] + dY[1] * m[3] + dY[2] * m[6]) * Jac * rhoDi;
     const R Vy = (dY[0] * m[1] + dY[1] * m[4] + dY[2] * m[7]) * Jac * rhoDi;
     const R Vz = (dY[0] * m[2] + dY[1] * m[5] + dY[2] * m[8]) * Jac * rhoDi;
-    Vk1[n] = Vx;
-    Vk2[n] = Vy;
-    Vk3[n] = Vz;
+    const R hk = H.h(P, n);
+    Yn[n] = R(0.5) * (y[im] + y[ic]);
+    Vn[n] = Vx * n0 + Vy * n1 + Vz * n2;
     sum1 += Vx;
     sum2 += Vy;
     sum3 += Vz;
-  }
-  const R n0 = m[3 * dir], n1 = m[3 * dir + 1], n2 = m[3 * dir + 2];
-  R fh1 = 0, fh2 = 0, fh3 = 0;
+    fh1 += Vx * hk;
+    fh2 += Vy * hk;
+    fh3 += Vz * hk;
+    yh += Yn[n] * hk;
+    if ((n + 1) % 3 == 0) {
+      // three species' loads in flight at a time (42): left alone the compiler
+      // issues all species' first and holds 126 values
+      __builtin_amdgcn_sched_barrier(0);
+      asm volatile("" : "+v"(sum1), "+v"(sum2), "+v"(sum3), "+v"(fh1), "+v"(fh2), "+v"(fh3), "+v"(yh));
+      asm volatile("" ::: "memory");
 #pragma unroll
-  for (int n = 0; n < NS; ++n) {
-    const R Yn = R(0.5) * (Yi[im + (long)n * NP] + Yi[ic + (long)n * NP]);
-    const R V1 = Vk1[n] - sum1 * Yn;
-    const R V2 = Vk2[n] - sum2 * Yn;
-    const R V3 = Vk3[n] - sum3 * Yn;
-    Fd[f + n * nf] = V1 * n0 + V2 * n1 + V3 * n2;
-    fh1 += V1 * hi[n];
-    fh2 += V2 * hi[n];
-    fh3 += V3 * hi[n];
+      for (int k = n - 2; k <= n; ++k) asm volatile("" : "+v"(Vn[k]), "+v"(Yn[k]));
+    }
   }
-  Fh[f] = fh1;
-  Fh[f + nf] = fh2;
-  Fh[f + 2 * nf] = fh3;
+  const R sn = sum1 * n0 + sum2 * n1 + sum3 * n2;
+#pragma unroll
+  for (int n = 0; n < NS; ++n) Fd[f + n * nf] = Vn[n] - sn * Yn[n];
+  Fh[f] = fh1 - sum1 * yh;
+  Fh[f + nf] = fh2 - sum2 * yh;
+  Fh[f + 2 * nf] = fh3 - sum3 * yh;
 }
 
 // ---------------------------------------------------------------------------
@@ -427,10 +458,13 @@ int launch_viscous(f3d_ctx* c, int dir, void* Fv, const double* Q, const void* c
   const Geom& g = c->g;
   const long nf = (long)(g.Nx + (dir == 0)) * (g.Ny + (dir == 1)) * (g.Nz + (dir == 2));
   const dim3 gr(nblocks(nf)), bl(kBlock);
-  if (c->precision == F3D_FP64)
-    hipLaunchKernelGGL((k_viscous<double, double>), gr, bl, 0, s, (double*)Fv, Q, mk<double>(M),
-                       (const double*)J, (const double*)lam, (const double*)mu,
-                       (const double*)Fh, tag, g, dir);
+  if (c->precision == F3D_FP64) {
+    const auto k = dir == 0   ? k_viscous<double, double, 0>
+                   : dir == 1 ? k_viscous<double, double, 1>
+                              : k_viscous<double, double, 2>;
+    hipLaunchKernelGGL(k, gr, bl, 0, s, (double*)Fv, Q, mk<double>(M), (const double*)J,
+                       (const double*)lam, (const double*)mu, (const double*)Fh, tag, g);
+  }
   else if (dir != 0) {
     dim3 mg;
     int seg;
@@ -444,13 +478,13 @@ int launch_viscous(f3d_ctx* c, int dir, void* Fv, const double* Q, const void* c
                          mk<double>(M), (const double*)J, (const float*)lam, (const float*)mu,
                          (const float*)Fh, tag, g, dir, seg);
   } else if (mf)
-    hipLaunchKernelGGL((k_viscous<float, float>), gr, bl, 0, s, (float*)Fv, Q, mk<float>(M),
+    hipLaunchKernelGGL((k_viscous<float, float, 0>), gr, bl, 0, s, (float*)Fv, Q, mk<float>(M),
                        (const float*)J, (const float*)lam, (const float*)mu, (const float*)Fh,
-                       tag, g, dir);
+                       tag, g);
   else
-    hipLaunchKernelGGL((k_viscous<float, double>), gr, bl, 0, s, (float*)Fv, Q, mk<double>(M),
+    hipLaunchKernelGGL((k_viscous<float, double, 0>), gr, bl, 0, s, (float*)Fv, Q, mk<double>(M),
                        (const double*)J, (const float*)lam, (const float*)mu, (const float*)Fh,
-                       tag, g, dir);
+                       tag, g);
   return hip_check(hipGetLastError(), "viscous_flux");
 }
 
@@ -461,10 +495,13 @@ static void spec_visc_ns(f3d_ctx* c, int dir, void* Fd, const double* Q, const v
   const Geom& g = c->g;
   const long nf = (long)(g.Nx + (dir == 0)) * (g.Ny + (dir == 1)) * (g.Nz + (dir == 2));
   const dim3 gr(nblocks(nf)), bl(kBlock);
-  if (c->precision == F3D_FP64)
-    hipLaunchKernelGGL((k_spec_viscous<NS, double, double>), gr, bl, 0, s, (double*)Fd, Q,
-                       (const double*)Yi, mk<double>(M), (const double*)J, (const double*)D,
-                       (double*)Fh, tag, c->dparams, g, dir);
+  if (c->precision == F3D_FP64) {
+    const auto k = dir == 0   ? k_spec_viscous<NS, double, double, 0>
+                   : dir == 1 ? k_spec_viscous<NS, double, double, 1>
+                              : k_spec_viscous<NS, double, double, 2>;
+    hipLaunchKernelGGL(k, gr, bl, 0, s, (double*)Fd, Q, (const double*)Yi, mk<double>(M),
+                       (const double*)J, (const double*)D, (double*)Fh, tag, c->dparams, g);
+  }
   else if (dir != 0) {
     dim3 mg;
     int seg;
@@ -478,13 +515,13 @@ static void spec_visc_ns(f3d_ctx* c, int dir, void* Fd, const double* Q, const v
                          (const float*)Yi, mk<double>(M), (const double*)J, (const float*)D,
                          (float*)Fh, tag, c->dparams, g, dir, seg);
   } else if (mf)
-    hipLaunchKernelGGL((k_spec_viscous<NS, float, float>), gr, bl, 0, s, (float*)Fd, Q,
+    hipLaunchKernelGGL((k_spec_viscous<NS, float, float, 0>), gr, bl, 0, s, (float*)Fd, Q,
                        (const float*)Yi, mk<float>(M), (const float*)J, (const float*)D,
-                       (float*)Fh, tag, c->dparams, g, dir);
+                       (float*)Fh, tag, c->dparams, g);
   else
-    hipLaunchKernelGGL((k_spec_viscous<NS, float, double>), gr, bl, 0, s, (float*)Fd, Q,
+    hipLaunchKernelGGL((k_spec_viscous<NS, float, double, 0>), gr, bl, 0, s, (float*)Fd, Q,
                        (const float*)Yi, mk<double>(M), (const double*)J, (const float*)D,
-                       (float*)Fh, tag, c->dparams, g, dir);
+                       (float*)Fh, tag, c->dparams, g);
 }
 
 int launch_spec_viscous(f3d_ctx* c, int dir, void* Fd, const double* Q, const void* Yi,
