@@ -573,6 +573,10 @@ int launch_species_split(f3d_ctx* c, const double* rhoi, const double* Q, void* 
 int launch_shock_sensor(f3d_ctx* c, void* phi, const double* Q, hipStream_t s);
 int launch_weno(f3d_ctx* c, int dir, void* F, const void* phi, const void* Fp, const void* Fm,
                 int NV, const int64_t* tag, hipStream_t s);
+// x sweep of both variable groups, splitting and reconstruction fused (FP64,
+// no tag): F [faces, 5], Fi [faces, Ns]; M: the sweep's three metrics
+int launch_conv_x(f3d_ctx* c, void* F, void* Fi, const void* phi, const double* Q,
+                  const double* rhoi, const void* const* M, hipStream_t s);
 int launch_viscous(f3d_ctx* c, int dir, void* Fv, const double* Q, const void* const* M,
                    const void* J, const void* lam, const void* mu, const void* Fh,
                    const int64_t* tag, hipStream_t s, bool mf = false);

@@ -45,12 +45,14 @@ def test_fill_pairs_of_faces(mech, kinds):
     ctx.close()
 
 
-@pytest.mark.parametrize("shape", [(4, 4, 4), (65, 7, 5), (9, 33, 34), (70, 66, 9)])
+@pytest.mark.parametrize("shape", [(4, 4, 4), (65, 7, 5), (9, 33, 34), (70, 66, 9), (128, 4, 5),
+                                   (257, 5, 4)])
 @pytest.mark.parametrize("mech", ["air5", "h2_lidryer"])
 def test_stage_on_small_and_ragged_blocks(mech, shape):
     """One FP64 stage on blocks of one short segment, several, a remainder
-    segment and a partial wave: 1e-12 normwise per field, the FP64 path's
-    parity bar."""
+    segment and a partial wave (marches), and of x lines that take one to four
+    waves or two segments of the fused x sweep: 1e-12 normwise per field, the
+    FP64 path's parity bar."""
     import flame3d_amd.abi as abi
     import flame3d_amd.cases as cases
     import flame3d_amd.mech as mm
