@@ -269,7 +269,7 @@ __device__ inline void h_specs(const DevParams* P, R T, R* h) {
 // operations the per-cell formulas had.  With div_const below: point-implicit
 // air step 150x75x50 119.8 -> 90.4 us, three FP32 stage ends 256x192x128 2.62
 // -> 2.11 ms, surrogate step 192x128x128 3.93 -> 3.52 ms.
-struct NasaSet {
+struct alignas(16) NasaSet {
   double c0m1, c1, c2, c3, c4;  // a1 - 1, a2 .. a5
   double d5;                    // 0 below the breakpoint, a6(high) - a6(low) above
   double c0, c5, c6, pad;       // a1, a6, a7
@@ -329,7 +329,11 @@ __device__ __forceinline__ double div_const(double a, double b, double rb) {
 // InternalEnergy, thermo.jl:219-228, and CV, thermo.jl:194-203 (FP64), at the
 // same temperature.  RCP: rho_k e_k times 1/W_k instead of divided by W_k (one
 // rounding differs; the Newton chemistry and the warm-started e -> T use it).
-template <int NS, bool RCP = false>
+// ONE: one species at a time, for kernels that other waves keep busy (left
+// alone the compiler loads every species' set first: 205 VGPRs in the FP32
+// stage end instead of 101, and 720 instead of 635 us at 256x192x128; on a
+// block that does not fill the chip all loads first is the faster order).
+template <int NS, bool RCP = false, bool ONE = false>
 __device__ inline void energy_cv(const NasaTab<NS>& N, const DevParams* P, double T,
                                  const double* rhoi, double& e_out, double& cv_out) {
   const double T2 = 0.5 * T * T;
@@ -348,15 +352,16 @@ __device__ inline void energy_cv(const NasaTab<NS>& N, const DevParams* P, doubl
     es += RCP ? rhoi[n] * e * P->rmw[n] : div_const(rhoi[n] * e, P->mw[n], P->rmw[n]);
     cs += RCP ? (cp - 1) * rhoi[n] * P->rmw[n]
               : div_const((cp - 1) * rhoi[n], P->mw[n], P->rmw[n]);
+    if (ONE) __builtin_amdgcn_sched_barrier(0);
   }
   e_out = es * P->Ru;
   cv_out = cs * P->Ru;
 }
-template <int NS, bool RCP = false>
+template <int NS, bool RCP = false, bool ONE = false>
 __device__ inline double cv_mix(const NasaTab<NS>& N, const DevParams* P, double T,
                                 const double* rhoi) {
   double e, cv;
-  energy_cv<NS, RCP>(N, P, T, rhoi, e, cv);
+  energy_cv<NS, RCP, ONE>(N, P, T, rhoi, e, cv);
   return cv;
 }
 template <int NS, bool RCP = false>
@@ -379,7 +384,7 @@ __device__ inline double pmixture(const DevParams* P, double T, const double* rh
 
 // Where GetT starts: the energies at the ends of the fits' range, the result
 // outside it (linear extrapolation), and e / A_s inside it.
-template <int NS>
+template <int NS, bool ONE>
 __device__ inline bool get_T_start(const NasaTab<NS>& N, const DevParams* P, double ein,
                                    const double* rhoi, double& t1) {
   const double tmin = P->min_temp, tmax = P->max_temp;
@@ -393,11 +398,11 @@ __device__ inline bool get_T_start(const NasaTab<NS>& N, const DevParams* P, dou
   emin *= P->Ru;
   emax *= P->Ru;
   if (ein < emin) {
-    t1 = tmin - (emin - ein) / cv_mix<NS>(N, P, tmin, rhoi);
+    t1 = tmin - (emin - ein) / cv_mix<NS, false, ONE>(N, P, tmin, rhoi);
     return false;
   }
   if (ein > emax) {
-    t1 = tmax - (emax - ein) / cv_mix<NS>(N, P, tmax, rhoi);
+    t1 = tmax - (emax - ein) / cv_mix<NS, false, ONE>(N, P, tmax, rhoi);
     return false;
   }
   t1 = ein / As;
@@ -407,16 +412,16 @@ __device__ inline bool get_T_start(const NasaTab<NS>& N, const DevParams* P, dou
 
 // GetT, thermo.jl:231-282 (FP64 Newton e -> T; tol 1e-3 K, <= 30 updates,
 // +-100 K step clamp, linear extrapolation outside [min_temp, max_temp]).
-template <int NS>
+template <int NS, bool ONE = false>
 __device__ inline double get_T(const NasaTab<NS>& N, const DevParams* P, double ein,
                                const double* rhoi) {
   const double tol = 1e-3;
   double t1;
-  if (!get_T_start<NS>(N, P, ein, rhoi, t1)) return t1;
+  if (!get_T_start<NS, ONE>(N, P, ein, rhoi, t1)) return t1;
   double x1 = 0.0, x2 = 0.0;  // t1 one and two updates ago
   for (int m = 0; m < 30; ++m) {
     double e1, cv;
-    energy_cv<NS>(N, P, t1, rhoi, e1, cv);
+    energy_cv<NS, false, ONE>(N, P, t1, rhoi, e1, cv);
     double dt = (ein - e1) / cv;
     if (dt > 100.0) {
       dt = 100.0;
@@ -457,11 +462,11 @@ __device__ inline double get_T_gap(const NasaTab<NS>& N, const DevParams* P, dou
                                    const double* rhoi) {
   const double tol = 1e-3;
   double t1;
-  if (!get_T_start<NS>(N, P, ein, rhoi, t1)) return t1;
+  if (!get_T_start<NS, true>(N, P, ein, rhoi, t1)) return t1;
   double x1 = 0.0, x2 = 0.0;  // t1 one and two updates ago
   for (int m = 0; m < 30; ++m) {
     double e1, cv;
-    energy_cv<NS, true>(N, P, t1, rhoi, e1, cv);
+    energy_cv<NS, true, true>(N, P, t1, rhoi, e1, cv);
     double dt = (ein - e1) / cv;
     if (dt > 100.0) {
       dt = 100.0;
@@ -498,13 +503,13 @@ __device__ inline double get_T_from(const NasaTab<NS>& N, const DevParams* P, do
                                     const double* rhoi, double T_guess) {
   const double tol = 1e-3;
   const double tmin = P->min_temp, tmax = P->max_temp;
-  if (!(T_guess >= tmin && T_guess <= tmax)) return get_T<NS>(N, P, ein, rhoi);
+  if (!(T_guess >= tmin && T_guess <= tmax)) return get_T<NS, true>(N, P, ein, rhoi);
   double t1 = T_guess;
   bool done = false;
   double dt_prev = 0.0;
   for (int m = 0; m < 30; ++m) {
     double e1, cv;
-    energy_cv<NS, true>(N, P, t1, rhoi, e1, cv);
+    energy_cv<NS, true, true>(N, P, t1, rhoi, e1, cv);
     double dt = (ein - e1) / cv;
     if (dt > 100.0) {
       dt = 100.0;
@@ -524,7 +529,7 @@ __device__ inline double get_T_from(const NasaTab<NS>& N, const DevParams* P, do
     dt_prev = dt;
     t1 += dt;
   }
-  if (!done || !(t1 >= tmin && t1 <= tmax)) return get_T<NS>(N, P, ein, rhoi);
+  if (!done || !(t1 >= tmin && t1 <= tmax)) return get_T<NS, true>(N, P, ein, rhoi);
   // within 0.5 K of a breakpoint (the jumps of the fits are <= 0.2 K wide):
   // where the jump is narrower than the tolerance, or the fits overlap (two
   // roots), the start decides where the update stops; take get_T's end point
