@@ -53,15 +53,18 @@ __device__ inline float gelu(float x, float& dg) {
 // the loss L = sum (y - t)^2 / (B * NOUT) and its partial loss to
 // partial[blockIdx.x][0 .. NPARAM].
 // ---------------------------------------------------------------------------
+// Rows are padded by 16 bytes so that the 16-byte operand reads of 16 rows fall
+// into different banks (rows of 64 or 128 bytes share theirs).
+constexpr int kTilePad = 8;
 struct TileLds {
-  __bf16 X[64][NN_INP];    // [s][k], forward operand of layer 0
-  __bf16 Xt[NN_INP][64];   // [k][s], weight-gradient operand of layer 0
-  __bf16 At[3][NN_H][64];  // hidden activations [o][s] (weight-gradient operands)
+  __bf16 X[64][NN_INP + kTilePad];    // [s][k], forward operand of layer 0
+  __bf16 Xt[NN_INP][64 + kTilePad];   // [k][s], weight-gradient operand of layer 0
+  __bf16 At[3][NN_H][64 + kTilePad];  // hidden activations [o][s] (weight-gradient operands)
   union {
-    __bf16 A[2][64][NN_H];  // forward ping-pong [s][o]
+    __bf16 A[2][64][NN_H + kTilePad];  // forward ping-pong [s][o]
     struct {
-      __bf16 dZ[64][NN_H];   // backward: dZ [s][o] (data-gradient operand)
-      __bf16 dZt[NN_H][64];  // dZ^T [o][s] (weight-gradient operand)
+      __bf16 dZ[64][NN_H + kTilePad];   // backward: dZ [s][o] (data-gradient operand)
+      __bf16 dZt[NN_H][64 + kTilePad];  // dZ^T [o][s] (weight-gradient operand)
     } g;
   } u;
   float bsum[4][NN_H];  // per-wave bias-gradient partial sums
@@ -226,28 +229,48 @@ __global__ void __launch_bounds__(256)
   if (tid == 0) part[NN_NPARAM] = L.red[0] / ((float)B * (float)nout);
 }
 
-// Sum of the per-tile partials (gradient and loss), one thread per slot.
-__global__ void __launch_bounds__(256)
-    k_nn_reduce(const float* __restrict__ partial, int ntiles, float* __restrict__ out) {
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p > NN_NPARAM) return;
+// Sum over the tiles of the partials (gradient and loss): blocks of 64 slots,
+// kSumWays threads per slot, each over every kSumWays-th tile, then a tree.
+// One thread per slot walking all tiles is a chain of 128 loads at the
+// training batch (30 us); this is 8 loads and four additions deep (4 us).
+// Valid in the threads of way 0.
+constexpr int kSumSlots = 64, kSumWays = 16;
+__device__ inline float nn_tile_sum(const float* __restrict__ partial, int ntiles, int p) {
+  __shared__ float acc[kSumWays][kSumSlots];
+  const int x = threadIdx.x, y = threadIdx.y;
   float s = 0.0f;
-  for (int t = 0; t < ntiles; ++t) s += partial[(long)t * (NN_NPARAM + 1) + p];
-  out[p] = s;
+  if (p <= NN_NPARAM) {
+#pragma unroll 8
+    for (int t = y; t < ntiles; t += kSumWays) s += partial[(long)t * (NN_NPARAM + 1) + p];
+  }
+  acc[y][x] = s;
+  __syncthreads();
+#pragma unroll
+  for (int w = kSumWays / 2; w > 0; w >>= 1) {
+    if (y < w) acc[y][x] += acc[y + w][x];
+    __syncthreads();
+  }
+  return acc[0][x];
+}
+
+__global__ void __launch_bounds__(kSumSlots * kSumWays)
+    k_nn_reduce(const float* __restrict__ partial, int ntiles, float* __restrict__ out) {
+  const int p = blockIdx.x * kSumSlots + threadIdx.x;
+  const float g = nn_tile_sum(partial, ntiles, p);
+  if (threadIdx.y == 0 && p <= NN_NPARAM) out[p] = g;
 }
 
 // Adam (Kingma & Ba 2015) on the FP32 master weights; refreshes the BF16
 // copies (row-major and transposed).  Padded weights stay zero: their
 // gradient is zero and they start at zero.
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(kSumSlots * kSumWays)
     k_nn_adam(const float* __restrict__ partial, int ntiles, float* __restrict__ master,
               float* __restrict__ m1, float* __restrict__ m2, __bf16* __restrict__ Wb,
               __bf16* __restrict__ Wtb, float lr, float b1, float b2, float eps, float bc1,
               float bc2, float* __restrict__ loss_out) {
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p > NN_NPARAM) return;
-  float g = 0.0f;
-  for (int t = 0; t < ntiles; ++t) g += partial[(long)t * (NN_NPARAM + 1) + p];
+  const int p = blockIdx.x * kSumSlots + threadIdx.x;
+  const float g = nn_tile_sum(partial, ntiles, p);
+  if (threadIdx.y != 0 || p > NN_NPARAM) return;
   if (p == NN_NPARAM) {
     if (loss_out) *loss_out = g;
     return;
@@ -1137,7 +1160,7 @@ int f3d_nn_grad(f3d_ctx* c, const float* X, const float* Y, int32_t B, float* gr
   hipLaunchKernelGGL(k_nn_train_tile, dim3(tiles), dim3(256), 0, s, X, Y, B, c->g.Ns + 2, c->g.Ns,
                      (const __bf16*)c->nn_Wb, (const __bf16*)c->nn_Wtb, c->nn_master,
                      c->nn_partial);
-  hipLaunchKernelGGL(k_nn_reduce, dim3(nblocks(NN_NPARAM + 1)), dim3(kBlock), 0, s,
+  hipLaunchKernelGGL(k_nn_reduce, dim3(nblocks(NN_NPARAM + 1, kSumSlots)), dim3(kSumSlots, kSumWays), 0, s,
                      c->nn_partial, (int)tiles, grad);
   return hip_check(hipGetLastError(), "f3d_nn_grad");
 }
@@ -1156,7 +1179,7 @@ int f3d_nn_train_step(f3d_ctx* c, const float* X, const float* Y, int32_t B, flo
   hipLaunchKernelGGL(k_nn_train_tile, dim3(tiles), dim3(256), 0, s, X, Y, B, c->g.Ns + 2, c->g.Ns,
                      (const __bf16*)c->nn_Wb, (const __bf16*)c->nn_Wtb, c->nn_master,
                      c->nn_partial);
-  hipLaunchKernelGGL(k_nn_adam, dim3(nblocks(NN_NPARAM + 1)), dim3(kBlock), 0, s, c->nn_partial,
+  hipLaunchKernelGGL(k_nn_adam, dim3(nblocks(NN_NPARAM + 1, kSumSlots)), dim3(kSumSlots, kSumWays), 0, s, c->nn_partial,
                      (int)tiles, c->nn_master, c->nn_m1, c->nn_m2, (__bf16*)c->nn_Wb,
                      (__bf16*)c->nn_Wtb, lr, (float)b1, (float)b2, 1e-8f, bc1, bc2, loss);
   return hip_check(hipGetLastError(), "f3d_nn_train_step");
@@ -1180,7 +1203,7 @@ int f3d_nn_train_step_static(f3d_ctx* c, const float* X, const float* Y, int32_t
   const float bc2 = (float)(1.0 - std::pow(b2, (double)c->nn_step));
   hipLaunchKernelGGL(k_nn_train_tile, dim3(tiles), dim3(256), 0, s, X, Y, B, c->g.Ns + 2, c->g.Ns,
                      (const __bf16*)c->nn_Wb, (const __bf16*)c->nn_Wtb, c->nn_master, part);
-  hipLaunchKernelGGL(k_nn_adam, dim3(nblocks(NN_NPARAM + 1)), dim3(kBlock), 0, s, part,
+  hipLaunchKernelGGL(k_nn_adam, dim3(nblocks(NN_NPARAM + 1, kSumSlots)), dim3(kSumSlots, kSumWays), 0, s, part,
                      (int)tiles, c->nn_master, c->nn_m1, c->nn_m2, (__bf16*)c->nn_Wb,
                      (__bf16*)c->nn_Wtb, lr, (float)b1, (float)b2, 1e-8f, bc1, bc2, loss);
   return hip_check(hipGetLastError(), "f3d_nn_train_step_static");
