@@ -24,23 +24,32 @@ namespace f3d {
 // The special cases (NaN, overflow, underflow, zero, negative, infinite
 // arguments) are selects on the result, not branches: a wave carries one
 // straight line of arithmetic through the rate evaluation.
+// Horner's step p r + c with the constant in a scalar register: left to the
+// compiler the constants become vector registers hoisted out of the Newton
+// loop and spilled, each step then waiting for a scratch load.
+__device__ __forceinline__ double horner(double p, double r, double c) {
+  double d;
+  asm("v_fma_f64 %0, %1, %2, %3" : "=v"(d) : "v"(p), "v"(r), "s"(c));
+  return d;
+}
+
 __device__ inline double f3d_exp(double x) {
   const double kd = floor(x * 1.4426950408889634 + 0.5);
   const double r = (x - kd * 6.93147180369123816490e-01) - kd * 1.90821492927058770002e-10;
   double p = 1.0 / 6227020800.0;  // 1/13!
-  p = fma(p, r, 1.0 / 479001600.0);
-  p = fma(p, r, 1.0 / 39916800.0);
-  p = fma(p, r, 1.0 / 3628800.0);
-  p = fma(p, r, 1.0 / 362880.0);
-  p = fma(p, r, 1.0 / 40320.0);
-  p = fma(p, r, 1.0 / 5040.0);
-  p = fma(p, r, 1.0 / 720.0);
-  p = fma(p, r, 1.0 / 120.0);
-  p = fma(p, r, 1.0 / 24.0);
-  p = fma(p, r, 1.0 / 6.0);
-  p = fma(p, r, 0.5);
-  p = fma(p, r, 1.0);
-  p = fma(p, r, 1.0);
+  p = horner(p, r, 1.0 / 479001600.0);
+  p = horner(p, r, 1.0 / 39916800.0);
+  p = horner(p, r, 1.0 / 3628800.0);
+  p = horner(p, r, 1.0 / 362880.0);
+  p = horner(p, r, 1.0 / 40320.0);
+  p = horner(p, r, 1.0 / 5040.0);
+  p = horner(p, r, 1.0 / 720.0);
+  p = horner(p, r, 1.0 / 120.0);
+  p = horner(p, r, 1.0 / 24.0);
+  p = horner(p, r, 1.0 / 6.0);
+  p = horner(p, r, 0.5);
+  p = horner(p, r, 1.0);
+  p = horner(p, r, 1.0);
   p = ldexp(p, (int)kd);
   p = x > 709.782712893384 ? __builtin_inf() : p;
   return x < -745.1332191019412 ? 0.0 : p;
@@ -55,16 +64,16 @@ __device__ inline double f3d_log(double x) {
   const double s = (m - 1.0) / (m + 1.0);
   const double z = s * s;
   double p = 1.0 / 21.0;
-  p = fma(p, z, 1.0 / 19.0);
-  p = fma(p, z, 1.0 / 17.0);
-  p = fma(p, z, 1.0 / 15.0);
-  p = fma(p, z, 1.0 / 13.0);
-  p = fma(p, z, 1.0 / 11.0);
-  p = fma(p, z, 1.0 / 9.0);
-  p = fma(p, z, 1.0 / 7.0);
-  p = fma(p, z, 1.0 / 5.0);
-  p = fma(p, z, 1.0 / 3.0);
-  p = fma(p, z, 1.0);
+  p = horner(p, z, 1.0 / 19.0);
+  p = horner(p, z, 1.0 / 17.0);
+  p = horner(p, z, 1.0 / 15.0);
+  p = horner(p, z, 1.0 / 13.0);
+  p = horner(p, z, 1.0 / 11.0);
+  p = horner(p, z, 1.0 / 9.0);
+  p = horner(p, z, 1.0 / 7.0);
+  p = horner(p, z, 1.0 / 5.0);
+  p = horner(p, z, 1.0 / 3.0);
+  p = horner(p, z, 1.0);
   const double ed = (double)e;
   double v = ed * 6.93147180369123816490e-01 + (ed * 1.90821492927058770002e-10 + (2.0 * s) * p);
   v = x == __builtin_inf() ? x : v;
@@ -391,10 +400,21 @@ __device__ inline void production_rate_at(const NasaTab<NS>& N, const DevParams*
 // (finite at zero concentration) plus the [M] derivative of three-body and
 // falloff rates with the falloff factor held fixed (the Lindemann part).
 // One pass over the reactions: the transcendentals are shared with wdot.
-template <int NS, class K = KinRT>
+// CI: the three species, at run time (CarrierRT) or as constants (CarrierCT),
+// which with compile-time reaction tables leaves of the block only the terms
+// that are there.
+struct CarrierRT {
+  int c[3];
+  __device__ int operator[](int j) const { return c[j]; }
+};
+template <int A, int B, int C>
+struct CarrierCT {
+  __device__ constexpr int operator[](int j) const { return j == 0 ? A : j == 1 ? B : C; }
+};
+template <int NS, class K, class CI>
 __device__ inline void production_rate_block3(const NasaTab<NS>& N,
                                               const DevParams* __restrict__ P, const double* sc,
-                                              double T, const int (&ci)[3], double* wdot,
+                                              double T, const CI ci, double* wdot,
                                               double (&M)[3][3]) {
   const K Kp(P);
   const double lgT = f3d_log(T);
@@ -409,7 +429,8 @@ __device__ inline void production_rate_block3(const NasaTab<NS>& N,
   for (int j = 0; j < 3; ++j) {
     double v = 0.0;
 #pragma unroll
-    for (int m = 0; m < NS; ++m) v += (m == ci[j]) ? sc[m] : 0.0;  // register select, no scratch
+    for (int m = 0; m < NS; ++m)
+      if (m == ci[j]) v = sc[m];  // register select, no scratch
     cc[j] = v;
 #pragma unroll
     for (int i = 0; i < 3; ++i) M[i][j] = 0.0;
@@ -510,6 +531,20 @@ __device__ inline void production_rate_block3(const NasaTab<NS>& N,
         const int dl = Kp.vr(n, cr) - Kp.vf(n, cr);
         if (dl != 0) M[i][j] += d * (double)dl;
       }
+    }
+    if constexpr (K::kConst) {
+      // the sums are formed here: deferred, each would keep
+      // the terms of several reactions in registers
+#pragma unroll
+      for (int m = 0; m < NS; ++m)
+        if (Kp.vf(n, m) != Kp.vr(n, m)) asm volatile("" : "+v"(wdot[m]));
+#pragma unroll
+      for (int i = 0; i < 3; ++i)
+#pragma unroll
+        for (int j = 0; j < 3; ++j)
+          if (ci[i] >= 0 && ci[j] >= 0 && Kp.vf(n, ci[i]) != Kp.vr(n, ci[i]) &&
+              (rt != 1 || Kp.vf(n, ci[j]) != 0 || Kp.vr(n, ci[j]) != 0))
+            asm volatile("" : "+v"(M[i][j]));
     }
   });
 }

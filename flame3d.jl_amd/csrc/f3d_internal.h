@@ -96,6 +96,8 @@ struct f3d_ctx {
   long nn_partial_tiles = 0;
   void* nn_cfg = nullptr;  // device NNDev
   double nn_dt = 0;
+  int nn_chain[3] = {-1, -1, -1};  // chain carriers of the configuration
+  int nn_label_mode = 0;
   long nn_step = 0;
   int8_t* nn_status = nullptr;  // per-cell gate codes [Nx*Ny*Nz] when the caller passes none
   int32_t* nn_fbcount = nullptr;  // rejected cells per 64-cell tile, then their offsets

@@ -28,6 +28,7 @@
 namespace f3d {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 __device__ inline f32x4 mfma(const bf16x8& a, const bf16x8& b, const f32x4& c) {
@@ -306,17 +307,20 @@ __global__ void __launch_bounds__(256)
 // the FP32 outputs: a layer's 4x4 (or 4x2) 16x16 output tiles stay in
 // registers until every lane has read the previous activations.
 // ---------------------------------------------------------------------------
-// Rows are padded by 16 bytes (one float for Y): a 16-byte MFMA operand read
-// by the 16 lanes of a quarter-wave then spans different bank groups instead
-// of the same one (an unpadded row of 64 bf16 is 128 B, a whole bank cycle).
+// Rows are padded by 16 bytes: a 16-byte MFMA operand read by the 16 lanes of
+// a quarter-wave then spans different bank groups instead of the same one (an
+// unpadded row of 64 bf16 is 128 B, a whole bank cycle).
 constexpr int kRowPad = 8;
 union FwdLds {
   __bf16 X[64][NN_INP + kRowPad];
   __bf16 A[64][NN_H + kRowPad];
-  float Y[64][NN_OUTP + 1];
+  float Y[64][NN_OUTP + 4];
 };
 
-// one dense layer for the wave's 64 samples: NI inputs, NO outputs (compile-time)
+// one dense layer for the wave's 64 samples: NI inputs, NO outputs (compile-time).
+// The weights are the MFMA's A operand, so a lane receives four consecutive
+// outputs of one sample and stores them with one write (8 bytes of bf16, or 16
+// of float) instead of four 2-byte writes 144 bytes apart.
 template <int NI, int NO, bool LAST>
 __device__ __forceinline__ void nn_layer_wave(FwdLds& L, const __bf16* __restrict__ W,
                                      const float* __restrict__ bias, int lane) {
@@ -328,34 +332,49 @@ __device__ __forceinline__ void nn_layer_wave(FwdLds& L, const __bf16* __restric
     for (int st = 0; st < 4; ++st) acc[st][ot] = {0, 0, 0, 0};
 #pragma unroll
     for (int kk = 0; kk < NI / 32; ++kk) {
-      const bf16x8 b = ld8(W + (16 * ot + r16) * NI + 32 * kk + 8 * q);
+      const bf16x8 w = ld8(W + (16 * ot + r16) * NI + 32 * kk + 8 * q);
 #pragma unroll
       for (int st = 0; st < 4; ++st) {
         const __bf16* src = (NI == NN_INP) ? &L.X[16 * st + r16][32 * kk + 8 * q]
                                            : &L.A[16 * st + r16][32 * kk + 8 * q];
-        acc[st][ot] = mfma(ld8(src), b, acc[st][ot]);
+        acc[st][ot] = mfma(w, ld8(src), acc[st][ot]);
       }
     }
   }
   __syncthreads();  // every lane has read this layer's input tile
 #pragma unroll
   for (int ot = 0; ot < NO / 16; ++ot) {
-    const int o = 16 * ot + r16;
-    const float bo = bias[o];
+    const int o = 16 * ot + 4 * q;
+    const f32x4 bo = *reinterpret_cast<const f32x4*>(bias + o);
 #pragma unroll
-    for (int st = 0; st < 4; ++st)
+    for (int st = 0; st < 4; ++st) {
+      const int s = 16 * st + r16;
+      if (LAST) {
+        *reinterpret_cast<f32x4*>(&L.Y[s][o]) = acc[st][ot] + bo;
+      } else {
+        bf16x4 h;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int s = 16 * st + 4 * q + i;
-        if (LAST) {
-          L.Y[s][o] = acc[st][ot][i] + bo;
-        } else {
+        for (int i = 0; i < 4; ++i) {
           float d;
-          L.A[s][o] = (__bf16)gelu(acc[st][ot][i] + bo, d);
+          h[i] = (__bf16)gelu(acc[st][ot][i] + bo[i], d);
         }
+        *reinterpret_cast<bf16x4*>(&L.A[s][o]) = h;
       }
+    }
   }
   __syncthreads();
+}
+
+// a lane's input row, inputs xn[0 .. nin) and zeros
+template <class F>
+__device__ __forceinline__ void nn_put_input(FwdLds& L, int lane, F&& x) {
+#pragma unroll
+  for (int k = 0; k < NN_INP; k += 8) {
+    bf16x8 v;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = (__bf16)x(k + i);
+    *reinterpret_cast<bf16x8*>(&L.X[lane][k]) = v;
+  }
 }
 
 __device__ __forceinline__ void nn_forward_wave(FwdLds& L, const __bf16* __restrict__ Wb,
@@ -373,7 +392,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4)))
   __shared__ __align__(16) FwdLds L;
   const int lane = threadIdx.x;
   const long s0 = (long)blockIdx.x * 64;
-  for (int k = 0; k < NN_INP; ++k) L.X[lane][k] = (__bf16)(k < nin ? Xg[(s0 + lane) * nin + k] : 0.0f);
+  nn_put_input(L, lane, [&](int k) { return k < nin ? Xg[(s0 + lane) * nin + k] : 0.0f; });
   __syncthreads();
   nn_forward_wave(L, Wb, master, lane);
   for (int o = 0; o < nout; ++o) Yg[(s0 + lane) * nout + o] = L.Y[lane][o];
@@ -536,8 +555,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4)))
   // a tile with no reacting cell (cold gas, tagged cells) skips the network;
   // the workgroup is one wave, so the exit is uniform over the workgroup
   if (!__any(act)) return;
-#pragma unroll
-  for (int k = 0; k < NN_INP; ++k) L.X[lane][k] = (__bf16)(k < NIN ? xn[k] : 0.0f);
+  nn_put_input(L, lane, [&](int k) { return k < NIN ? xn[k < NIN ? k : 0] : 0.0f; });
   __syncthreads();
   nn_forward_wave(L, Wb, master, lane);
   if (act) {
@@ -561,7 +579,9 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4)))
 // stores the candidate state of every cell still accepted (rho_k', T', e',
 // the energy change) to `cand` ([NS + 3][cells], FP64); k_nn_gate evaluates
 // the rate-based gates 5-7 on it and commits or rejects.
-template <int NS>
+// LM: the label mode, 3 (the shipped networks') as a constant or -1 (read at
+// run time): with the pow of mode 1 in the same kernel its registers spill.
+template <int NS, int LM>
 __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3)))
     k_nn_pred(const double* __restrict__ Q, const double* __restrict__ rhoi,
               const DevParams* __restrict__ P, const NNDev* __restrict__ C, Geom g,
@@ -587,16 +607,17 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3))
   // post_predict (reactions.jl:26-56) on the de-normalized outputs
   const double rinv = 1.0 / fmax(rho, kEps);
   const double lam = (double)C->boxcox_lambda;
+  const int mode = LM >= 0 ? LM : C->label_mode;
   double Y[NS], dY0[NS], dY[NS], S[NS];
 #pragma unroll
   for (int n = 0; n < NS; ++n) {
     Y[n] = fmax(r[n] * rinv, 0.0);
     const double o = (double)(out[(long)n * ncell + id] * C->out_std[n] + C->out_mean[n]);
-    if (C->label_mode == 0) {
+    if (mode == 0) {
       dY0[n] = o;
-    } else if (C->label_mode == 2) {
+    } else if (mode == 2) {
       dY0[n] = (double)C->label_scale[n] * sinh(o);
-    } else if (C->label_mode == 3) {
+    } else if (mode == 3) {
       const double sk = fmin((double)C->label_scale[n],
                              fmax((double)C->label_floor, (double)C->label_rel * Y[n]));
       dY0[n] = sk * sinh(o);
@@ -625,7 +646,7 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3))
     }
     if (gross > 0.0 && worst > (double)C->elem_tol * gross) eok = false;
   }
-  if (C->label_mode == 3) {
+  if (mode == 3) {
     // per-cell weights S_k = (s_k + |dY0_k|)^2: dY = dY0 - S E^T (E S E^T)^-1 E dY0
     if (!project_weighted<NS>(C, P, S, dY0, dY)) eok = false;
   } else {
@@ -648,7 +669,7 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3))
     double esum = 0.0;
 #pragma unroll
     for (int n = 0; n < NS; ++n) esum += fabs(P->hfm[n] * dY[n]);
-    if (!(esum * rho <= (double)C->dT_max * cv_mix<NS, true>(N, P, T, r))) code = 5;
+    if (!(esum * rho <= (double)C->dT_max * cv_mix<NS, true, true>(N, P, T, r))) code = 5;
   }
   if (code == 1) {
     double rn[NS], dei = 0.0, sr = 0.0;
@@ -674,12 +695,13 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3))
   if (code != 1) status[id] = (int8_t)code;
 }
 
-template <int NS, class K = KinRT>
+// CI: the chain carriers of gate 7, from the configuration or as constants.
+template <int NS, class K, class CI>
 __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2)))
     k_nn_gate(double* __restrict__ U, double* __restrict__ Q, double* __restrict__ rhoi,
               const DevParams* __restrict__ P, const NNDev* __restrict__ C, Geom g, double dt,
               const double* __restrict__ cand, int32_t* __restrict__ tile_count,
-              int8_t* __restrict__ status) {
+              int8_t* __restrict__ status, const CI carriers) {
   __shared__ NasaTab<NS> N;
   N.fill(P);
   const long ncell = (long)g.Nx * g.Ny * g.Nz;
@@ -704,12 +726,11 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))
 #pragma unroll
       for (int n = 0; n < NS; ++n) sc[n] = rn[n] * P->cmw[n];
       if (C->chain_max > 0.0f) {
-        const int cidx[3] = {C->chain_idx[0], C->chain_idx[1], C->chain_idx[2]};
-        production_rate_block3<NS, K>(N, P, sc, Tn, cidx, wdot, Mc);
+        production_rate_block3<NS, K>(N, P, sc, Tn, carriers, wdot, Mc);
       } else {
         production_rate_at<NS, false>(N, P, sc, Tn, Adum, wdot);
       }
-      const double cvn = cv_mix<NS, true>(N, P, Tn, rn);
+      const double cvn = cv_mix<NS, true, true>(N, P, Tn, rn);
       if (res_on) {
         double rmax = 0.0, esum = 0.0;
 #pragma unroll
@@ -931,6 +952,34 @@ static int nn_partials(f3d_ctx* c, long tiles) {
   return F3D_OK;
 }
 
+// The gate kernel's instance: constant carriers with the compiled-in tables
+// when the configuration names the carriers the shipped networks gate on (H,
+// O, OH of the hydrogen mechanism, O of air), else the run-time reaction loop:
+// with constant tables, run-time carriers put three tests on every species of
+// every unrolled reaction (180 KB of code, half of it scalar).
+static bool nn_carriers(const f3d_ctx* c, int a, int b, int d) {
+  return c->nn_chain[0] == a && c->nn_chain[1] == b && c->nn_chain[2] == d;
+}
+static CarrierRT nn_carriers_rt(const f3d_ctx* c) {
+  return CarrierRT{{c->nn_chain[0], c->nn_chain[1], c->nn_chain[2]}};
+}
+template <int NS>
+static void launch_pred(f3d_ctx* c, const double* Q, const double* rhoi, int8_t* st,
+                        hipStream_t s) {
+  const long ncell = (long)c->g.Nx * c->g.Ny * c->g.Nz;
+  const auto k = c->nn_label_mode == 3 ? k_nn_pred<NS, 3> : k_nn_pred<NS, -1>;
+  hipLaunchKernelGGL(k, dim3(nblocks(ncell)), dim3(kBlock), 0, s, Q, rhoi, c->dparams,
+                     (const NNDev*)c->nn_cfg, c->g, c->nn_out, c->nn_cand, st);
+}
+template <int NS, class K, class CI>
+static void launch_gate(f3d_ctx* c, double* U, double* Q, double* rhoi, double dt, int8_t* st,
+                        hipStream_t s, const CI carriers) {
+  const long ncell = (long)c->g.Nx * c->g.Ny * c->g.Nz;
+  hipLaunchKernelGGL((k_nn_gate<NS, K, CI>), dim3(nblocks(ncell)), dim3(kBlock), 0, s, U, Q, rhoi,
+                     c->dparams, (const NNDev*)c->nn_cfg, c->g, dt, c->nn_cand, c->nn_fbcount, st,
+                     carriers);
+}
+
 // Scratch of f3d_nn_train_step_static: the per-tile partial gradients and
 // losses of at most kStaticTiles tiles of 64 samples (batch <= 8192), 6.4 MB.
 // Every tile writes all of its NN_NPARAM + 1 slots, so nothing needs
@@ -1101,6 +1150,8 @@ int f3d_nn_init(f3d_ctx* c, const f3d_nn_config* cfg) {
     c->nn_ready = true;
   }
   c->nn_dt = cfg->dt;
+  c->nn_label_mode = cfg->label_mode;
+  for (int j = 0; j < 3; ++j) c->nn_chain[j] = h.chain_idx[j];
   return hip_check(hipMemcpy(c->nn_cfg, &h, sizeof(NNDev), hipMemcpyHostToDevice), "f3d_nn_init");
 }
 
@@ -1160,8 +1211,8 @@ int f3d_nn_grad(f3d_ctx* c, const float* X, const float* Y, int32_t B, float* gr
   hipLaunchKernelGGL(k_nn_train_tile, dim3(tiles), dim3(256), 0, s, X, Y, B, c->g.Ns + 2, c->g.Ns,
                      (const __bf16*)c->nn_Wb, (const __bf16*)c->nn_Wtb, c->nn_master,
                      c->nn_partial);
-  hipLaunchKernelGGL(k_nn_reduce, dim3(nblocks(NN_NPARAM + 1, kSumSlots)), dim3(kSumSlots, kSumWays), 0, s,
-                     c->nn_partial, (int)tiles, grad);
+  hipLaunchKernelGGL(k_nn_reduce, dim3(nblocks(NN_NPARAM + 1, kSumSlots)),
+                     dim3(kSumSlots, kSumWays), 0, s, c->nn_partial, (int)tiles, grad);
   return hip_check(hipGetLastError(), "f3d_nn_grad");
 }
 
@@ -1179,8 +1230,8 @@ int f3d_nn_train_step(f3d_ctx* c, const float* X, const float* Y, int32_t B, flo
   hipLaunchKernelGGL(k_nn_train_tile, dim3(tiles), dim3(256), 0, s, X, Y, B, c->g.Ns + 2, c->g.Ns,
                      (const __bf16*)c->nn_Wb, (const __bf16*)c->nn_Wtb, c->nn_master,
                      c->nn_partial);
-  hipLaunchKernelGGL(k_nn_adam, dim3(nblocks(NN_NPARAM + 1, kSumSlots)), dim3(kSumSlots, kSumWays), 0, s, c->nn_partial,
-                     (int)tiles, c->nn_master, c->nn_m1, c->nn_m2, (__bf16*)c->nn_Wb,
+  hipLaunchKernelGGL(k_nn_adam, dim3(nblocks(NN_NPARAM + 1, kSumSlots)),
+                     dim3(kSumSlots, kSumWays), 0, s, c->nn_partial, (int)tiles, c->nn_master, c->nn_m1, c->nn_m2, (__bf16*)c->nn_Wb,
                      (__bf16*)c->nn_Wtb, lr, (float)b1, (float)b2, 1e-8f, bc1, bc2, loss);
   return hip_check(hipGetLastError(), "f3d_nn_train_step");
 }
@@ -1203,8 +1254,8 @@ int f3d_nn_train_step_static(f3d_ctx* c, const float* X, const float* Y, int32_t
   const float bc2 = (float)(1.0 - std::pow(b2, (double)c->nn_step));
   hipLaunchKernelGGL(k_nn_train_tile, dim3(tiles), dim3(256), 0, s, X, Y, B, c->g.Ns + 2, c->g.Ns,
                      (const __bf16*)c->nn_Wb, (const __bf16*)c->nn_Wtb, c->nn_master, part);
-  hipLaunchKernelGGL(k_nn_adam, dim3(nblocks(NN_NPARAM + 1, kSumSlots)), dim3(kSumSlots, kSumWays), 0, s, part,
-                     (int)tiles, c->nn_master, c->nn_m1, c->nn_m2, (__bf16*)c->nn_Wb,
+  hipLaunchKernelGGL(k_nn_adam, dim3(nblocks(NN_NPARAM + 1, kSumSlots)),
+                     dim3(kSumSlots, kSumWays), 0, s, part, (int)tiles, c->nn_master, c->nn_m1, c->nn_m2, (__bf16*)c->nn_Wb,
                      (__bf16*)c->nn_Wtb, lr, (float)b1, (float)b2, 1e-8f, bc1, bc2, loss);
   return hip_check(hipGetLastError(), "f3d_nn_train_step_static");
 }
@@ -1240,7 +1291,6 @@ int f3d_nn_chem(f3d_ctx* c, double* U, double* Q, double* rhoi, double dt, int32
   const bool timed = c->nn_timing;
   if (timed) (void)hipEventRecord(c->nn_ev[0], s);
   // every tile writes its count, so no clearing is needed
-  const unsigned nb = nblocks(ncell);
   if (c->g.Ns == 9)
     hipLaunchKernelGGL((k_nn_net<9>), dim3((unsigned)ntile), dim3(64), 0, s, Q, rhoi, tag,
                        c->dparams, (const NNDev*)c->nn_cfg, (const __bf16*)c->nn_Wb, c->nn_master,
@@ -1251,25 +1301,17 @@ int f3d_nn_chem(f3d_ctx* c, double* U, double* Q, double* rhoi, double dt, int32
                        c->g, c->nn_out, st);
   if (timed) (void)hipEventRecord(c->nn_ev[1], s);
   if (c->g.Ns == 9) {
-    hipLaunchKernelGGL((k_nn_pred<9>), dim3(nb), dim3(kBlock), 0, s, Q, rhoi, c->dparams,
-                       (const NNDev*)c->nn_cfg, c->g, c->nn_out, c->nn_cand, st);
-    if (c->kin_table == F3D_KIN_H2_LIDRYER)
-      hipLaunchKernelGGL((k_nn_gate<9, KinCT<MechH2LiDryer>>), dim3(nb), dim3(kBlock), 0, s, U, Q,
-                         rhoi, c->dparams, (const NNDev*)c->nn_cfg, c->g, dt, c->nn_cand,
-                         c->nn_fbcount, st);
+    launch_pred<9>(c, Q, rhoi, st, s);
+    if (c->kin_table == F3D_KIN_H2_LIDRYER && nn_carriers(c, 3, 4, 5))
+      launch_gate<9, KinCT<MechH2LiDryer>>(c, U, Q, rhoi, dt, st, s, CarrierCT<3, 4, 5>());
     else
-      hipLaunchKernelGGL((k_nn_gate<9>), dim3(nb), dim3(kBlock), 0, s, U, Q, rhoi, c->dparams,
-                         (const NNDev*)c->nn_cfg, c->g, dt, c->nn_cand, c->nn_fbcount, st);
+      launch_gate<9, KinRT>(c, U, Q, rhoi, dt, st, s, nn_carriers_rt(c));
   } else {
-    hipLaunchKernelGGL((k_nn_pred<5>), dim3(nb), dim3(kBlock), 0, s, Q, rhoi, c->dparams,
-                       (const NNDev*)c->nn_cfg, c->g, c->nn_out, c->nn_cand, st);
-    if (c->kin_table == F3D_KIN_AIR5)
-      hipLaunchKernelGGL((k_nn_gate<5, KinCT<MechAir5>>), dim3(nb), dim3(kBlock), 0, s, U, Q,
-                         rhoi, c->dparams, (const NNDev*)c->nn_cfg, c->g, dt, c->nn_cand,
-                         c->nn_fbcount, st);
+    launch_pred<5>(c, Q, rhoi, st, s);
+    if (c->kin_table == F3D_KIN_AIR5 && nn_carriers(c, 0, -1, -1))
+      launch_gate<5, KinCT<MechAir5>>(c, U, Q, rhoi, dt, st, s, CarrierCT<0, -1, -1>());
     else
-      hipLaunchKernelGGL((k_nn_gate<5>), dim3(nb), dim3(kBlock), 0, s, U, Q, rhoi, c->dparams,
-                         (const NNDev*)c->nn_cfg, c->g, dt, c->nn_cand, c->nn_fbcount, st);
+      launch_gate<5, KinRT>(c, U, Q, rhoi, dt, st, s, nn_carriers_rt(c));
   }
   if (timed) (void)hipEventRecord(c->nn_ev[2], s);
   // tile counts -> tile offsets; the chunk sums sit after the tile counts
