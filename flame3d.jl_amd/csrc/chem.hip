@@ -9,16 +9,21 @@
 // are wave-uniform branches that skip the zero terms the reference adds; for a
 // shipped mechanism it is unrolled over the compiled-in tables.
 //
-// The Newton mode is bound by instruction issue at one wave per SIMD (its
-// system takes the register file), so what counts is how many instructions an
-// iteration takes and how long a wave waits for its slowest cell.  128^3 H2/O2
-// reactors (2.45 iterations per cell on average, 5.0 for the slowest of 64):
-// 28.6 ms with the reactions in a run-time loop, branches in exp and log,
-// every pivot exchange taken and 256-thread blocks; 8.84 ms with one
-// instantiation per reaction, selects, exchanges only where a lane needs them
-// and one-wave blocks; 8.01 ms with the NASA-7 sets in LDS and read once per
-// iteration, and the parameter block's quotients read where they are used.
+// The Newton mode is bound by instruction issue at two waves per SIMD, so what
+// counts is how many instructions an iteration takes and how long a wave waits
+// for its slowest cell.  128^3 H2/O2 reactors (2.45 iterations per cell on
+// average, 5.0 for the slowest of 64): 28.6 ms with the reactions in a run-time
+// loop, branches in exp and log, every pivot exchange taken and 256-thread
+// blocks; 8.84 ms with one instantiation per reaction, selects, exchanges only
+// where a lane needs them and one-wave blocks; 8.01 ms with the NASA-7 sets in
+// LDS and read once per iteration, and the parameter block's quotients read
+// where they are used; 3.44 ms with every sum formed where its terms are (an
+// empty asm after each reaction and each species), the series' constants in
+// scalar registers and the initial densities read again at the end instead of
+// kept: fewer values are held across an iteration, so that two waves fit a
+// SIMD with 240 bytes of scratch where one took 850.
 #include "f3d_chem.h"
+#include "f3d_chem_rows.h"
 #include "f3d_internal.h"
 #include "f3d_mech_tables.h"
 
@@ -26,6 +31,17 @@ namespace f3d {
 
 // Most backward-Euler substeps the Newton mode tries before giving up.
 constexpr int kNewtonMaxSub = 64;
+// In a pass over a cell list: iterations of the first step after which a cell
+// goes to the half-wave solve (f3d_chem_rows.h).  A list's wave ends with its
+// slowest cell; one of 56 iterations takes 1.0 ms here, 0.1 + 0.42 ms this way.
+// 64^3 reactors, 151610 of them listed, whole surrogate step: 0.91 ms with 8,
+// 0.90 with 6, 0.88 with 5, 0.87 with 4 (1.23 ms all here); but with 4 a tenth
+// of a flame's cells would go.
+constexpr int kNewtonFirst = 5;
+// Most cells that go: two for each half wave the device holds.  A half wave
+// has a twentieth of the one-thread solve's throughput, so where slow cells
+// are many the rest go on in their threads.
+constexpr int kRowsMost = 4096;
 
 // One backward-Euler solve over h of the reactor (rho_k, T) from (r, T),
 // total energy fixed at E0: Newton on
@@ -39,11 +55,12 @@ constexpr int kNewtonMaxSub = 64;
 typedef const __attribute__((address_space(4))) DevParams ConstParams;
 
 // Per-lane values that an iteration needs now and then live in LDS (the
-// Jacobian takes the registers): the substep's initial densities, the
-// reactor's, and the species' g/RT, h/RT and energy derivatives at T.
+// Jacobian takes the registers): the substep's initial densities and the
+// species' g/RT, h/RT and energy derivatives at T.  With the NASA-7 table
+// 20 KB for Ns = 9, an eighth of a compute unit's LDS: two waves per SIMD.
 template <int NS>
 struct NewtonLds {
-  double r0[NS][64], rs[NS][64], g[NS][64], h[NS][64], de[NS][64];
+  double rs[NS][64], g[NS][64], h[NS][64], de[NS][64];
 };
 template <int NS>
 struct GibbsLds {
@@ -99,11 +116,15 @@ __device__ inline bool be_solve(const NasaTab<NS>& N, NewtonLds<NS>& L, int lane
         E += r[n] * e * P->rmw[n];
         cv += (cp - 1) * r[n] * P->rmw[n];
         L.de[n][lane] = e * P->Rmw[n] + P->hfm[n];
+        // formed here: sunk to their use, the sums would keep every fit alive
+        // across the assembly
+        asm volatile("" : "+v"(E), "+v"(cv));
       }
       E *= P->Ru;
       cv *= P->Ru;
 #pragma unroll
       for (int n = 0; n < NS; ++n) E += P->hfm[n] * r[n];
+      asm volatile("" : "+v"(E));
     }
     // rate Jacobian in A[0..NS-1][0..NS-1], d wdot / dT in A[0..NS-1][NS]
     production_rate<NS, true, true, N1, true, true, K>(P0, sc, T, lgT, invT,
@@ -152,18 +173,21 @@ __device__ inline bool be_solve(const NasaTab<NS>& N, NewtonLds<NS>& L, int lane
 }
 
 // Threads per block: one wave in the Newton mode, whose registers leave room
-// for one wave per SIMD, so a block of four waves would hold three SIMDs until
-// its slowest wave (the one with the most iterations) has ended.
+// for two waves per SIMD: a block of four would hold their places until its
+// slowest wave (the one with the most iterations) has ended.
 constexpr int chem_block(int mode) { return mode == 2 ? 64 : kBlock; }
 
+// Two waves per SIMD asked for where the tables are compiled in; with the
+// run-time loop the matrices would spill.
 // mode 0: eval_gpu_stiff, 1: eval_gpu, 2: backward-Euler Newton.  K: the
 // reaction parameters, from the parameter block or compiled in (KinCT).
 template <int NS, int MODE, class K = KinRT>
-__global__ void __launch_bounds__(chem_block(MODE))
+__global__ void __launch_bounds__(chem_block(MODE)) __attribute__((amdgpu_waves_per_eu(K::kConst ? 2 : 1)))
     k_chem(double* __restrict__ U, double* __restrict__ Q, double* __restrict__ rhoi, double dt,
            int maxiter, double rtol, double ttol, int32_t* __restrict__ iters,
            const int64_t* __restrict__ tag, const DevParams* __restrict__ P, Geom g, int bug,
-           const int32_t* __restrict__ list, long nwork) {
+           const int32_t* __restrict__ list, long nwork, int32_t* __restrict__ later,
+           int32_t* __restrict__ nlater) {
   __shared__ NasaTab<NS> N;
   N.fill(P);
   // one thread per interior cell, or per entry of an ordered cell list (the
@@ -222,10 +246,7 @@ __global__ void __launch_bounds__(chem_block(MODE))
     const int lane = threadIdx.x;
     double rho_tot = 0.0;
 #pragma unroll
-    for (int n = 0; n < NS; ++n) {
-      L.r0[n][lane] = r[n];
-      rho_tot += r[n];
-    }
+    for (int n = 0; n < NS; ++n) rho_tot += r[n];
     double E0 = internal_energy<NS, true>(N, P, T0, r);
 #pragma unroll
     for (int n = 0; n < NS; ++n) E0 += P->hfm[n] * r[n];
@@ -235,25 +256,37 @@ __global__ void __launch_bounds__(chem_block(MODE))
     int it = 0;
     bool ok = false;
     double T = T0;
-    for (int nsub = 1; nsub <= kNewtonMaxSub && !ok; nsub *= 2) {
+    bool first = later != nullptr;
+    for (int nsub = 1; nsub <= kNewtonMaxSub && !ok;) {
 #pragma unroll
-      for (int n = 0; n < NS; ++n) r[n] = L.r0[n][lane];
+      for (int n = 0; n < NS; ++n) r[n] = rhoi[p + n * NP];  // written at the end only
       T = T0;
       ok = true;
       const double h = dt / nsub;
+      const int limit = first ? min(maxiter, kNewtonFirst) : maxiter;
       for (int k = 0; k < nsub && ok; ++k)
-        ok = be_solve<NS, K>(N, L, lane, P, r, T, h, E0, rho_tot, T_lo, T_hi, maxiter, rtol, ttol,
+        ok = be_solve<NS, K>(N, L, lane, P, r, T, h, E0, rho_tot, T_lo, T_hi, limit, rtol, ttol,
                              it);
+      if (first && !ok) {  // left to k_newton_rows, from the start, or begun again here
+        const int slot = atomicAdd(nlater, 1);
+        if (slot < kRowsMost) {
+          later[slot] = (int32_t)id;
+          return;
+        }
+        first = false;
+        continue;
+      }
+      if (!ok) nsub *= 2;
     }
     if (!ok) {  // no admissible solution: the reactor is left unreacted
 #pragma unroll
-      for (int n = 0; n < NS; ++n) r[n] = L.r0[n][lane];
+      for (int n = 0; n < NS; ++n) r[n] = rhoi[p + n * NP];
       it = -it;
     }
     if (iters) iters[id] = it;
     double dei = 0;
 #pragma unroll
-    for (int n = 0; n < NS; ++n) dei += -P->hfm[n] * (r[n] - L.r0[n][lane]);
+    for (int n = 0; n < NS; ++n) dei += -P->hfm[n] * (r[n] - rhoi[p + n * NP]);
     chem_epilogue<NS>(N, P, U, Q, rhoi, p, NP, r, dei);
   }
 }
@@ -261,19 +294,31 @@ __global__ void __launch_bounds__(chem_block(MODE))
 template <int NS, class K>
 static void chem_k(f3d_ctx* c, int mode, double* U, double* Q, double* rhoi, double dt,
                    int maxiter, double rtol, double ttol, int32_t* iters, const int64_t* tag,
-                   hipStream_t s, const int32_t* list, long nlist) {
+                   hipStream_t s, const int32_t* list, long nlist, int32_t* later, int32_t* nlater) {
   const long n = list ? nlist : (long)c->g.Nx * c->g.Ny * c->g.Nz;
   if (n <= 0) return;
   const int bug = c->bug_compat & 1;
   if (mode == 0)
     hipLaunchKernelGGL((k_chem<NS, 0, K>), dim3(nblocks(n)), dim3(kBlock), 0, s, U, Q, rhoi, dt,
-                       maxiter, rtol, ttol, iters, tag, c->dparams, c->g, bug, list, n);
+                       maxiter, rtol, ttol, iters, tag, c->dparams, c->g, bug, list, n, nullptr, nullptr);
   else if (mode == 1)
     hipLaunchKernelGGL((k_chem<NS, 1, K>), dim3(nblocks(n)), dim3(kBlock), 0, s, U, Q, rhoi, dt,
-                       maxiter, rtol, ttol, iters, tag, c->dparams, c->g, bug, list, n);
+                       maxiter, rtol, ttol, iters, tag, c->dparams, c->g, bug, list, n, nullptr, nullptr);
   else
-    hipLaunchKernelGGL((k_chem<NS, 2, K>), dim3(nblocks(n, chem_block(2))), dim3(chem_block(2)), 0, s, U, Q, rhoi, dt,
-                       maxiter, rtol, ttol, iters, tag, c->dparams, c->g, bug, list, n);
+    hipLaunchKernelGGL((k_chem<NS, 2, K>), dim3(nblocks(n, chem_block(2))), dim3(chem_block(2)),
+                       0, s, U, Q, rhoi, dt, maxiter, rtol, ttol, iters, tag, c->dparams, c->g, bug, list, n, later, nlater);
+}
+
+// the list pass's slow cells: as many waves as the device holds stride over them
+template <class T>
+static void launch_rows(f3d_ctx* c, double* U, double* Q, double* rhoi, double dt, int maxiter,
+                        double rtol, double ttol, hipStream_t s, long nlist,
+                        const int32_t* later, const int32_t* nlater) {
+  const long most = std::min(nlist, (long)kRowsMost);
+  const long nb = std::min(resident_blocks(&k_newton_rows<T>, 64, &c->rows_blocks),
+                           (most + kRowCells - 1) / kRowCells);
+  hipLaunchKernelGGL((k_newton_rows<T>), dim3((unsigned)nb), dim3(64), 0, s, U, Q, rhoi, dt,
+                     maxiter, rtol, ttol, c->dparams, c->g, kNewtonMaxSub, later, nlater, kRowsMost);
 }
 
 // the compiled-in tables of the context's mechanism when it is one of the
@@ -281,34 +326,40 @@ static void chem_k(f3d_ctx* c, int mode, double* U, double* Q, double* rhoi, dou
 template <int NS>
 static void chem_ns(f3d_ctx* c, int mode, double* U, double* Q, double* rhoi, double dt,
                     int maxiter, double rtol, double ttol, int32_t* iters, const int64_t* tag,
-                    hipStream_t s, const int32_t* list, long nlist) {
+                    hipStream_t s, const int32_t* list, long nlist, int32_t* later, int32_t* nlater) {
   if constexpr (NS == MechH2LiDryer::NS) {
     if (c->kin_table == F3D_KIN_H2_LIDRYER) {
       chem_k<NS, KinCT<MechH2LiDryer>>(c, mode, U, Q, rhoi, dt, maxiter, rtol, ttol, iters, tag,
-                                       s, list, nlist);
+                                       s, list, nlist, later, nlater);
+      if (later && nlist > 0)
+        launch_rows<MechH2LiDryer>(c, U, Q, rhoi, dt, maxiter, rtol, ttol, s, nlist, later, nlater);
       return;
     }
   }
   if constexpr (NS == MechAir5::NS) {
     if (c->kin_table == F3D_KIN_AIR5) {
       chem_k<NS, KinCT<MechAir5>>(c, mode, U, Q, rhoi, dt, maxiter, rtol, ttol, iters, tag, s,
-                                  list, nlist);
+                                  list, nlist, later, nlater);
+      if (later && nlist > 0)
+        launch_rows<MechAir5>(c, U, Q, rhoi, dt, maxiter, rtol, ttol, s, nlist, later, nlater);
       return;
     }
   }
-  chem_k<NS, KinRT>(c, mode, U, Q, rhoi, dt, maxiter, rtol, ttol, iters, tag, s, list, nlist);
+  chem_k<NS, KinRT>(c, mode, U, Q, rhoi, dt, maxiter, rtol, ttol, iters, tag, s, list, nlist, nullptr,
+                    nullptr);
 }
 
 int launch_chem(f3d_ctx* c, int mode, double* U, double* Q, double* rhoi, double dt,
                 int maxiter, double rtol, double ttol, int32_t* iters, const int64_t* tag,
-                hipStream_t s, const int32_t* list, long nlist) {
+                hipStream_t s, const int32_t* list, long nlist, int32_t* later,
+                int32_t* nlater) {
   if (mode == 0 && (c->bug_compat & 1) && c->g.Ns < 6) {
     set_error("bug_compat coeffs_lo[n,6] read needs Ns >= 6 (it reads past the array for Ns < 6)");
     return F3D_ERR_ARG;
   }
   switch (c->g.Ns) {
-    case 5: chem_ns<5>(c, mode, U, Q, rhoi, dt, maxiter, rtol, ttol, iters, tag, s, list, nlist); break;
-    case 9: chem_ns<9>(c, mode, U, Q, rhoi, dt, maxiter, rtol, ttol, iters, tag, s, list, nlist); break;
+    case 5: chem_ns<5>(c, mode, U, Q, rhoi, dt, maxiter, rtol, ttol, iters, tag, s, list, nlist, later, nlater); break;
+    case 9: chem_ns<9>(c, mode, U, Q, rhoi, dt, maxiter, rtol, ttol, iters, tag, s, list, nlist, later, nlater); break;
     default: set_error("chemistry: Ns must be 5 or 9"); return F3D_ERR_UNSUPPORTED;
   }
   return hip_check(hipGetLastError(), "chem");

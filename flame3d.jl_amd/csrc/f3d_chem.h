@@ -380,6 +380,22 @@ __device__ inline void production_rate(const DevParams* __restrict__ P, const do
         }
       }
     }
+    if constexpr (K::kConst) {
+      // the sums are formed here: deferred, each would keep the terms of
+      // several reactions in registers next to the Jacobian
+#pragma unroll
+      for (int l = 0; l < NS; ++l) {
+        if (Kp.vr(n, l) == Kp.vf(n, l)) continue;
+        asm volatile("" : "+v"(wdot[l]));
+        if (TDER) asm volatile("" : "+v"(A[l][NA - 1]));
+        if (JAC) {
+#pragma unroll
+          for (int m = 0; m < NS; ++m)
+            if (Kp.vf(n, m) != 0 || Kp.vr(n, m) != 0 || (FULL && rt != 1 && Kp.ef(n, m) != 0.0))
+              asm volatile("" : "+v"(A[l][m]));
+        }
+      }
+    }
   });
 }
 
@@ -532,9 +548,7 @@ __device__ inline void production_rate_block3(const NasaTab<NS>& N,
         if (dl != 0) M[i][j] += d * (double)dl;
       }
     }
-    if constexpr (K::kConst) {
-      // the sums are formed here: deferred, each would keep
-      // the terms of several reactions in registers
+    if constexpr (K::kConst) {  // the sums are formed here (see production_rate)
 #pragma unroll
       for (int m = 0; m < NS; ++m)
         if (Kp.vf(n, m) != Kp.vr(n, m)) asm volatile("" : "+v"(wdot[m]));

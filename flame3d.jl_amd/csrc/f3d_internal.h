@@ -65,8 +65,8 @@ struct f3d_ctx {
   int sensor_kind = 0;  // F3D_SENSOR_PRESSURE / F3D_SENSOR_DUCROS
   int stage_kind = 0;   // F3D_STAGE_FUSED / F3D_STAGE_GRANULAR (F3D_FP32 contexts)
   int kin_table = 0;    // F3D_KIN_*: the chemistry kernels' reaction-parameter source
-  // resident blocks of the march kernels on the device (0: not queried)
-  long spec_waves = 0, visc_waves = 0, conv_blocks = 0, weno_waves = 0;
+  // resident blocks of the march kernels and the row solve on the device (0: not queried)
+  long spec_waves = 0, visc_waves = 0, conv_blocks = 0, weno_waves = 0, rows_blocks = 0;
   f3d::DevParams host_params;
   f3d::DevParams* dparams = nullptr;
   // boundary fills
@@ -102,7 +102,7 @@ struct f3d_ctx {
   int8_t* nn_status = nullptr;  // per-cell gate codes [Nx*Ny*Nz] when the caller passes none
   int32_t* nn_fbcount = nullptr;  // rejected cells per 64-cell tile, then their offsets
   int32_t* nn_fblist = nullptr;   // rejected cell ids in cell order [Nx*Ny*Nz]
-  int32_t* nn_fbtotal = nullptr;  // number of rejected cells
+  int32_t* nn_fbtotal = nullptr;  // number of rejected cells, and of those taken a second time
   float* nn_out = nullptr;        // the network's raw outputs [Ns][Nx*Ny*Nz] for the epilogue
   double* nn_cand = nullptr;      // the epilogue's candidate states [Ns + 3][Nx*Ny*Nz]
   // f3d_nn_timing: events around the last f3d_nn_chem's network kernel, its
@@ -624,6 +624,7 @@ int launch_get_y(f3d_ctx* c, double* Yi, const double* rhoi, const double* Q,
 int launch_fill(f3d_ctx* c, double* Q, double* U, double* rhoi, hipStream_t s);
 int launch_chem(f3d_ctx* c, int mode, double* U, double* Q, double* rhoi, double dt,
                 int maxiter, double rtol, double ttol, int32_t* iters, const int64_t* tag,
-                hipStream_t s, const int32_t* list = nullptr, long nlist = 0);
+                hipStream_t s, const int32_t* list = nullptr, long nlist = 0,
+                int32_t* later = nullptr, int32_t* nlater = nullptr);
 
 }  // namespace f3d

@@ -816,7 +816,10 @@ __global__ void __launch_bounds__(1024) k_nn_scan(int32_t* __restrict__ cnt, lon
     cnt[i] = run;
     run += c;
   }
-  if (t == 1023) *total = part[1023];
+  if (t == 1023) {
+    total[0] = part[1023];
+    total[1] = 0;  // the fallback's slow cells, counted by the Newton pass
+  }
 }
 
 // The tile counts are scanned in chunks of kScanChunk tiles: k_scan_sums
@@ -1134,7 +1137,7 @@ int f3d_nn_init(f3d_ctx* c, const f3d_nn_config* cfg) {
                hipMalloc(&c->nn_status, ncell) == hipSuccess &&
                hipMalloc(&c->nn_fbcount, sizeof(int32_t) * (ntile + nchunk)) == hipSuccess &&
                hipMalloc(&c->nn_fblist, sizeof(int32_t) * ncell) == hipSuccess &&
-               hipMalloc(&c->nn_fbtotal, sizeof(int32_t)) == hipSuccess &&
+               hipMalloc(&c->nn_fbtotal, 2 * sizeof(int32_t)) == hipSuccess &&
                hipMalloc(&c->nn_out, sizeof(float) * ncell * ns) == hipSuccess &&
                hipMalloc(&c->nn_cand, sizeof(double) * ncell * (ns + 3)) == hipSuccess;
     if (!okm) {
@@ -1339,7 +1342,7 @@ int f3d_nn_chem(f3d_ctx* c, double* U, double* Q, double* rhoi, double dt, int32
   if (timed) (void)hipEventRecord(c->nn_ev[4], s);  // after the read-back
   if (nfb > 0) {
     rc = launch_chem(c, 2, U, Q, rhoi, dt, maxiter, rtol, ttol, nullptr, tag, s, c->nn_fblist,
-                     nfb);
+                     nfb, reinterpret_cast<int32_t*>(c->nn_out), c->nn_fbtotal + 1);
     if (rc) return rc;
   }
   if (timed) {

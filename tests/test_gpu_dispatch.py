@@ -1,6 +1,9 @@
 """Branches of the launch rules at the sizes where they can go wrong, against
 the FP64 oracle: boundary fills whose two faces share a launch or run in turn,
-and the marches' segment counts on blocks too small to fill the chip."""
+the marches' segment counts on blocks too small to fill the chip, and the
+surrogate fallback's second pass over the cells of many Newton iterations."""
+import os
+
 import numpy as np
 import pytest
 import torch
@@ -74,4 +77,49 @@ def test_stage_on_small_and_ragged_blocks(mech, shape):
     torch.cuda.synchronize()
     for got, ref in ((Qg, Qo), (Ug, U), (rg, ro)):
         assert rel_err(to_np(got), ref) < 1e-12
+    ctx.close()
+
+
+@pytest.mark.parametrize("maxiter", [1, 5, 6, 50])
+@pytest.mark.parametrize("mech,shape", [("h2_lidryer", (32, 31, 9)), ("h2_lidryer", (5, 4, 4)),
+                                        ("air5", (17, 9, 6))])
+def test_fallback_equals_newton(mech, shape, maxiter):
+    """Cells that the surrogate rejects (every reacting one: a chain bound of
+    1e-30) are advanced by a pass over the list and those of more than five
+    iterations, or of a failed first step, by the half-wave solve.  Both form
+    every sum in the order of the Newton mode: equal bit for bit, also where
+    no substep count converges and the cell stays unreacted, and (one
+    iteration allowed) where more cells are slow than the second pass takes."""
+    import flame3d_amd.abi as abi
+    import flame3d_amd.cases as cases
+    import flame3d_amd.mech as mm
+    import flame3d_amd.surrogate as sur
+    m = mm.load(mech)
+    h2 = mech == "h2_lidryer"
+    if h2:
+        Q, r = cases.chem_cells(shape, m, seed=7)
+        dt = sur.DT
+    else:
+        Q, r = cases.chem_cells_air(shape, m, seed=7, T_range=(1500.0, 6000.0),
+                                    P_atm=(0.02, 0.1))
+        dt = sur.AIR_DT
+    Q, r = Q.cuda().contiguous(), r.cuda().contiguous()
+    U = torch.zeros((5,) + tuple(Q.shape[1:]), dtype=torch.float64, device="cuda")
+    ctx = abi.Context(*shape, m, "fp64")
+    path = os.path.join(os.path.dirname(sur.DEFAULT_PATH), "air5_surrogate.npz")
+    sur.attach(ctx, *([] if h2 else [path]), chain_max=1e-30)
+    Un, Qn, rn = U.clone(), Q.clone(), r.clone()
+    it = torch.zeros(shape[::-1], dtype=torch.int32, device="cuda")
+    ctx.chem_newton(Un, Qn, rn, dt, maxiter, 1e-10, 1e-6, iters=it)
+    st = torch.zeros(shape[::-1], dtype=torch.int8, device="cuda")
+    nfb = int(ctx.nn_chem(U, Q, r, dt, maxiter, 1e-10, 1e-6, status=st))
+    torch.cuda.synchronize()
+    print(f"\n[fallback] {mech} {shape} maxiter {maxiter}: {nfb} of {st.numel()} rejected, "
+          f"iterations up to {int(it.abs().max())}, {int((it < 0).sum())} left unreacted")
+    back = st != 1
+    assert int(back.sum()) > st.numel() // 2
+    if h2 and st.numel() > 1000:
+        assert bool((back & ((it.abs() > 5) | (it < 0))).any())  # the second pass had work
+    for got, ref in ((U, Un), (Q, Qn), (r, rn)):
+        assert torch.equal(sur.interior(got)[back.flatten()], sur.interior(ref)[back.flatten()])
     ctx.close()
