@@ -9,7 +9,7 @@
 // decomposition (solver.jl:22-56) never reach HBM; the stage end applies
 // U += J dt rhs (div.jl:16-84), linComb and c2Prim in one pass.
 //
-// x sweeps: one 256-thread block per segment of up to 256 cells of an x line;
+// x sweeps: one block of up to 320 threads per segment of up to 304 cells of an x line;
 // the split fluxes (convective) or the face values (diffusive) of the segment
 // are staged in LDS so each point is read from HBM once and each face is
 // evaluated once; the face-flux difference of a cell reads its two faces
@@ -29,7 +29,18 @@
 
 namespace f3d {
 
-constexpr int kXSeg = 256;  // cells per x-line block
+// x-line blocks: a thread to each staged point (the cells and up to eight more)
+// and at most kXMost cells, a line split into equal segments beyond that.  With
+// 256 cells and 256 threads the staged points past the 256th and the last face
+// were a second pass of the first and of the last wave, the others waiting; a
+// line of 300 cells took a second block of 256 threads for 44 cells.  At
+// 300x127x127 (air): convective 619 -> 461 us, viscous 336 -> 184, species
+// 308 -> 168; at 256^3 (H2/air): 640, 720 -> 639 and 1022 -> 926 us.
+constexpr int kXThreads = 320, kXMost = 304;
+// MOST: the cells a kernel's LDS holds, kXMost (the _long kernels) or this: a
+// sixth less LDS, a block more per compute unit (at 256^3, with the larger:
+// convective 741 us, species 1176 with its face values beside the metrics).
+constexpr int kXFew = 256;
 constexpr int kConvSeg = 32;  // cells per march segment (convective)
 constexpr int kViscSeg = 64;  // cells per march segment (viscous)
 
@@ -37,35 +48,46 @@ __device__ inline void rhs_put(float* __restrict__ r, long i, float d, int acc) 
   r[i] = acc ? r[i] + d : d;
 }
 
+// An x-line block's segment of a line.
+struct XSegment {
+  int b, c, c0, nc;  // line (b, c), first cell, cells
+};
+__device__ inline XSegment x_segment(const Geom& g, int seg) {
+  const unsigned nseg = (g.Nx + seg - 1) / seg;
+  const unsigned L = xcd_block();
+  const unsigned line = L / nseg;
+  XSegment x;
+  x.c0 = (int)(L % nseg) * seg;
+  x.b = (int)(line % g.Ny);
+  x.c = (int)(line / g.Ny);
+  x.nc = min(seg, g.Nx - x.c0);
+  return x;
+}
+
 // ---------------------------------------------------------------------------
 // Convective x sweep
 // ---------------------------------------------------------------------------
-template <int NS>
-__global__ void __launch_bounds__(kXSeg)
-    k_sw_conv_x(float* __restrict__ rhs, const double* __restrict__ Q,
-                const double* __restrict__ rhoi, const float* __restrict__ A1,
-                const float* __restrict__ A2, const float* __restrict__ A3,
-                const float* __restrict__ phi, const DevParams* __restrict__ P, Geom g,
-                int acc) {
+template <int NS, int MOST>
+__device__ __forceinline__ void conv_x_line(
+    float* __restrict__ rhs, const double* __restrict__ Q,
+    const double* __restrict__ rhoi, const float* __restrict__ A1,
+    const float* __restrict__ A2, const float* __restrict__ A3,
+    const float* __restrict__ phi, const DevParams* __restrict__ P, Geom g,
+    int acc, int seg) {
   constexpr int NV = 5 + NS;
-  constexpr int NPT = kXSeg + 8;
+  constexpr int NPT = MOST + 8;
+  static_assert(MOST + 8 <= kXThreads && MOST + NV <= kXThreads, "a thread to a point");
   __shared__ float sp[NV][NPT];
   __shared__ float sm[NV][NPT];
   __shared__ float sphi[NPT];
-  const int nseg = (g.Nx + kXSeg - 1) / kXSeg;
-  const unsigned L = xcd_block();
-  const int seg = (int)(L % (unsigned)nseg);
-  const int line = (int)(L / (unsigned)nseg);
-  const int b = line % g.Ny, c = line / g.Ny;
-  const int c0 = seg * kXSeg;
-  const int nc = min(kXSeg, g.Nx - c0);
+  const XSegment x = x_segment(g, seg);
+  const int nc = x.nc;
   const int t = threadIdx.x;
   const long NP = g.NP;
-  // point q of the segment is padded i = c0 + q (cell c0 + q - NG)
-  const long row = (long)c0 + (long)g.Nxt * ((b + NG) + (long)g.Nyt * (c + NG));
-  const float sw = PT<float>::sweps2(P);
-  for (int q = t; q < nc + 8; q += kXSeg) {
-    const long p = row + q;
+  if (t < nc + 8) {
+    // point t of the segment is padded i = c0 + t (cell c0 + t - NG)
+    const long p = (long)x.c0 + (long)g.Nxt * ((x.b + NG) + (long)g.Nyt * (x.c + NG)) + t;
+    const float sw = PT<float>::sweps2(P);
     const float u = (float)Q[p + NP], v = (float)Q[p + 2 * NP], w = (float)Q[p + 3 * NP];
     const float a1 = A1[p], a2 = A2[p], a3 = A3[p];
     float fp[5], fm[5];
@@ -73,8 +95,8 @@ __global__ void __launch_bounds__(kXSeg)
                        a3, sw, fp, fm);
 #pragma unroll
     for (int n = 0; n < 5; ++n) {
-      sp[n][q] = fp[n];
-      sm[n][q] = fm[n];
+      sp[n][t] = fp[n];
+      sm[n][t] = fm[n];
     }
     const float un = a1 * u + a2 * v + a3 * w;
     const float Ep = 0.5f * (un + fabsf(un));
@@ -82,10 +104,10 @@ __global__ void __launch_bounds__(kXSeg)
 #pragma unroll
     for (int n = 0; n < NS; ++n) {
       const float r = (float)rhoi[p + (long)n * NP];
-      sp[5 + n][q] = Ep * r;
-      sm[5 + n][q] = Em * r;
+      sp[5 + n][t] = Ep * r;
+      sm[5 + n][t] = Em * r;
     }
-    sphi[q] = phi[p];
+    sphi[t] = phi[p];
   }
   __syncthreads();
   // face f (0..nc) between cells c0+f-1 and c0+f: stencil points q = f .. f+7
@@ -100,14 +122,15 @@ __global__ void __launch_bounds__(kXSeg)
       }
     }, fv);
   }
-  // the segment's last face, one variable per thread
+  // the segment's last face, one variable per thread of those after the cells
   float fl = 0.0f;
-  if (t < NV) {
+  const int n1 = t - nc;
+  if (n1 >= 0 && n1 < NV) {
     const int br = weno_branch<float>(fmaxf(sphi[nc + 3], sphi[nc + 4]), P);
     float pv[8], mv[8];
     for (int k = 0; k < 8; ++k) {
-      pv[k] = sp[t][nc + k];
-      mv[k] = sm[t][nc + k];
+      pv[k] = sp[n1][nc + k];
+      mv[k] = sm[n1][nc + k];
     }
     fl = weno_face_v<float>(pv, mv, br, P);
   }
@@ -117,14 +140,36 @@ __global__ void __launch_bounds__(kXSeg)
 #pragma unroll
     for (int n = 0; n < NV; ++n) sf[n][t] = fv[n];
   }
-  if (t < NV) sf[t][nc] = fl;
+  if (n1 >= 0 && n1 < NV) sf[n1][nc] = fl;
   __syncthreads();
   if (t < nc) {
     const long NC = (long)g.Nx * g.Ny * g.Nz;
-    const long cell = (c0 + t) + (long)g.Nx * (b + (long)g.Ny * c);
+    const long cell = (x.c0 + t) + (long)g.Nx * (x.b + (long)g.Ny * x.c);
 #pragma unroll
     for (int n = 0; n < NV; ++n) rhs_put(rhs, n * NC + cell, sf[n][t] - sf[n][t + 1], acc);
   }
+}
+
+template <int NS>
+__global__ void __launch_bounds__(kXThreads)
+    k_sw_conv_x(
+        float* __restrict__ rhs, const double* __restrict__ Q,
+        const double* __restrict__ rhoi, const float* __restrict__ A1,
+        const float* __restrict__ A2, const float* __restrict__ A3,
+        const float* __restrict__ phi, const DevParams* __restrict__ P, Geom g,
+        int acc, int seg) {
+  conv_x_line<NS, kXFew>(rhs, Q, rhoi, A1, A2, A3, phi, P, g, acc, seg);
+}
+
+template <int NS>
+__global__ void __launch_bounds__(kXThreads)
+    k_sw_conv_x_long(
+        float* __restrict__ rhs, const double* __restrict__ Q,
+        const double* __restrict__ rhoi, const float* __restrict__ A1,
+        const float* __restrict__ A2, const float* __restrict__ A3,
+        const float* __restrict__ phi, const DevParams* __restrict__ P, Geom g,
+        int acc, int seg) {
+  conv_x_line<NS, kXMost>(rhs, Q, rhoi, A1, A2, A3, phi, P, g, acc, seg);
 }
 
 // ---------------------------------------------------------------------------
@@ -407,87 +452,81 @@ struct FMet {
 // two cells (viscous.jl:1-142: the face average of the cells' transverse
 // differences, the fourth-order normal difference), then its stresses and
 // heat flux; the face values go back to LDS for the difference of each
-// cell's two faces (rhs 1..4).  A full segment has kXSeg + 1 faces: its last
-// thread also takes the last face.
-__global__ void __launch_bounds__(kXSeg)
-    k_sw_visc_x(float* __restrict__ rhs, const double* __restrict__ Q, FMet M,
-                const float* __restrict__ J, const float* __restrict__ lam,
-                const float* __restrict__ mu, Geom g) {
-  constexpr int NE = kXSeg + 2;  // cells -1 .. nc
-  constexpr int NQ = kXSeg + 4;  // cells -2 .. nc + 1
-  __shared__ float sm[12][NE];   // metrics, J, mu, lambda
+// cell's two faces (rhs 1..4).  Thread t takes staged entry t and face t.
+template <int MOST>
+__device__ __forceinline__ void visc_x_line(
+    float* __restrict__ rhs, const double* __restrict__ Q, FMet M,
+    const float* __restrict__ J, const float* __restrict__ lam,
+    const float* __restrict__ mu, Geom g, int seg) {
+  constexpr int NE = MOST + 2;  // cells -1 .. nc
+  constexpr int NQ = MOST + 4;  // cells -2 .. nc + 1
+  __shared__ float sm[12][NE];    // metrics, J, mu, lambda
   __shared__ float sq[2][NQ], sy[2][NE], sz[2][NE];
-  __shared__ float sf[4][kXSeg + 1];
-  const int nseg = (g.Nx + kXSeg - 1) / kXSeg;
-  const unsigned L = xcd_block();
-  const int seg = (int)(L % (unsigned)nseg);
-  const int line = (int)(L / (unsigned)nseg);
-  const int b = line % g.Ny, c = line / g.Ny;
-  const int c0 = seg * kXSeg;
-  const int nc = min(kXSeg, g.Nx - c0);
+  __shared__ float sf[4][MOST + 1];
+  const XSegment x = x_segment(g, seg);
+  const int nc = x.nc;
   const int t = threadIdx.x;
   const long NP = g.NP, ty = g.Nxt, tz = (long)g.Nxt * g.Nyt;
-  const long row = (long)(c0 + NG) + ty * (b + NG) + tz * (c + NG);  // cell 0
+  const long row = (long)(x.c0 + NG) + ty * (x.b + NG) + tz * (x.c + NG);  // cell 0
   const int qv[4] = {1, 2, 3, 5};  // u, v, w, T
-  // variable k's loads of entries t and t + kXSeg of the staged ranges (the
-  // second exists for t < 4 in a full segment)
-  double rq[2], rt[2][8];
+  const bool pq = t < nc + 4, pe = t < nc + 2;
+  // variable k's loads of entry t of the staged ranges
+  double rq, rt[8];
   auto fetch = [&](int k) {
     const double* fq = Q + qv[k] * NP;
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int i = t + j * kXSeg;
-      if (i < nc + 4) rq[j] = fq[row + i - 2];
-      if (i < nc + 2) {
-        const long ic = row + i - 1;
-        rt[j][0] = fq[ic + ty];
-        rt[j][1] = fq[ic - ty];
-        rt[j][2] = fq[ic + 2 * ty];
-        rt[j][3] = fq[ic - 2 * ty];
-        rt[j][4] = fq[ic + tz];
-        rt[j][5] = fq[ic - tz];
-        rt[j][6] = fq[ic + 2 * tz];
-        rt[j][7] = fq[ic - 2 * tz];
-      }
+    if (pq) rq = fq[row + t - 2];
+    if (pe) {
+      const long ic = row + t - 1;
+      rt[0] = fq[ic + ty];
+      rt[1] = fq[ic - ty];
+      rt[2] = fq[ic + 2 * ty];
+      rt[3] = fq[ic - 2 * ty];
+      rt[4] = fq[ic + tz];
+      rt[5] = fq[ic - tz];
+      rt[6] = fq[ic + 2 * tz];
+      rt[7] = fq[ic - 2 * tz];
     }
   };
   fetch(0);
-  for (int i = t; i < nc + 2; i += kXSeg) {
-    const long ic = row + i - 1;
+  if (pe) {
+    const long ic = row + t - 1;
 #pragma unroll
-    for (int q = 0; q < 9; ++q) sm[q][i] = M.m[q][ic];
-    sm[9][i] = J[ic];
-    sm[10][i] = mu[ic];
-    sm[11][i] = lam[ic];
+    for (int q = 0; q < 9; ++q) sm[q][t] = M.m[q][ic];
+    sm[9][t] = J[ic];
+    sm[10][t] = mu[ic];
+    sm[11][t] = lam[ic];
   }
   const float c12 = 1.0f / 12.0f, c23 = 2.0f / 3.0f;
-  const bool own = t <= nc;                          // face t
-  const bool extra = nc == kXSeg && t == kXSeg - 1;  // and face kXSeg
-  float dq[4][3], vel[3], dx[4][3], vx[3];           // face t's and the extra face's
-  auto grads = [&](int f, int bb, int k, float (&d)[4][3], float (&vv)[3]) {
-    d[k][0] = 1.25f * (sq[bb][f + 2] - sq[bb][f + 1]) - c12 * (sq[bb][f + 3] - sq[bb][f]);
-    d[k][1] = 0.5f * (sy[bb][f] + sy[bb][f + 1]);
-    d[k][2] = 0.5f * (sz[bb][f] + sz[bb][f + 1]);
-    if (k < 3) vv[k] = (sq[bb][f + 1] + sq[bb][f + 2]) * 0.5f;
-  };
+  const bool own = t <= nc;  // face t
+  float d[4][3], vv[3];
+  // the right-hand side that the block adds to, on its way since the last variable
+  const long NC = (long)g.Nx * g.Ny * g.Nz;
+  const long cell = (x.c0 + t) + (long)g.Nx * (x.b + (long)g.Ny * x.c);
+  float old[4];
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
     const int bb = k & 1;
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int i = t + j * kXSeg;
-      if (i < nc + 4) sq[bb][i] = (float)rq[j];
-      if (i < nc + 2) {
-        sy[bb][i] = c23 * ((float)rt[j][0] - (float)rt[j][1]) - c12 * ((float)rt[j][2] - (float)rt[j][3]);
-        sz[bb][i] = c23 * ((float)rt[j][4] - (float)rt[j][5]) - c12 * ((float)rt[j][6] - (float)rt[j][7]);
-      }
+    if (pq) sq[bb][t] = (float)rq;
+    if (pe) {
+      sy[bb][t] = c23 * ((float)rt[0] - (float)rt[1]) - c12 * ((float)rt[2] - (float)rt[3]);
+      sz[bb][t] = c23 * ((float)rt[4] - (float)rt[5]) - c12 * ((float)rt[6] - (float)rt[7]);
     }
-    if (k + 1 < 4) fetch(k + 1);
+    if (k + 1 < 4) {
+      fetch(k + 1);
+    } else if (t < nc) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) old[q] = rhs[(q + 1) * NC + cell];
+    }
     __syncthreads();
-    if (own) grads(t, bb, k, dq, vel);
-    if (extra) grads(kXSeg, bb, k, dx, vx);
+    if (own) {
+      d[k][0] = 1.25f * (sq[bb][t + 2] - sq[bb][t + 1]) - c12 * (sq[bb][t + 3] - sq[bb][t]);
+      d[k][1] = 0.5f * (sy[bb][t] + sy[bb][t + 1]);
+      d[k][2] = 0.5f * (sz[bb][t] + sz[bb][t + 1]);
+      if (k < 3) vv[k] = (sq[bb][t + 1] + sq[bb][t + 2]) * 0.5f;
+    }
   }
-  auto stress = [&](int f, const float (&d)[4][3], const float (&vv)[3]) {
+  if (own) {
+    const int f = t;
     float m[9];
 #pragma unroll
     for (int q = 0; q < 9; ++q) m[q] = (sm[q][f] + sm[q][f + 1]) * 0.5f;
@@ -516,17 +555,29 @@ __global__ void __launch_bounds__(kXSeg)
     sf[1][f] = n0 * t12 + n1 * t22 + n2 * t23;
     sf[2][f] = n0 * t13 + n1 * t23 + n2 * t33;
     sf[3][f] = n0 * E1 + n1 * E2 + n2 * E3;
-  };
-  if (own) stress(t, dq, vel);
-  if (extra) stress(kXSeg, dx, vx);
+  }
   __syncthreads();
   if (t < nc) {
-    const long NC = (long)g.Nx * g.Ny * g.Nz;
-    const long cell = (c0 + t) + (long)g.Nx * (b + (long)g.Ny * c);
     // diffusive fluxes enter with the opposite sign of the convective ones
 #pragma unroll
-    for (int q = 0; q < 4; ++q) rhs_put(rhs, (q + 1) * NC + cell, sf[q][t + 1] - sf[q][t], 1);
+    for (int q = 0; q < 4; ++q) rhs[(q + 1) * NC + cell] = old[q] + (sf[q][t + 1] - sf[q][t]);
   }
+}
+
+__global__ void __launch_bounds__(kXThreads)
+    k_sw_visc_x(
+        float* __restrict__ rhs, const double* __restrict__ Q, FMet M,
+        const float* __restrict__ J, const float* __restrict__ lam,
+        const float* __restrict__ mu, Geom g, int seg) {
+  visc_x_line<kXFew>(rhs, Q, M, J, lam, mu, g, seg);
+}
+
+__global__ void __launch_bounds__(kXThreads)
+    k_sw_visc_x_long(
+        float* __restrict__ rhs, const double* __restrict__ Q, FMet M,
+        const float* __restrict__ J, const float* __restrict__ lam,
+        const float* __restrict__ mu, Geom g, int seg) {
+  visc_x_line<kXMost>(rhs, Q, M, J, lam, mu, g, seg);
 }
 
 // x-line block of the species-diffusion sweep with each cell's inputs read
@@ -536,156 +587,149 @@ __global__ void __launch_bounds__(kXSeg)
 // species, the next species' loads in flight across it); face f (between
 // cells f-1 and f) forms its gradient from them
 // (viscous.jl:430-507: the face average of the cells' transverse central
-// differences, the fourth-order normal difference).  A full segment has
-// nc + 1 = kXSeg + 1 faces: its last thread also takes the last face.
-template <int NS>
-__global__ void __launch_bounds__(kXSeg)
-    k_sw_spec_x(float* __restrict__ rhs, const double* __restrict__ Q,
-                const float* __restrict__ Yi, FMet M, const float* __restrict__ J,
-                const float* __restrict__ D, const DevParams* __restrict__ P, Geom g) {
-  constexpr int NE = kXSeg + 2;  // cells -1 .. nc
-  constexpr int NY = kXSeg + 4;  // cells -2 .. nc + 1
-  __shared__ float sm[12][NE];   // metrics, J, rho, T
+// differences, the fourth-order normal difference).  Thread t takes staged
+// entry t and face t, whose metrics it keeps over the species.  Bound by the
+// latency of a block's chain of loads and barriers, so by the blocks that fit a
+// compute unit: the metrics' LDS is used again for the face values and the
+// registers are held to 72 (at 256^3, 1176 us with 76 and 941 with 72; the
+// right-hand side fetched with the last species: 926).
+template <int NS, int MOST>
+__device__ __forceinline__ void spec_x_line(
+    float* __restrict__ rhs, const double* __restrict__ Q,
+    const float* __restrict__ Yi, FMet M, const float* __restrict__ J,
+    const float* __restrict__ D, const DevParams* __restrict__ P, Geom g, int seg) {
+  constexpr int NE = MOST + 2;  // cells -1 .. nc
+  constexpr int NY = MOST + 4;  // cells -2 .. nc + 1
   __shared__ float sy[2][NY], scy[2][NE], scz[2][NE], sd[2][NE];
-  __shared__ float sf[NS + 1][kXSeg + 1];
-  __shared__ float sx[4][NS];  // the extra face's V_x, V_y, V_z and Y
-  const int nseg = (g.Nx + kXSeg - 1) / kXSeg;
-  const unsigned L = xcd_block();
-  const int seg = (int)(L % (unsigned)nseg);
-  const int line = (int)(L / (unsigned)nseg);
-  const int b = line % g.Ny, c = line / g.Ny;
-  const int c0 = seg * kXSeg;
-  const int nc = min(kXSeg, g.Nx - c0);
+  __shared__ union {
+    float m[12][NE];            // metrics, J, rho, T, read at the first species
+    float f[NS + 1][MOST + 1];  // face values, written after the last
+  } sh;
+  auto& sm = sh.m;
+  auto& sf = sh.f;
+  const XSegment x = x_segment(g, seg);
+  const int nc = x.nc;
   const int t = threadIdx.x;
   const long NP = g.NP, ty = g.Nxt, tz = (long)g.Nxt * g.Nyt;
-  const long row = (long)(c0 + NG) + ty * (b + NG) + tz * (c + NG);  // cell 0
-  for (int i = t; i < nc + 2; i += kXSeg) {
-    const long ic = row + i - 1;
-#pragma unroll
-    for (int q = 0; q < 9; ++q) sm[q][i] = M.m[q][ic];
-    sm[9][i] = J[ic];
-    sm[10][i] = (float)Q[ic];
-    sm[11][i] = (float)Q[ic + 5 * NP];
-  }
-  const bool own = t <= nc;                       // face t
-  const bool extra = nc == kXSeg && t == kXSeg - 1;  // and face kXSeg
-  const float c12 = 1.0f / 12.0f;
-  float V[3][NS], Yn[NS];
-  // V_k of face f (staged index f: cell f-1, f + 1: cell f) for species n
-  auto fspec = [&](int f, int bb, float* out) {
-    float m[9];
-#pragma unroll
-    for (int q = 0; q < 9; ++q) m[q] = (sm[q][f] + sm[q][f + 1]) * 0.5f;
-    const float Jac = (sm[9][f] + sm[9][f + 1]) * 0.5f;
-    const float rho = (sm[10][f] + sm[10][f + 1]) * 0.5f;
-    const float rhoDi = (sd[bb][f] + sd[bb][f + 1]) * rho;
-    const float dY0 = 1.25f * (sy[bb][f + 2] - sy[bb][f + 1]) - c12 * (sy[bb][f + 3] - sy[bb][f]);
-    const float dY1 = 0.25f * (scy[bb][f + 1] + scy[bb][f]);
-    const float dY2 = 0.25f * (scz[bb][f + 1] + scz[bb][f]);
-    out[0] = (dY0 * m[0] + dY1 * m[3] + dY2 * m[6]) * Jac * rhoDi;
-    out[1] = (dY0 * m[1] + dY1 * m[4] + dY2 * m[7]) * Jac * rhoDi;
-    out[2] = (dY0 * m[2] + dY1 * m[5] + dY2 * m[8]) * Jac * rhoDi;
-    out[3] = 0.5f * (sy[bb][f + 1] + sy[bb][f + 2]);
-  };
+  const long row = (long)(x.c0 + NG) + ty * (x.b + NG) + tz * (x.c + NG);  // cell 0
+  const bool py = t < nc + 4, pe = t < nc + 2;
   // species n + 1's loads are issued before species n's barrier and faces
-  // (entries t and t + kXSeg of the staged ranges; the second exists for
-  // t < 4 in a full segment)
-  float ry[2], rt[2][5];
+  float ry, rt[5];
   auto fetch = [&](int n) {
     const float* y = Yi + (long)n * NP;
-#pragma unroll
-    for (int k = 0; k < 2; ++k) {
-      const int i = t + k * kXSeg;
-      if (i < nc + 4) ry[k] = y[row + i - 2];
-      if (i < nc + 2) {
-        const long ic = row + i - 1;
-        rt[k][0] = y[ic + ty];
-        rt[k][1] = y[ic - ty];
-        rt[k][2] = y[ic + tz];
-        rt[k][3] = y[ic - tz];
-        rt[k][4] = D[ic + (long)n * NP];
-      }
+    if (py) ry = y[row + t - 2];
+    if (pe) {
+      const long ic = row + t - 1;
+      rt[0] = y[ic + ty];
+      rt[1] = y[ic - ty];
+      rt[2] = y[ic + tz];
+      rt[3] = y[ic - tz];
+      rt[4] = D[ic + (long)n * NP];
     }
   };
   fetch(0);
+  if (pe) {
+    const long ic = row + t - 1;
+#pragma unroll
+    for (int q = 0; q < 9; ++q) sm[q][t] = M.m[q][ic];
+    sm[9][t] = J[ic];
+    sm[10][t] = (float)Q[ic];
+    sm[11][t] = (float)Q[ic + 5 * NP];
+  }
+  const bool own = t <= nc;  // face t
+  const float c12 = 1.0f / 12.0f;
+  float V[3][NS], Yn[NS];
+  float m[9], Jac, rho, T;  // of the face
+  // the right-hand side that the block adds to, on its way since the last species
+  const long NC = (long)g.Nx * g.Ny * g.Nz;
+  const long cell = (x.c0 + t) + (long)g.Nx * (x.b + (long)g.Ny * x.c);
+  float old[NS + 1];
 #pragma unroll
   for (int n = 0; n < NS; ++n) {
     const int bb = n & 1;
-#pragma unroll
-    for (int k = 0; k < 2; ++k) {
-      const int i = t + k * kXSeg;
-      if (i < nc + 4) sy[bb][i] = ry[k];
-      if (i < nc + 2) {
-        scy[bb][i] = rt[k][0] - rt[k][1];
-        scz[bb][i] = rt[k][2] - rt[k][3];
-        sd[bb][i] = rt[k][4];
-      }
+    if (py) sy[bb][t] = ry;
+    if (pe) {
+      scy[bb][t] = rt[0] - rt[1];
+      scz[bb][t] = rt[2] - rt[3];
+      sd[bb][t] = rt[4];
     }
-    if (n + 1 < NS) fetch(n + 1);
+    if (n + 1 < NS) {
+      fetch(n + 1);
+    } else if (t < nc) {
+#pragma unroll
+      for (int k = 0; k <= NS; ++k) old[k] = rhs[(k < NS ? 5 + k : 4) * NC + cell];
+    }
     __syncthreads();
-    float o[4];
     if (own) {
-      fspec(t, bb, o);
-      V[0][n] = o[0];
-      V[1][n] = o[1];
-      V[2][n] = o[2];
-      Yn[n] = o[3];
-    }
-    if (extra) {
-      fspec(kXSeg, bb, o);
+      if (n == 0) {
 #pragma unroll
-      for (int k = 0; k < 4; ++k) sx[k][n] = o[k];
+        for (int q = 0; q < 9; ++q) m[q] = (sm[q][t] + sm[q][t + 1]) * 0.5f;
+        Jac = (sm[9][t] + sm[9][t + 1]) * 0.5f;
+        rho = (sm[10][t] + sm[10][t + 1]) * 0.5f;
+        T = (sm[11][t] + sm[11][t + 1]) * 0.5f;
+      }
+      const float rhoDi = (sd[bb][t] + sd[bb][t + 1]) * rho;
+      const float dY0 =
+          1.25f * (sy[bb][t + 2] - sy[bb][t + 1]) - c12 * (sy[bb][t + 3] - sy[bb][t]);
+      const float dY1 = 0.25f * (scy[bb][t + 1] + scy[bb][t]);
+      const float dY2 = 0.25f * (scz[bb][t + 1] + scz[bb][t]);
+      V[0][n] = (dY0 * m[0] + dY1 * m[3] + dY2 * m[6]) * Jac * rhoDi;
+      V[1][n] = (dY0 * m[1] + dY1 * m[4] + dY2 * m[7]) * Jac * rhoDi;
+      V[2][n] = (dY0 * m[2] + dY1 * m[5] + dY2 * m[8]) * Jac * rhoDi;
+      Yn[n] = 0.5f * (sy[bb][t + 1] + sy[bb][t + 2]);
     }
   }
   // the face's corrected diffusion velocities, its species fluxes and the
   // enthalpy flux n . sum_k V_k h_k
-  auto ffin = [&](int f, const float (&Vf)[3][NS], const float (&Yf)[NS]) {
-    const float n0 = (sm[0][f] + sm[0][f + 1]) * 0.5f;
-    const float n1 = (sm[1][f] + sm[1][f + 1]) * 0.5f;
-    const float n2 = (sm[2][f] + sm[2][f + 1]) * 0.5f;
-    const float T = (sm[11][f] + sm[11][f + 1]) * 0.5f;
+  if (NS == 1) __syncthreads();  // with more species a barrier lies between the uses of sh
+  if (own) {
+    const float n0 = m[0], n1 = m[1], n2 = m[2];
     float hi[NS];
     h_specs<NS, float>(P, T, hi);
     float s1 = 0, s2 = 0, s3 = 0;
 #pragma unroll
     for (int n = 0; n < NS; ++n) {
-      s1 += Vf[0][n];
-      s2 += Vf[1][n];
-      s3 += Vf[2][n];
+      s1 += V[0][n];
+      s2 += V[1][n];
+      s3 += V[2][n];
     }
     float fh1 = 0, fh2 = 0, fh3 = 0;
 #pragma unroll
     for (int n = 0; n < NS; ++n) {
-      const float V1 = Vf[0][n] - s1 * Yf[n];
-      const float V2 = Vf[1][n] - s2 * Yf[n];
-      const float V3 = Vf[2][n] - s3 * Yf[n];
-      sf[n][f] = V1 * n0 + V2 * n1 + V3 * n2;
+      const float V1 = V[0][n] - s1 * Yn[n];
+      const float V2 = V[1][n] - s2 * Yn[n];
+      const float V3 = V[2][n] - s3 * Yn[n];
+      sf[n][t] = V1 * n0 + V2 * n1 + V3 * n2;
       fh1 += V1 * hi[n];
       fh2 += V2 * hi[n];
       fh3 += V3 * hi[n];
     }
-    sf[NS][f] = n0 * fh1 + n1 * fh2 + n2 * fh3;
-  };
-  if (own) ffin(t, V, Yn);
-  if (extra) {
-    float Vx[3][NS], Yx[NS];
-#pragma unroll
-    for (int n = 0; n < NS; ++n) {
-      Vx[0][n] = sx[0][n];
-      Vx[1][n] = sx[1][n];
-      Vx[2][n] = sx[2][n];
-      Yx[n] = sx[3][n];
-    }
-    ffin(kXSeg, Vx, Yx);
+    sf[NS][t] = n0 * fh1 + n1 * fh2 + n2 * fh3;
   }
   __syncthreads();
   if (t < nc) {
-    const long NC = (long)g.Nx * g.Ny * g.Nz;
-    const long cell = (c0 + t) + (long)g.Nx * (b + (long)g.Ny * c);
 #pragma unroll
-    for (int n = 0; n < NS; ++n) rhs_put(rhs, (5 + n) * NC + cell, sf[n][t + 1] - sf[n][t], 1);
-    rhs_put(rhs, 4 * NC + cell, sf[NS][t + 1] - sf[NS][t], 1);
+    for (int n = 0; n <= NS; ++n)
+      rhs[(n < NS ? 5 + n : 4) * NC + cell] = old[n] + (sf[n][t + 1] - sf[n][t]);
   }
+}
+
+template <int NS>
+__global__ void __launch_bounds__(kXThreads) __attribute__((amdgpu_waves_per_eu(7)))
+    k_sw_spec_x(
+        float* __restrict__ rhs, const double* __restrict__ Q,
+        const float* __restrict__ Yi, FMet M, const float* __restrict__ J,
+        const float* __restrict__ D, const DevParams* __restrict__ P, Geom g, int seg) {
+  spec_x_line<NS, kXFew>(rhs, Q, Yi, M, J, D, P, g, seg);
+}
+
+template <int NS>
+__global__ void __launch_bounds__(kXThreads) __attribute__((amdgpu_waves_per_eu(7)))
+    k_sw_spec_x_long(
+        float* __restrict__ rhs, const double* __restrict__ Q,
+        const float* __restrict__ Yi, FMet M, const float* __restrict__ J,
+        const float* __restrict__ D, const DevParams* __restrict__ P, Geom g, int seg) {
+  spec_x_line<NS, kXMost>(rhs, Q, Yi, M, J, D, P, g, seg);
 }
 
 // ---------------------------------------------------------------------------
@@ -1006,6 +1050,21 @@ __global__ void __launch_bounds__(kBlock)
 }
 
 // ---- launchers --------------------------------------------------------------
+// Segment length, blocks and threads (a multiple of a wave that holds a
+// segment's cells and `more` staged points) of the x-line kernels.
+struct XLaunch {
+  int seg;
+  unsigned blocks, threads;
+};
+static XLaunch x_launch(const Geom& g, int more) {
+  const int nseg = (g.Nx + kXMost - 1) / kXMost;
+  XLaunch l;
+  l.seg = (g.Nx + nseg - 1) / nseg;
+  l.blocks = (unsigned)((g.Nx + l.seg - 1) / l.seg) * g.Ny * g.Nz;
+  l.threads = (l.seg + more + 63) / 64 * 64;
+  return l;
+}
+
 // Convective sweep of direction dir into rhs (acc = 0: the first sweep of the
 // stage stores, later sweeps add).  A[3]: the sweep's metrics (float copies).
 template <int NS>
@@ -1013,10 +1072,10 @@ static void conv_ns(f3d_ctx* c, int dir, float* rhs, const double* Q, const doub
                     const float* const* A, const float* phi, int acc, hipStream_t s) {
   const Geom& g = c->g;
   if (dir == 0) {
-    const int nseg = (g.Nx + kXSeg - 1) / kXSeg;
-    const long nb = (long)nseg * g.Ny * g.Nz;
-    hipLaunchKernelGGL((k_sw_conv_x<NS>), dim3((unsigned)nb), dim3(kXSeg), 0, s, rhs, Q, rhoi,
-                       A[0], A[1], A[2], phi, c->dparams, g, acc);
+    const XLaunch l = x_launch(g, std::max(8, 5 + NS));
+    const auto k = l.seg <= kXFew ? k_sw_conv_x<NS> : k_sw_conv_x_long<NS>;
+    hipLaunchKernelGGL(k, dim3(l.blocks), dim3(l.threads), 0, s, rhs, Q, rhoi,
+                       A[0], A[1], A[2], phi, c->dparams, g, acc, l.seg);
   } else {
     const int nd = dir == 1 ? g.Ny : g.Nz;
     const unsigned nl = (g.Nx + 63) / 64, nt = dir == 1 ? g.Nz : g.Ny;
@@ -1056,12 +1115,13 @@ static void diff_ns(f3d_ctx* c, int dir, float* rhs, const double* Q, const floa
                     const float* D, hipStream_t s) {
   const Geom& g = c->g;
   if (dir == 0) {
-    const int nseg = (g.Nx + kXSeg - 1) / kXSeg;
-    const long nb = (long)nseg * g.Ny * g.Nz;
-    hipLaunchKernelGGL(k_sw_visc_x, dim3((unsigned)nb), dim3(kXSeg), 0, s, rhs, Q, M, J, lam, mu,
-                       g);
-    hipLaunchKernelGGL((k_sw_spec_x<NS>), dim3((unsigned)nb), dim3(kXSeg), 0, s, rhs, Q, Yi, M,
-                       J, D, c->dparams, g);
+    const XLaunch l = x_launch(g, 4);
+    const auto kv = l.seg <= kXFew ? k_sw_visc_x : k_sw_visc_x_long;
+    const auto ks = l.seg <= kXFew ? k_sw_spec_x<NS> : k_sw_spec_x_long<NS>;
+    hipLaunchKernelGGL(kv, dim3(l.blocks), dim3(l.threads), 0, s, rhs, Q, M, J, lam, mu,
+                       g, l.seg);
+    hipLaunchKernelGGL(ks, dim3(l.blocks), dim3(l.threads), 0, s, rhs, Q, Yi, M,
+                       J, D, c->dparams, g, l.seg);
   } else {
     const int nd = dir == 1 ? g.Ny : g.Nz;
     const unsigned nl = (g.Nx + 63) / 64, nt = dir == 1 ? g.Nz : g.Ny;

@@ -1,7 +1,7 @@
 """Branches of the launch rules at the sizes where they can go wrong, against
 the FP64 oracle: boundary fills whose two faces share a launch or run in turn,
-the marches' segment counts on blocks too small to fill the chip, and the
-surrogate fallback's second pass over the cells of many Newton iterations."""
+the marches' segment counts on blocks too small to fill the chip, the x-line
+kernels' segments, and the surrogate fallback's second pass over the cells of many Newton iterations."""
 import os
 
 import numpy as np
@@ -123,3 +123,22 @@ def test_fallback_equals_newton(mech, shape, maxiter):
     for got, ref in ((U, Un), (Q, Qn), (r, rn)):
         assert torch.equal(sur.interior(got)[back.flatten()], sur.interior(ref)[back.flatten()])
     ctx.close()
+
+
+@pytest.mark.parametrize("mech,nx,scheme", [
+    ("air5", 4, None), ("air5", 56, "weno7"), ("air5", 60, None), ("h2_lidryer", 61, None),
+    ("h2_lidryer", 256, None), ("h2_lidryer", 257, "weno7"), ("air5", 304, "weno7"),
+    ("air5", 305, None), ("h2_lidryer", 305, None), ("air5", 609, "weno7")])
+def test_x_line_segments(mech, nx, scheme):
+    """The fused FP32 stage on x lines at the edges of its rules: the smallest,
+    those whose cells and staged points just fill or just exceed a number of
+    waves, the largest of the smaller and of the larger LDS tile, and lines of
+    two and three segments; the granular stage's bars of test_gpu_sweeps."""
+    import flame3d_amd.abi as abi
+    from test_gpu_sweeps import _cmp, _stage_pair
+    sc = {"recon_kind": abi.RECON_WENO7} if scheme else None
+    print(f"\n[x lines] {mech} nx={nx} {scheme}", flush=True)
+    f, g = _stage_pair(mech, (nx, 5, 6), scheme=sc)
+    _cmp(f[0], g[0], "dU", 1e-4)
+    _cmp(f[1], g[1], "drho_k", 1e-4)
+    _cmp(f[2], g[2], "Q", 1e-5)
