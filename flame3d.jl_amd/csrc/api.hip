@@ -730,11 +730,14 @@ int f3d_rk3_stage(f3d_ctx* c, int32_t KRK, double* U, double* Un, double* rhoi, 
     RET(launch_sweep_stage_end(c, KRK, U, Un, rhoi, rhon, Q, rhs, dt, J, s));
     return launch_fill(c, Q, U, rhoi, s);
   }
-  // FP64 without a tag: the x sweep splits and reconstructs in one pass, so
+  // FP64 without a tag: the x and y sweeps split and reconstruct in one pass;
   // Fp, Fm hold the z sweep's split fluxes afterwards as they do here (with a
   // tag, points that the split skips keep an earlier sweep's values)
-  const int d0 = (!mf && !tag) ? 1 : 0;
-  if (d0) RET(launch_conv_x(c, w[W_Fx], w[W_Fxi], w[W_phi], Q, rhoi, M, s));
+  const int d0 = (!mf && !tag) ? 2 : 0;
+  if (d0) {
+    RET(launch_conv_x(c, w[W_Fx], w[W_Fxi], w[W_phi], Q, rhoi, M, s));
+    RET(launch_conv_y(c, w[W_Fy], w[W_Fyi], w[W_phi], Q, rhoi, M, s));
+  }
   // specAdvance, solver.jl:40-56
   for (int d = d0; d < 3; ++d) {
     RET(launch_species_split(c, rhoi, Q, w[W_Fpi], w[W_Fmi], M[3 * d], M[3 * d + 1],

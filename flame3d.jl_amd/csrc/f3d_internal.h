@@ -66,7 +66,8 @@ struct f3d_ctx {
   int stage_kind = 0;   // F3D_STAGE_FUSED / F3D_STAGE_GRANULAR (F3D_FP32 contexts)
   int kin_table = 0;    // F3D_KIN_*: the chemistry kernels' reaction-parameter source
   // resident blocks of the march kernels and the row solve on the device (0: not queried)
-  long spec_waves = 0, visc_waves = 0, conv_blocks = 0, weno_waves = 0, rows_blocks = 0;
+  long spec_waves = 0, visc_waves = 0, conv_blocks = 0, weno_waves = 0, rows_blocks = 0,
+       fuse_blocks = 0;
   f3d::DevParams host_params;
   f3d::DevParams* dparams = nullptr;
   // boundary fills
@@ -583,6 +584,8 @@ int launch_weno(f3d_ctx* c, int dir, void* F, const void* phi, const void* Fp, c
 // x sweep of both variable groups, splitting and reconstruction fused (FP64,
 // no tag): F [faces, 5], Fi [faces, Ns]; M: the sweep's three metrics
 int launch_conv_x(f3d_ctx* c, void* F, void* Fi, const void* phi, const double* Q,
+                  const double* rhoi, const void* const* M, hipStream_t s);
+int launch_conv_y(f3d_ctx* c, void* F, void* Fi, const void* phi, const double* Q,
                   const double* rhoi, const void* const* M, hipStream_t s);
 int launch_viscous(f3d_ctx* c, int dir, void* Fv, const double* Q, const void* const* M,
                    const void* J, const void* lam, const void* mu, const void* Fh,

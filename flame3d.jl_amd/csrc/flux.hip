@@ -357,6 +357,196 @@ int launch_conv_x(f3d_ctx* c, void* F, void* Fi, const void* phi, const double* 
   return hip_check(hipGetLastError(), "conv_x");
 }
 
+// y sweep of the flow and species fluxes: a wave marches 64 neighbouring lines
+// through a segment of faces with the stencil windows of at most three
+// variables in registers (207, two waves per SIMD), the rows of the next two
+// faces on their way; the waves that share their lines' u, v, w and metrics
+// follow each other.  Two faces a step, so that the windows move by two (every
+// face: 319 us); blocks of one wave, because five of two hundred registers each
+// would leave three of a compute unit's eight places empty (435 us).  128^3,
+// 9 species: 257 us with two segments a line (one 306, three 310, four 280,
+// five 294; two variables a wave and three waves per SIMD 336), against 184 us
+// (splits) + 282 us (reconstruction) in four launches.
+constexpr int kFuseRows = 128;  // most faces of a segment
+constexpr int kFuseStep = 2;  // faces of a step
+struct FuseLine {
+  long base, s;    // padded index of the line's row 0, the rows' stride
+  long f, fs, nf;  // face 0 of the line, the faces' stride, the faces of a variable
+  int j0, j1;      // the segment's faces; face j reads the padded rows j .. j + 7
+};
+template <int N, int V0>
+struct FuseRow {
+  double u, v, w, a1, a2, a3, phi, r[V0 < 0 ? N : 3];  // r: rho_k, or rho, p, e
+};
+
+// V0 >= 0: the flow fluxes V0 .. V0 + N - 1; V0 < 0: the N species from n0 on
+template <int N, int V0>
+__device__ inline void fuse_march(double* __restrict__ F, const double* __restrict__ Q,
+                                  const double* __restrict__ rhoi,
+                                  const double* __restrict__ A1, const double* __restrict__ A2,
+                                  const double* __restrict__ A3, const double* __restrict__ phi,
+                                  const DevParams* __restrict__ P, long NP, const FuseLine& m,
+                                  int n0) {
+  constexpr int C = kFuseStep;
+  const double sw = PT<double>::sweps2(P);
+  auto load = [&](int row, FuseRow<N, V0>& x) {
+    const long p = m.base + (long)row * m.s;
+    x.u = Q[p + NP];
+    x.v = Q[p + 2 * NP];
+    x.w = Q[p + 3 * NP];
+    x.a1 = A1[p];
+    x.a2 = A2[p];
+    x.a3 = A3[p];
+    if constexpr (V0 < 0) {
+#pragma unroll
+      for (int n = 0; n < N; ++n) x.r[n] = rhoi[p + (long)(n0 + n) * NP];
+    } else {
+      x.r[0] = Q[p];
+      x.r[1] = Q[p + 4 * NP];
+      x.r[2] = Q[p + 6 * NP];
+    }
+  };
+  double pw[N][C + 7], mw[N][C + 7];  // F+ and F- of the rows j .. j + C + 6
+  auto split = [&](const FuseRow<N, V0>& x, int k) {
+    if constexpr (V0 < 0) {
+      const double un = x.a1 * x.u + x.a2 * x.v + x.a3 * x.w;
+      const double Ep = 0.5 * (un + fabs(un));
+      const double Em = 0.5 * (un - fabs(un));
+#pragma unroll
+      for (int n = 0; n < N; ++n) {
+        pw[n][k] = Ep * x.r[n];
+        mw[n][k] = Em * x.r[n];
+      }
+    } else {
+      double fp[5], fm[5];
+      split_point<double>(x.r[0], x.u, x.v, x.w, x.r[1], x.r[2], x.a1, x.a2, x.a3, sw, fp, fm);
+#pragma unroll
+      for (int n = 0; n < N; ++n) {
+        pw[n][k] = fp[V0 + n];
+        mw[n][k] = fm[V0 + n];
+      }
+    }
+  };
+  const int last = m.j1 + 6;  // the last row the segment reads
+  FuseRow<N, V0> x[C];
+  // the rows of the faces j .. j + C - 1 that the window lacks
+  auto ahead = [&](int j) {
+#pragma unroll
+    for (int k = 0; k < C; ++k) {
+      const int row = min(j + 7 + k, last);
+      load(row, x[k]);
+      x[k].phi = phi[m.base + (long)(row - 3) * m.s];
+    }
+  };
+#pragma unroll
+  for (int k = 0; k < 7; ++k) {
+    FuseRow<N, V0> y;
+    load(m.j0 + k, y);
+    split(y, C + k);
+  }
+  double ph = phi[m.base + (long)(m.j0 + 3) * m.s];
+  ahead(m.j0);
+  double* const f = F + m.f + (long)(V0 < 0 ? n0 : V0) * m.nf;
+  for (int j = m.j0; j < m.j1; j += C) {
+#pragma unroll
+    for (int n = 0; n < N; ++n)
+#pragma unroll
+      for (int k = 0; k < 7; ++k) {
+        pw[n][k] = pw[n][k + C];
+        mw[n][k] = mw[n][k + C];
+      }
+    double pn[C];
+#pragma unroll
+    for (int k = 0; k < C; ++k) {
+      split(x[k], 7 + k);
+      pn[k] = x[k].phi;
+    }
+    if (j + C < m.j1) ahead(j + C);
+#pragma unroll
+    for (int k = 0; k < C; ++k) {
+      const int br = weno_branch<double>(fmax(ph, pn[k]), P);
+      ph = pn[k];
+      if (j + k < m.j1) {
+        double fv[N];
+        weno_faces_v<double, N>(br, P, [&](int n, double* pv, double* mv) {
+#pragma unroll
+          for (int i = 0; i < 8; ++i) {
+            pv[i] = pw[n][k + i];
+            mv[i] = mw[n][k + i];
+          }
+        }, fv);
+#pragma unroll
+        for (int n = 0; n < N; ++n) f[(long)(j + k) * m.fs + n * m.nf] = fv[n];
+      }
+    }
+  }
+}
+
+// waves that share a line: flow fluxes 0-2 and 3-4, then three species each
+constexpr int fuse_groups(int ns) { return 2 + (ns + 2) / 3; }
+template <int NS>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2)))
+    k_conv_y(double* __restrict__ F, double* __restrict__ Fi, const double* __restrict__ Q,
+             const double* __restrict__ rhoi, const double* __restrict__ A1,
+             const double* __restrict__ A2, const double* __restrict__ A3,
+             const double* __restrict__ phi, const DevParams* __restrict__ P, Geom g, int seg) {
+  constexpr int G = fuse_groups(NS);
+  const unsigned nb = gridDim.x * gridDim.y * gridDim.z;
+  const unsigned L = xcd_remap(blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z), nb);
+  const int w = (int)(L % G);
+  const unsigned B = L / G, nl = gridDim.x / G;
+  const int a = (int)(B % nl) * 64 + threadIdx.x;
+  const int c = (int)((B / nl) % gridDim.y);
+  const int sgi = (int)(B / (nl * gridDim.y));
+  const int nd = g.Ny + 1;
+  FuseLine m;
+  m.j0 = sgi * seg;
+  m.j1 = min(m.j0 + seg, nd);
+  if (a >= g.Nx || m.j0 >= m.j1) return;
+  m.s = g.Nxt;
+  m.base = (a + NG) + (long)g.Nxt * g.Nyt * (c + NG);
+  m.f = a + (long)g.Nx * nd * c;
+  m.fs = g.Nx;
+  m.nf = (long)g.Nx * nd * g.Nz;
+  constexpr int R = NS % 3;  // species of the last wave, if not three
+  const long NP = g.NP;
+  if (w == 0)
+    fuse_march<3, 0>(F, Q, rhoi, A1, A2, A3, phi, P, NP, m, 0);
+  else if (w == 1)
+    fuse_march<2, 3>(F, Q, rhoi, A1, A2, A3, phi, P, NP, m, 0);
+  else if (R != 0 && w == G - 1)
+    fuse_march<R != 0 ? R : 1, -1>(Fi, Q, rhoi, A1, A2, A3, phi, P, NP, m, NS - R);
+  else if (NS >= 3)
+    fuse_march<3, -1>(Fi, Q, rhoi, A1, A2, A3, phi, P, NP, m, 3 * (w - 2));
+}
+
+int launch_conv_y(f3d_ctx* c, void* F, void* Fi, const void* phi, const double* Q,
+                  const double* rhoi, const void* const* M, hipStream_t s) {
+  const Geom& g = c->g;
+  const int nd = g.Ny + 1;
+  const unsigned nl = (g.Nx + 63) / 64;
+#define F3D_CY(NS_)                                                                           \
+  {                                                                                           \
+    const long cap = resident_blocks(&k_conv_y<NS_>, 64, &c->fuse_blocks);                    \
+    const long lines = (long)nl * g.Nz * fuse_groups(NS_);                                    \
+    const int nseg = fill_segments((nd + kFuseRows - 1) / kFuseRows, cap, lines, nd);         \
+    const int seg = (nd + nseg - 1) / nseg;                                                   \
+    hipLaunchKernelGGL((k_conv_y<NS_>), dim3(nl * fuse_groups(NS_), g.Nz,                     \
+                                             (nd + seg - 1) / seg),                           \
+                       dim3(64), 0, s, (double*)F, (double*)Fi, Q, rhoi, (const double*)M[3], \
+                       (const double*)M[4], (const double*)M[5], (const double*)phi,          \
+                       c->dparams, g, seg);                                                   \
+  }
+  switch (g.Ns) {
+    case 1: F3D_CY(1); break;
+    case 5: F3D_CY(5); break;
+    case 9: F3D_CY(9); break;
+    default: set_error("conv_y: Ns must be 1, 5 or 9"); return F3D_ERR_UNSUPPORTED;
+  }
+#undef F3D_CY
+  return hip_check(hipGetLastError(), "conv_y");
+}
+
 // ---- launchers --------------------------------------------------------------
 int launch_flux_split(f3d_ctx* c, const double* Q, void* Fp, void* Fm, const void* Ax,
                       const void* Ay, const void* Az, const int64_t* tag, hipStream_t s,

@@ -49,7 +49,7 @@ def test_fill_pairs_of_faces(mech, kinds):
 
 
 @pytest.mark.parametrize("shape", [(4, 4, 4), (65, 7, 5), (9, 33, 34), (70, 66, 9), (128, 4, 5),
-                                   (257, 5, 4)])
+                                   (257, 5, 4), (5, 127, 4), (66, 131, 70)])
 @pytest.mark.parametrize("mech", ["air5", "h2_lidryer"])
 def test_stage_on_small_and_ragged_blocks(mech, shape):
     """One FP64 stage on blocks of one short segment, several, a remainder
