@@ -69,7 +69,7 @@ struct TileLds {
     } g;
   } u;
   float bsum[4][NN_H];  // per-wave bias-gradient partial sums
-  float red[256];
+  float red[8];         // per-wave loss
 };
 
 // sum over the four 16-lane groups holding the same column (lanes r, r+16, r+32, r+48)
@@ -79,16 +79,22 @@ __device__ inline float sum_q(float v) {
   return v;
 }
 
-__global__ void __launch_bounds__(256)
+// Two waves to 16 samples, each half of a layer's outputs: a batch of 8192 is
+// 128 blocks, one on every other compute unit, so a block's time is its chain
+// of products, GELUs and barriers (with one wave to 16 samples 17.9 us, with two
+// and transposed copies stored four samples at a time 15.2; all weights fetched
+// into registers first: no faster).
+constexpr int kTileThreads = 512;
+__global__ void __launch_bounds__(kTileThreads)
     k_nn_train_tile(const float* __restrict__ Xg, const float* __restrict__ Tg, int B, int nin,
                     int nout, const __bf16* __restrict__ Wb, const __bf16* __restrict__ Wtb,
                     const float* __restrict__ master, float* __restrict__ partial) {
   __shared__ __align__(16) TileLds L;
   const int tid = threadIdx.x;
-  const int w = tid >> 6, lane = tid & 63;
+  const int w = (tid >> 6) & 3, half = tid >> 8, lane = tid & 63;
   const int r16 = lane & 15, q = lane >> 4;
   const long s0 = (long)blockIdx.x * 64;
-  for (int e = tid; e < 64 * NN_INP; e += 256) {
+  for (int e = tid; e < 64 * NN_INP; e += kTileThreads) {
     const int s = e / NN_INP, k = e % NN_INP;
     const float v = (k < nin) ? Xg[(s0 + s) * nin + k] : 0.0f;
     L.X[s][k] = (__bf16)v;
@@ -96,14 +102,15 @@ __global__ void __launch_bounds__(256)
   }
   __syncthreads();
   const int sw = 16 * w;  // this wave's first sample on the data path
-  float gp[3][4][4];      // GELU' of the wave's hidden pre-activations
+  float gp[3][2][4];      // GELU' of the wave's hidden pre-activations
   // ---- forward, hidden layers ----
   for (int l = 0; l < 3; ++l) {
     const int NI = nn_in_dim(l);
     const __bf16* W = Wb + nn_w_off(l);
     const float* bias = master + nn_b_off(l);
 #pragma unroll
-    for (int ot = 0; ot < NN_H / 16; ++ot) {
+    for (int j = 0; j < NN_H / 32; ++j) {
+      const int ot = 2 * half + j;
       f32x4 acc = {0, 0, 0, 0};
       for (int kk = 0; kk < NI / 32; ++kk) {
         const bf16x8 a = (l == 0) ? ld8(&L.X[sw + r16][32 * kk + 8 * q])
@@ -113,69 +120,67 @@ __global__ void __launch_bounds__(256)
       }
       const int o = 16 * ot + r16;
       const float bo = bias[o];
+      bf16x4 at;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int s = sw + 4 * q + i;
         float d;
-        const __bf16 a = (__bf16)gelu(acc[i] + bo, d);
-        gp[l][ot][i] = d;
-        L.u.A[l & 1][s][o] = a;
-        L.At[l][o][s] = a;
+        at[i] = (__bf16)gelu(acc[i] + bo, d);
+        gp[l][j][i] = d;
+        L.u.A[l & 1][s][o] = at[i];
       }
+      *reinterpret_cast<bf16x4*>(&L.At[l][o][sw + 4 * q]) = at;
     }
     __syncthreads();
   }
   // ---- output layer and dL/dy (the output layer is linear: dZ4 = dL/dy) ----
   float lsum = 0.0f;
-  f32x4 yv[NN_OUTP / 16];
+  f32x4 yv;
+  static_assert(NN_OUTP == 32, "an output tile to a wave");
+  const int oy = 16 * half + r16;
   {
     const __bf16* W = Wb + nn_w_off(3);
-#pragma unroll
-    for (int ot = 0; ot < NN_OUTP / 16; ++ot) {
-      f32x4 acc = {0, 0, 0, 0};
-      for (int kk = 0; kk < NN_H / 32; ++kk) {
-        const bf16x8 a = ld8(&L.u.A[0][sw + r16][32 * kk + 8 * q]);
-        const bf16x8 b = ld8(W + (16 * ot + r16) * NN_H + 32 * kk + 8 * q);
-        acc = mfma(a, b, acc);
-      }
-      yv[ot] = acc;
+    f32x4 acc = {0, 0, 0, 0};
+    for (int kk = 0; kk < NN_H / 32; ++kk) {
+      const bf16x8 a = ld8(&L.u.A[0][sw + r16][32 * kk + 8 * q]);
+      const bf16x8 b = ld8(W + oy * NN_H + 32 * kk + 8 * q);
+      acc = mfma(a, b, acc);
     }
+    yv = acc;
   }
   __syncthreads();  // A[0] (layer-2 output) fully read before dZ overwrites the union
   {
     const float* bias = master + nn_b_off(3);
     const float scale = 2.0f / ((float)B * (float)nout);
+    float bs = 0.0f;
+    bf16x4 zt;
 #pragma unroll
-    for (int ot = 0; ot < NN_OUTP / 16; ++ot) {
-      const int o = 16 * ot + r16;
-      float bs = 0.0f;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int s = sw + 4 * q + i;
-        float g = 0.0f;
-        if (o < nout) {
-          const float d = yv[ot][i] + bias[o] - Tg[(s0 + s) * nout + o];
-          lsum += d * d;
-          g = scale * d;
-        }
-        bs += g;
-        L.u.g.dZ[s][o] = (__bf16)g;
-        L.u.g.dZt[o][s] = (__bf16)g;
+    for (int i = 0; i < 4; ++i) {
+      const int s = sw + 4 * q + i;
+      float g = 0.0f;
+      if (oy < nout) {
+        const float d = yv[i] + bias[oy] - Tg[(s0 + s) * nout + oy];
+        lsum += d * d;
+        g = scale * d;
       }
-      bs = sum_q(bs);
-      if (q == 0) L.bsum[w][o] = bs;
+      bs += g;
+      zt[i] = (__bf16)g;
+      L.u.g.dZ[s][oy] = zt[i];
     }
+    *reinterpret_cast<bf16x4*>(&L.u.g.dZt[oy][sw + 4 * q]) = zt;
+    bs = sum_q(bs);
+    if (q == 0) L.bsum[w][oy] = bs;
   }
   __syncthreads();
   float* part = partial + (long)blockIdx.x * (NN_NPARAM + 1);
   // ---- backward, layers 3..0 ----
   for (int l = 3; l >= 0; --l) {
     const int NI = nn_in_dim(l), NO = nn_out_dim(l);
-    for (int o = tid; o < NO; o += 256)
+    for (int o = tid; o < NO; o += kTileThreads)
       part[nn_b_off(l) + o] = L.bsum[0][o] + L.bsum[1][o] + L.bsum[2][o] + L.bsum[3][o];
     // weight gradient dW[o][k] = sum_s dZ[s][o] A_prev[s][k], output tiles over the waves
     const int nto = NO / 16, ntk = NI / 16;
-    for (int t = w; t < nto * ntk; t += 4) {
+    for (int t = tid >> 6; t < nto * ntk; t += kTileThreads / 64) {
       const int ot = t / ntk, kt = t % ntk;
       f32x4 acc = {0, 0, 0, 0};
 #pragma unroll
@@ -191,43 +196,48 @@ __global__ void __launch_bounds__(256)
     }
     if (l == 0) break;
     // data gradient dA_prev[s][k] = sum_o dZ[s][o] W[o][k]  (W^T copy: [k][o])
-    f32x4 dA[4];
+    f32x4 dA[2];
     const __bf16* Wt = Wtb + nn_w_off(l);
 #pragma unroll
-    for (int kt = 0; kt < 4; ++kt) {
+    for (int j = 0; j < 2; ++j) {
+      const int kt = 2 * half + j;
       f32x4 acc = {0, 0, 0, 0};
       for (int ks = 0; ks < NO / 32; ++ks) {
         const bf16x8 a = ld8(&L.u.g.dZ[sw + r16][32 * ks + 8 * q]);
         const bf16x8 b = ld8(Wt + (16 * kt + r16) * NO + 32 * ks + 8 * q);
         acc = mfma(a, b, acc);
       }
-      dA[kt] = acc;
+      dA[j] = acc;
     }
     __syncthreads();  // all reads of dZ, dZ^T and bsum of layer l are done
 #pragma unroll
-    for (int kt = 0; kt < 4; ++kt) {
-      const int k = 16 * kt + r16;
+    for (int j = 0; j < 2; ++j) {
+      const int k = 16 * (2 * half + j) + r16;
       float bs = 0.0f;
+      bf16x4 zt;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int s = sw + 4 * q + i;
-        const float g = dA[kt][i] * gp[l - 1][kt][i];
+        const float g = dA[j][i] * gp[l - 1][j][i];
         bs += g;
-        L.u.g.dZ[s][k] = (__bf16)g;
-        L.u.g.dZt[k][s] = (__bf16)g;
+        zt[i] = (__bf16)g;
+        L.u.g.dZ[s][k] = zt[i];
       }
+      *reinterpret_cast<bf16x4*>(&L.u.g.dZt[k][sw + 4 * q]) = zt;
       bs = sum_q(bs);
       if (q == 0) L.bsum[w][k] = bs;
     }
     __syncthreads();
   }
-  L.red[tid] = lsum;
+#pragma unroll
+  for (int d = 32; d > 0; d >>= 1) lsum += __shfl_xor(lsum, d);
+  if (lane == 0) L.red[tid >> 6] = lsum;
   __syncthreads();
-  for (int st = 128; st > 0; st >>= 1) {
-    if (tid < st) L.red[tid] += L.red[tid + st];
-    __syncthreads();
+  if (tid == 0) {
+    float ls = 0.0f;
+    for (int i = 0; i < kTileThreads / 64; ++i) ls += L.red[i];
+    part[NN_NPARAM] = ls / ((float)B * (float)nout);
   }
-  if (tid == 0) part[NN_NPARAM] = L.red[0] / ((float)B * (float)nout);
 }
 
 // Sum over the tiles of the partials (gradient and loss): blocks of 64 slots,
@@ -1211,8 +1221,8 @@ int f3d_nn_grad(f3d_ctx* c, const float* X, const float* Y, int32_t B, float* gr
   const long tiles = B / 64;
   rc = nn_partials(c, tiles);
   if (rc) return rc;
-  hipLaunchKernelGGL(k_nn_train_tile, dim3(tiles), dim3(256), 0, s, X, Y, B, c->g.Ns + 2, c->g.Ns,
-                     (const __bf16*)c->nn_Wb, (const __bf16*)c->nn_Wtb, c->nn_master,
+  hipLaunchKernelGGL(k_nn_train_tile, dim3(tiles), dim3(kTileThreads), 0, s, X, Y, B,
+                     c->g.Ns + 2, c->g.Ns, (const __bf16*)c->nn_Wb, (const __bf16*)c->nn_Wtb, c->nn_master,
                      c->nn_partial);
   hipLaunchKernelGGL(k_nn_reduce, dim3(nblocks(NN_NPARAM + 1, kSumSlots)),
                      dim3(kSumSlots, kSumWays), 0, s, c->nn_partial, (int)tiles, grad);
@@ -1230,8 +1240,8 @@ int f3d_nn_train_step(f3d_ctx* c, const float* X, const float* Y, int32_t B, flo
   const double b1 = 0.9, b2 = 0.999;
   const float bc1 = (float)(1.0 - std::pow(b1, (double)c->nn_step));
   const float bc2 = (float)(1.0 - std::pow(b2, (double)c->nn_step));
-  hipLaunchKernelGGL(k_nn_train_tile, dim3(tiles), dim3(256), 0, s, X, Y, B, c->g.Ns + 2, c->g.Ns,
-                     (const __bf16*)c->nn_Wb, (const __bf16*)c->nn_Wtb, c->nn_master,
+  hipLaunchKernelGGL(k_nn_train_tile, dim3(tiles), dim3(kTileThreads), 0, s, X, Y, B,
+                     c->g.Ns + 2, c->g.Ns, (const __bf16*)c->nn_Wb, (const __bf16*)c->nn_Wtb, c->nn_master,
                      c->nn_partial);
   hipLaunchKernelGGL(k_nn_adam, dim3(nblocks(NN_NPARAM + 1, kSumSlots)),
                      dim3(kSumSlots, kSumWays), 0, s, c->nn_partial, (int)tiles, c->nn_master, c->nn_m1, c->nn_m2, (__bf16*)c->nn_Wb,
@@ -1255,8 +1265,8 @@ int f3d_nn_train_step_static(f3d_ctx* c, const float* X, const float* Y, int32_t
   const double b1 = 0.9, b2 = 0.999;
   const float bc1 = (float)(1.0 - std::pow(b1, (double)c->nn_step));
   const float bc2 = (float)(1.0 - std::pow(b2, (double)c->nn_step));
-  hipLaunchKernelGGL(k_nn_train_tile, dim3(tiles), dim3(256), 0, s, X, Y, B, c->g.Ns + 2, c->g.Ns,
-                     (const __bf16*)c->nn_Wb, (const __bf16*)c->nn_Wtb, c->nn_master, part);
+  hipLaunchKernelGGL(k_nn_train_tile, dim3(tiles), dim3(kTileThreads), 0, s, X, Y, B,
+                     c->g.Ns + 2, c->g.Ns, (const __bf16*)c->nn_Wb, (const __bf16*)c->nn_Wtb, c->nn_master, part);
   hipLaunchKernelGGL(k_nn_adam, dim3(nblocks(NN_NPARAM + 1, kSumSlots)),
                      dim3(kSumSlots, kSumWays), 0, s, part, (int)tiles, c->nn_master, c->nn_m1, c->nn_m2, (__bf16*)c->nn_Wb,
                      (__bf16*)c->nn_Wtb, lr, (float)b1, (float)b2, 1e-8f, bc1, bc2, loss);
