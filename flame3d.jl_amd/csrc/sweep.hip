@@ -29,18 +29,23 @@
 
 namespace f3d {
 
-// x-line blocks: a thread to each staged point (the cells and up to eight more)
-// and at most kXMost cells, a line split into equal segments beyond that.  With
-// 256 cells and 256 threads the staged points past the 256th and the last face
-// were a second pass of the first and of the last wave, the others waiting; a
-// line of 300 cells took a second block of 256 threads for 44 cells.  At
-// 300x127x127 (air): convective 619 -> 461 us, viscous 336 -> 184, species
-// 308 -> 168; at 256^3 (H2/air): 640, 720 -> 639 and 1022 -> 926 us.
+// x-line blocks: lines are split into equal segments of at most kXMost cells,
+// with threads in whole waves for a segment's cells and, in the diffusive
+// kernels, for its staged points as well (up to four more) and its last face.
+// With 256 cells and 256 threads these were second passes of the first and of
+// the last wave, the others waiting; a line of 300 cells took a second block of
+// 256 threads for 44 cells.  At 300x127x127 (air): convective 619 -> 461 us,
+// viscous 336 -> 184, species 308 -> 168; at 256^3 (H2/air) viscous 720 -> 639,
+// species 1022 -> 926.  The convective kernel, bound by instructions where the
+// flow has shocks, is slower with a wave for eight more points (256x128x128
+// with a shock, 282 us against 260), so there they stay a second pass.
 constexpr int kXThreads = 320, kXMost = 304;
-// MOST: the cells a kernel's LDS holds, kXMost (the _long kernels) or this: a
-// sixth less LDS, a block more per compute unit (at 256^3, with the larger:
-// convective 741 us, species 1176 with its face values beside the metrics).
-constexpr int kXFew = 256;
+// MOST: the cells a kernel's LDS holds, kXMost (the _long kernels), kXFew or
+// kXShort (the _short kernels): the less, the more blocks fit a compute unit.
+// At 256^3 with kXMost instead of kXFew: convective 741 instead of 639 us,
+// species 1176 instead of 926; at 128^3 (H2/air with a shock) with kXFew instead
+// of kXShort: 196, 126 instead of 163, 111 (256 threads for 128 cells: 180, 192).
+constexpr int kXFew = 256, kXShort = 128;
 constexpr int kConvSeg = 32;  // cells per march segment (convective)
 constexpr int kViscSeg = 64;  // cells per march segment (viscous)
 
@@ -76,7 +81,7 @@ __device__ __forceinline__ void conv_x_line(
     int acc, int seg) {
   constexpr int NV = 5 + NS;
   constexpr int NPT = MOST + 8;
-  static_assert(MOST + 8 <= kXThreads && MOST + NV <= kXThreads, "a thread to a point");
+  static_assert(MOST <= kXThreads, "a thread to a cell");
   __shared__ float sp[NV][NPT];
   __shared__ float sm[NV][NPT];
   __shared__ float sphi[NPT];
@@ -84,9 +89,9 @@ __device__ __forceinline__ void conv_x_line(
   const int nc = x.nc;
   const int t = threadIdx.x;
   const long NP = g.NP;
-  if (t < nc + 8) {
-    // point t of the segment is padded i = c0 + t (cell c0 + t - NG)
-    const long p = (long)x.c0 + (long)g.Nxt * ((x.b + NG) + (long)g.Nyt * (x.c + NG)) + t;
+  for (int i = t; i < nc + 8; i += blockDim.x) {
+    // point i of the segment is padded c0 + i (cell c0 + i - NG)
+    const long p = (long)x.c0 + (long)g.Nxt * ((x.b + NG) + (long)g.Nyt * (x.c + NG)) + i;
     const float sw = PT<float>::sweps2(P);
     const float u = (float)Q[p + NP], v = (float)Q[p + 2 * NP], w = (float)Q[p + 3 * NP];
     const float a1 = A1[p], a2 = A2[p], a3 = A3[p];
@@ -95,8 +100,8 @@ __device__ __forceinline__ void conv_x_line(
                        a3, sw, fp, fm);
 #pragma unroll
     for (int n = 0; n < 5; ++n) {
-      sp[n][t] = fp[n];
-      sm[n][t] = fm[n];
+      sp[n][i] = fp[n];
+      sm[n][i] = fm[n];
     }
     const float un = a1 * u + a2 * v + a3 * w;
     const float Ep = 0.5f * (un + fabsf(un));
@@ -104,10 +109,10 @@ __device__ __forceinline__ void conv_x_line(
 #pragma unroll
     for (int n = 0; n < NS; ++n) {
       const float r = (float)rhoi[p + (long)n * NP];
-      sp[5 + n][t] = Ep * r;
-      sm[5 + n][t] = Em * r;
+      sp[5 + n][i] = Ep * r;
+      sm[5 + n][i] = Em * r;
     }
-    sphi[t] = phi[p];
+    sphi[i] = phi[p];
   }
   __syncthreads();
   // face f (0..nc) between cells c0+f-1 and c0+f: stencil points q = f .. f+7
@@ -122,9 +127,10 @@ __device__ __forceinline__ void conv_x_line(
       }
     }, fv);
   }
-  // the segment's last face, one variable per thread of those after the cells
+  // the segment's last face, one variable per thread (those after the cells, if
+  // there are enough of them)
   float fl = 0.0f;
-  const int n1 = t - nc;
+  const int n1 = (int)blockDim.x - nc >= NV ? t - nc : t;
   if (n1 >= 0 && n1 < NV) {
     const int br = weno_branch<float>(fmaxf(sphi[nc + 3], sphi[nc + 4]), P);
     float pv[8], mv[8];
@@ -170,6 +176,17 @@ __global__ void __launch_bounds__(kXThreads)
         const float* __restrict__ phi, const DevParams* __restrict__ P, Geom g,
         int acc, int seg) {
   conv_x_line<NS, kXMost>(rhs, Q, rhoi, A1, A2, A3, phi, P, g, acc, seg);
+}
+
+template <int NS>
+__global__ void __launch_bounds__(kXThreads)
+    k_sw_conv_x_short(
+        float* __restrict__ rhs, const double* __restrict__ Q,
+        const double* __restrict__ rhoi, const float* __restrict__ A1,
+        const float* __restrict__ A2, const float* __restrict__ A3,
+        const float* __restrict__ phi, const DevParams* __restrict__ P, Geom g,
+        int acc, int seg) {
+  conv_x_line<NS, kXShort>(rhs, Q, rhoi, A1, A2, A3, phi, P, g, acc, seg);
 }
 
 // ---------------------------------------------------------------------------
@@ -580,6 +597,14 @@ __global__ void __launch_bounds__(kXThreads)
   visc_x_line<kXMost>(rhs, Q, M, J, lam, mu, g, seg);
 }
 
+__global__ void __launch_bounds__(kXThreads)
+    k_sw_visc_x_short(
+        float* __restrict__ rhs, const double* __restrict__ Q, FMet M,
+        const float* __restrict__ J, const float* __restrict__ lam,
+        const float* __restrict__ mu, Geom g, int seg) {
+  visc_x_line<kXShort>(rhs, Q, M, J, lam, mu, g, seg);
+}
+
 // x-line block of the species-diffusion sweep with each cell's inputs read
 // once: the metrics, J, rho and T of the cells -1 .. nc are staged in LDS,
 // then species by species Y_k of the cells -2 .. nc+1 and the transverse
@@ -730,6 +755,15 @@ __global__ void __launch_bounds__(kXThreads) __attribute__((amdgpu_waves_per_eu(
         const float* __restrict__ Yi, FMet M, const float* __restrict__ J,
         const float* __restrict__ D, const DevParams* __restrict__ P, Geom g, int seg) {
   spec_x_line<NS, kXMost>(rhs, Q, Yi, M, J, D, P, g, seg);
+}
+
+template <int NS>
+__global__ void __launch_bounds__(kXThreads) __attribute__((amdgpu_waves_per_eu(7)))
+    k_sw_spec_x_short(
+        float* __restrict__ rhs, const double* __restrict__ Q,
+        const float* __restrict__ Yi, FMet M, const float* __restrict__ J,
+        const float* __restrict__ D, const DevParams* __restrict__ P, Geom g, int seg) {
+  spec_x_line<NS, kXShort>(rhs, Q, Yi, M, J, D, P, g, seg);
 }
 
 // ---------------------------------------------------------------------------
@@ -1072,8 +1106,9 @@ static void conv_ns(f3d_ctx* c, int dir, float* rhs, const double* Q, const doub
                     const float* const* A, const float* phi, int acc, hipStream_t s) {
   const Geom& g = c->g;
   if (dir == 0) {
-    const XLaunch l = x_launch(g, std::max(8, 5 + NS));
-    const auto k = l.seg <= kXFew ? k_sw_conv_x<NS> : k_sw_conv_x_long<NS>;
+    const XLaunch l = x_launch(g, 0);
+    const auto k = l.seg <= kXShort ? k_sw_conv_x_short<NS>
+                   : l.seg <= kXFew ? k_sw_conv_x<NS> : k_sw_conv_x_long<NS>;
     hipLaunchKernelGGL(k, dim3(l.blocks), dim3(l.threads), 0, s, rhs, Q, rhoi,
                        A[0], A[1], A[2], phi, c->dparams, g, acc, l.seg);
   } else {
@@ -1116,8 +1151,10 @@ static void diff_ns(f3d_ctx* c, int dir, float* rhs, const double* Q, const floa
   const Geom& g = c->g;
   if (dir == 0) {
     const XLaunch l = x_launch(g, 4);
-    const auto kv = l.seg <= kXFew ? k_sw_visc_x : k_sw_visc_x_long;
-    const auto ks = l.seg <= kXFew ? k_sw_spec_x<NS> : k_sw_spec_x_long<NS>;
+    const auto kv = l.seg <= kXShort ? k_sw_visc_x_short
+                    : l.seg <= kXFew ? k_sw_visc_x : k_sw_visc_x_long;
+    const auto ks = l.seg <= kXShort ? k_sw_spec_x_short<NS>
+                    : l.seg <= kXFew ? k_sw_spec_x<NS> : k_sw_spec_x_long<NS>;
     hipLaunchKernelGGL(kv, dim3(l.blocks), dim3(l.threads), 0, s, rhs, Q, M, J, lam, mu,
                        g, l.seg);
     hipLaunchKernelGGL(ks, dim3(l.blocks), dim3(l.threads), 0, s, rhs, Q, Yi, M,

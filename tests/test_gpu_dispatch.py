@@ -127,13 +127,14 @@ def test_fallback_equals_newton(mech, shape, maxiter):
 
 @pytest.mark.parametrize("mech,nx,scheme", [
     ("air5", 4, None), ("air5", 56, "weno7"), ("air5", 60, None), ("h2_lidryer", 61, None),
+    ("h2_lidryer", 128, "weno7"), ("air5", 129, None), ("h2_lidryer", 129, None),
     ("h2_lidryer", 256, None), ("h2_lidryer", 257, "weno7"), ("air5", 304, "weno7"),
     ("air5", 305, None), ("h2_lidryer", 305, None), ("air5", 609, "weno7")])
 def test_x_line_segments(mech, nx, scheme):
     """The fused FP32 stage on x lines at the edges of its rules: the smallest,
     those whose cells and staged points just fill or just exceed a number of
-    waves, the largest of the smaller and of the larger LDS tile, and lines of
-    two and three segments; the granular stage's bars of test_gpu_sweeps."""
+    waves, the largest and one more of each LDS tile, and lines of two and three
+    segments; the granular stage's bars of test_gpu_sweeps."""
     import flame3d_amd.abi as abi
     from test_gpu_sweeps import _cmp, _stage_pair
     sc = {"recon_kind": abi.RECON_WENO7} if scheme else None
