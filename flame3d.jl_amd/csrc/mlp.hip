@@ -317,20 +317,20 @@ __global__ void __launch_bounds__(256)
 // the FP32 outputs: a layer's 4x4 (or 4x2) 16x16 output tiles stay in
 // registers until every lane has read the previous activations.
 // ---------------------------------------------------------------------------
-// Rows are padded by 16 bytes: a 16-byte MFMA operand read by the 16 lanes of
-// a quarter-wave then spans different bank groups instead of the same one (an
-// unpadded row of 64 bf16 is 128 B, a whole bank cycle).
+// Rows are padded by 16 bytes (one float for Y): a 16-byte MFMA operand read
+// by the 16 lanes of a quarter-wave then spans different bank groups instead
+// of the same one (an unpadded row of 64 bf16 is 128 B, a whole bank cycle).
 constexpr int kRowPad = 8;
 union FwdLds {
   __bf16 X[64][NN_INP + kRowPad];
   __bf16 A[64][NN_H + kRowPad];
-  float Y[64][NN_OUTP + 4];
+  float Y[64][NN_OUTP + 1];
 };
 
 // one dense layer for the wave's 64 samples: NI inputs, NO outputs (compile-time).
-// The weights are the MFMA's A operand, so a lane receives four consecutive
-// outputs of one sample and stores them with one write (8 bytes of bf16, or 16
-// of float) instead of four 2-byte writes 144 bytes apart.
+// (With the weights as the first operand a lane holds four outputs of a sample
+// and stores them with one write, but the layer takes longer: k_nn_net 432
+// instead of 394 us at 192x128x128.)
 template <int NI, int NO, bool LAST>
 __device__ __forceinline__ void nn_layer_wave(FwdLds& L, const __bf16* __restrict__ W,
                                      const float* __restrict__ bias, int lane) {
@@ -342,49 +342,34 @@ __device__ __forceinline__ void nn_layer_wave(FwdLds& L, const __bf16* __restric
     for (int st = 0; st < 4; ++st) acc[st][ot] = {0, 0, 0, 0};
 #pragma unroll
     for (int kk = 0; kk < NI / 32; ++kk) {
-      const bf16x8 w = ld8(W + (16 * ot + r16) * NI + 32 * kk + 8 * q);
+      const bf16x8 b = ld8(W + (16 * ot + r16) * NI + 32 * kk + 8 * q);
 #pragma unroll
       for (int st = 0; st < 4; ++st) {
         const __bf16* src = (NI == NN_INP) ? &L.X[16 * st + r16][32 * kk + 8 * q]
                                            : &L.A[16 * st + r16][32 * kk + 8 * q];
-        acc[st][ot] = mfma(w, ld8(src), acc[st][ot]);
+        acc[st][ot] = mfma(ld8(src), b, acc[st][ot]);
       }
     }
   }
   __syncthreads();  // every lane has read this layer's input tile
 #pragma unroll
   for (int ot = 0; ot < NO / 16; ++ot) {
-    const int o = 16 * ot + 4 * q;
-    const f32x4 bo = *reinterpret_cast<const f32x4*>(bias + o);
+    const int o = 16 * ot + r16;
+    const float bo = bias[o];
 #pragma unroll
-    for (int st = 0; st < 4; ++st) {
-      const int s = 16 * st + r16;
-      if (LAST) {
-        *reinterpret_cast<f32x4*>(&L.Y[s][o]) = acc[st][ot] + bo;
-      } else {
-        bf16x4 h;
+    for (int st = 0; st < 4; ++st)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
+      for (int i = 0; i < 4; ++i) {
+        const int s = 16 * st + 4 * q + i;
+        if (LAST) {
+          L.Y[s][o] = acc[st][ot][i] + bo;
+        } else {
           float d;
-          h[i] = (__bf16)gelu(acc[st][ot][i] + bo[i], d);
+          L.A[s][o] = (__bf16)gelu(acc[st][ot][i] + bo, d);
         }
-        *reinterpret_cast<bf16x4*>(&L.A[s][o]) = h;
       }
-    }
   }
   __syncthreads();
-}
-
-// a lane's input row, inputs xn[0 .. nin) and zeros
-template <class F>
-__device__ __forceinline__ void nn_put_input(FwdLds& L, int lane, F&& x) {
-#pragma unroll
-  for (int k = 0; k < NN_INP; k += 8) {
-    bf16x8 v;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) v[i] = (__bf16)x(k + i);
-    *reinterpret_cast<bf16x8*>(&L.X[lane][k]) = v;
-  }
 }
 
 __device__ __forceinline__ void nn_forward_wave(FwdLds& L, const __bf16* __restrict__ Wb,
@@ -402,7 +387,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4)))
   __shared__ __align__(16) FwdLds L;
   const int lane = threadIdx.x;
   const long s0 = (long)blockIdx.x * 64;
-  nn_put_input(L, lane, [&](int k) { return k < nin ? Xg[(s0 + lane) * nin + k] : 0.0f; });
+  for (int k = 0; k < NN_INP; ++k) L.X[lane][k] = (__bf16)(k < nin ? Xg[(s0 + lane) * nin + k] : 0.0f);
   __syncthreads();
   nn_forward_wave(L, Wb, master, lane);
   for (int o = 0; o < nout; ++o) Yg[(s0 + lane) * nout + o] = L.Y[lane][o];
@@ -565,7 +550,8 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4)))
   // a tile with no reacting cell (cold gas, tagged cells) skips the network;
   // the workgroup is one wave, so the exit is uniform over the workgroup
   if (!__any(act)) return;
-  nn_put_input(L, lane, [&](int k) { return k < NIN ? xn[k < NIN ? k : 0] : 0.0f; });
+#pragma unroll
+  for (int k = 0; k < NN_INP; ++k) L.X[lane][k] = (__bf16)(k < NIN ? xn[k] : 0.0f);
   __syncthreads();
   nn_forward_wave(L, Wb, master, lane);
   if (act) {
@@ -598,11 +584,13 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3))
               const float* __restrict__ out, double* __restrict__ cand,
               int8_t* __restrict__ status) {
   __shared__ NasaTab<NS> N;
-  N.fill(P);
   const long ncell = (long)g.Nx * g.Ny * g.Nz;
   const long id = gid();
-  if (id >= ncell) return;
-  int code = status[id];  // 0 inactive, 1 candidate, 2 Mahalanobis
+  int code = id < ncell ? status[id] : 0;  // 0 inactive, 1 candidate, 2 Mahalanobis
+  // a block of cold cells leaves before it builds its table (hot air jet,
+  // 192x128x128: 37 -> 29 us)
+  if (!__syncthreads_or(code == 1)) return;
+  N.fill(P);
   if (code != 1) return;
   const long NP = g.NP;
   const int a = (int)(id % g.Nx);
@@ -713,11 +701,11 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))
               const double* __restrict__ cand, int32_t* __restrict__ tile_count,
               int8_t* __restrict__ status, const CI carriers) {
   __shared__ NasaTab<NS> N;
-  N.fill(P);
   const long ncell = (long)g.Nx * g.Ny * g.Nz;
   const long id = gid();  // a wave holds the 64 cells of one tile
   const long NP = g.NP;
   int code = (id < ncell) ? status[id] : 0;
+  if (__syncthreads_or(code == 1)) N.fill(P);
   if (code == 1) {
     const int a = (int)(id % g.Nx);
     const int t = (int)(id / g.Nx);
