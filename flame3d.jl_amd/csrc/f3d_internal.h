@@ -124,6 +124,13 @@ int hip_check(hipError_t e, const char* what);
 constexpr int kBlock = 256;
 
 inline unsigned nblocks(long n, int block = kBlock) { return (unsigned)((n + block - 1) / block); }
+// Threads per block of a kernel of one thread per point or cell: single waves
+// up to one wave for each of the 1024 SIMDs, so that every wave has a compute
+// unit's caches and LDS as much to itself as there is room.  FP64 stage of
+// 24x16x12 H2/air (4608 cells), 64 against 256 threads: stage end 38 against 48
+// us, species and viscous faces 6.0 / 4.4 against 7.8 / 6.3, fill 4.7 against
+// 6.3; 60x27x27 air (43740 cells): stage end 14.1 / 14.2, faces 5.9 / 6.6.
+inline int small_block(long n) { return n <= 1024 * 64 ? 64 : kBlock; }
 
 // Segments per line of a march over nd cells or faces: n0, or more where a
 // launch of n0 `lines` blocks leaves half of the device's resident block slots

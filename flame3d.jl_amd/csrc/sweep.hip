@@ -1180,8 +1180,9 @@ static void stage_end_ns(f3d_ctx* c, int KRK, double* U, const double* Un, doubl
   const long n = (long)c->g.Nx * c->g.Ny * c->g.Nz;
   const int lin = KRK > 1;
   const double la = KRK == 2 ? 0.25 : 2.0 / 3.0, lb = KRK == 2 ? 0.75 : 1.0 / 3.0;
-  hipLaunchKernelGGL((k_sw_stage_end<NS>), dim3(nblocks(n)), dim3(kBlock), 0, s, U, Un, rhoi,
-                     rhon, Q, rhs, dt, J, c->dparams, c->g, lin, la, lb);
+  hipLaunchKernelGGL((k_sw_stage_end<NS>), dim3(nblocks(n, small_block(n))),
+                     dim3(small_block(n)), 0, s, U, Un, rhoi, rhon, Q, rhs, dt, J, c->dparams, c->g,
+                     lin, la, lb);
 }
 
 int launch_sweep_conv(f3d_ctx* c, int dir, float* rhs, const double* Q, const double* rhoi,

@@ -475,10 +475,11 @@ int launch_stage_end(f3d_ctx* c, int KRK, double* U, const double* Un, double* r
                      const int64_t* tag, hipStream_t s) {
   // F: Fx, Fy, Fz, Fvx, Fvy, Fvz, Fxi, Fyi, Fzi, Fdx, Fdy, Fdz
   const long n = (long)c->g.Nx * c->g.Ny * c->g.Nz;
+  const int blk = small_block(n);
   const int lin = KRK > 1;
   const double la = KRK == 2 ? 0.25 : 2.0 / 3.0, lb = KRK == 2 ? 0.75 : 1.0 / 3.0;
 #define F3D_SE(NS_, R_, W_)                                                                      \
-  hipLaunchKernelGGL((k_stage_end<NS_, R_, W_>), dim3(nblocks(n)), dim3(kBlock), 0, s, U, Un,   \
+  hipLaunchKernelGGL((k_stage_end<NS_, R_, W_>), dim3(nblocks(n, blk)), dim3(blk), 0, s, U, Un,          \
                      rhoi, rhon, Q, (const R_*)F[0], (const R_*)F[1], (const R_*)F[2],            \
                      (const R_*)F[3], (const R_*)F[4], (const R_*)F[5], (const R_*)F[6],          \
                      (const R_*)F[7], (const R_*)F[8], (const R_*)F[9], (const R_*)F[10],         \
@@ -530,10 +531,12 @@ static void mixture_ns(f3d_ctx* c, const double* Q, const double* rhoi, void* Yi
                        void* mu, void* D, const int64_t* tag, hipStream_t s) {
   const int NP = c->g.NP;
   if (c->precision == F3D_FP64)
-    hipLaunchKernelGGL((k_mixture<NS, double>), dim3(nblocks(NP)), dim3(kBlock), 0, s, Q, rhoi,
+    hipLaunchKernelGGL((k_mixture<NS, double>), dim3(nblocks(NP, small_block(NP))),
+                       dim3(small_block(NP)), 0, s, Q, rhoi,
                        (double*)Yi, (double*)lam, (double*)mu, (double*)D, tag, c->dparams, NP);
   else
-    hipLaunchKernelGGL((k_mixture<NS, float>), dim3(nblocks(NP)), dim3(kBlock), 0, s, Q, rhoi,
+    hipLaunchKernelGGL((k_mixture<NS, float>), dim3(nblocks(NP, small_block(NP))),
+                       dim3(small_block(NP)), 0, s, Q, rhoi,
                        (float*)Yi, (float*)lam, (float*)mu, (float*)D, tag, c->dparams, NP);
 }
 
@@ -621,7 +624,8 @@ int launch_fill(f3d_ctx* c, double* Q, double* U, double* rhoi, hipStream_t s) {
       if (!both) (turn == 0 ? b : a).depth = 0;
       const long n = (a.depth + b.depth) * plane;
       if (n == 0) continue;
-      hipLaunchKernelGGL(k_fill, dim3(nblocks(n)), dim3(kBlock), 0, s, Q, U, rhoi, g, dir, a, b,
+      const int blk = small_block(n);
+      hipLaunchKernelGGL(k_fill, dim3(nblocks(n, blk)), dim3(blk), 0, s, Q, U, rhoi, g, dir, a, b,
                          st);
       int rc = hip_check(hipGetLastError(), "fill");
       if (rc) return rc;

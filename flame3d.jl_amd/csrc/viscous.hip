@@ -457,7 +457,7 @@ int launch_viscous(f3d_ctx* c, int dir, void* Fv, const double* Q, const void* c
                    const int64_t* tag, hipStream_t s, bool mf) {
   const Geom& g = c->g;
   const long nf = (long)(g.Nx + (dir == 0)) * (g.Ny + (dir == 1)) * (g.Nz + (dir == 2));
-  const dim3 gr(nblocks(nf)), bl(kBlock);
+  const dim3 gr(nblocks(nf, small_block(nf))), bl(small_block(nf));
   if (c->precision == F3D_FP64) {
     const auto k = dir == 0   ? k_viscous<double, double, 0>
                    : dir == 1 ? k_viscous<double, double, 1>
@@ -494,7 +494,7 @@ static void spec_visc_ns(f3d_ctx* c, int dir, void* Fd, const double* Q, const v
                          const int64_t* tag, hipStream_t s, bool mf) {
   const Geom& g = c->g;
   const long nf = (long)(g.Nx + (dir == 0)) * (g.Ny + (dir == 1)) * (g.Nz + (dir == 2));
-  const dim3 gr(nblocks(nf)), bl(kBlock);
+  const dim3 gr(nblocks(nf, small_block(nf))), bl(small_block(nf));
   if (c->precision == F3D_FP64) {
     const auto k = dir == 0   ? k_spec_viscous<NS, double, double, 0>
                    : dir == 1 ? k_spec_viscous<NS, double, double, 1>
