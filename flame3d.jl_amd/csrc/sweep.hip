@@ -9,7 +9,7 @@
 // decomposition (solver.jl:22-56) never reach HBM; the stage end applies
 // U += J dt rhs (div.jl:16-84), linComb and c2Prim in one pass.
 //
-// x sweeps: one block of up to 320 threads per segment of up to 304 cells of an x line;
+// x sweeps: one block of 64 to 320 threads per segment of up to 304 cells of an x line;
 // the split fluxes (convective) or the face values (diffusive) of the segment
 // are staged in LDS so each point is read from HBM once and each face is
 // evaluated once; the face-flux difference of a cell reads its two faces
@@ -29,22 +29,31 @@
 
 namespace f3d {
 
-// x-line blocks: lines are split into equal segments of at most kXMost cells,
-// with threads in whole waves for a segment's cells and, in the diffusive
-// kernels, for its staged points as well (up to four more) and its last face.
-// With 256 cells and 256 threads these were second passes of the first and of
-// the last wave, the others waiting; a line of 300 cells took a second block of
-// 256 threads for 44 cells.  At 300x127x127 (air): convective 619 -> 461 us,
-// viscous 336 -> 184, species 308 -> 168; at 256^3 (H2/air) viscous 720 -> 639,
-// species 1022 -> 926.  The convective kernel, bound by instructions where the
-// flow has shocks, is slower with a wave for eight more points (256x128x128
-// with a shock, 282 us against 260), so there they stay a second pass.
+// x-line blocks: a line is one segment of up to kXMost cells, longer ones are
+// split into equal segments of at most kXMost (diffusive) or kXFew (convective)
+// cells.  The diffusive kernels have a thread for each of a segment's staged
+// points (four more than its cells) and its last face, in whole waves; with 256
+// cells and 256 threads these were second passes of the first and of the last
+// wave, the others waiting, and a line of 300 cells took a second block of 256
+// threads for 44 cells.  At 300x127x127 (air): convective 619 -> 461 us, viscous
+// 336 -> 184, species 308 -> 168; at 256^3 (H2/air) viscous 720 -> 639, species
+// 1022 -> 926.  The convective kernel, bound by instructions where the flow has
+// shocks, is slower with a wave for its eight more points (256x128x128 with a
+// shock, 282 us against 260), so there they stay a second pass.
+// kXMost: at most kXThreads - 4 = 316.  With 316 the larger tiles cost lines of
+// 257..304 cells 1-2 % in the diffusive sweeps, and lines of 305..316 cells gain
+// 5 % there (one segment instead of two) and lose up to 9 % in the convective
+// sweep of nine species.
 constexpr int kXThreads = 320, kXMost = 304;
 // MOST: the cells a kernel's LDS holds, kXMost (the _long kernels), kXFew or
 // kXShort (the _short kernels): the less, the more blocks fit a compute unit.
 // At 256^3 with kXMost instead of kXFew: convective 741 instead of 639 us,
 // species 1176 instead of 926; at 128^3 (H2/air with a shock) with kXFew instead
 // of kXShort: 196, 126 instead of 163, 111 (256 threads for 128 cells: 180, 192).
+// The convective kernel of kXFew cells always has 256 threads, a constant of its
+// loops, and takes the lines of more than kXMost cells too (2^21 cells, H2/air):
+// 192-cell lines 87 us, against 94 with whole waves for the cells; 560-cell
+// lines 92 us in three segments, against 109 in two of the _long kernel.
 constexpr int kXFew = 256, kXShort = 128;
 constexpr int kConvSeg = 32;  // cells per march segment (convective)
 constexpr int kViscSeg = 64;  // cells per march segment (viscous)
@@ -57,8 +66,7 @@ __device__ inline void rhs_put(float* __restrict__ r, long i, float d, int acc) 
 struct XSegment {
   int b, c, c0, nc;  // line (b, c), first cell, cells
 };
-__device__ inline XSegment x_segment(const Geom& g, int seg) {
-  const unsigned nseg = (g.Nx + seg - 1) / seg;
+__device__ inline XSegment x_segment(const Geom& g, int seg, unsigned nseg) {
   const unsigned L = xcd_block();
   const unsigned line = L / nseg;
   XSegment x;
@@ -72,24 +80,26 @@ __device__ inline XSegment x_segment(const Geom& g, int seg) {
 // ---------------------------------------------------------------------------
 // Convective x sweep
 // ---------------------------------------------------------------------------
-template <int NS, int MOST>
+// THREADS: the block's threads, 0: as launched
+template <int NS, int MOST, int THREADS>
 __device__ __forceinline__ void conv_x_line(
     float* __restrict__ rhs, const double* __restrict__ Q,
     const double* __restrict__ rhoi, const float* __restrict__ A1,
     const float* __restrict__ A2, const float* __restrict__ A3,
     const float* __restrict__ phi, const DevParams* __restrict__ P, Geom g,
-    int acc, int seg) {
+    int acc, int seg, unsigned nseg) {
   constexpr int NV = 5 + NS;
   constexpr int NPT = MOST + 8;
-  static_assert(MOST <= kXThreads, "a thread to a cell");
+  static_assert(MOST <= (THREADS > 0 ? THREADS : kXThreads), "a thread to a cell");
   __shared__ float sp[NV][NPT];
   __shared__ float sm[NV][NPT];
   __shared__ float sphi[NPT];
-  const XSegment x = x_segment(g, seg);
+  const XSegment x = x_segment(g, seg, nseg);
   const int nc = x.nc;
   const int t = threadIdx.x;
+  const int threads = THREADS > 0 ? THREADS : (int)blockDim.x;
   const long NP = g.NP;
-  for (int i = t; i < nc + 8; i += blockDim.x) {
+  for (int i = t; i < nc + 8; i += threads) {
     // point i of the segment is padded c0 + i (cell c0 + i - NG)
     const long p = (long)x.c0 + (long)g.Nxt * ((x.b + NG) + (long)g.Nyt * (x.c + NG)) + i;
     const float sw = PT<float>::sweps2(P);
@@ -127,10 +137,10 @@ __device__ __forceinline__ void conv_x_line(
       }
     }, fv);
   }
-  // the segment's last face, one variable per thread (those after the cells, if
-  // there are enough of them)
+  // the segment's last face, one variable per thread (in a block of whole waves
+  // those after the cells, if there are enough of them)
   float fl = 0.0f;
-  const int n1 = (int)blockDim.x - nc >= NV ? t - nc : t;
+  const int n1 = THREADS == 0 && threads - nc >= NV ? t - nc : t;
   if (n1 >= 0 && n1 < NV) {
     const int br = weno_branch<float>(fmaxf(sphi[nc + 3], sphi[nc + 4]), P);
     float pv[8], mv[8];
@@ -157,14 +167,14 @@ __device__ __forceinline__ void conv_x_line(
 }
 
 template <int NS>
-__global__ void __launch_bounds__(kXThreads)
+__global__ void __launch_bounds__(kXFew)
     k_sw_conv_x(
         float* __restrict__ rhs, const double* __restrict__ Q,
         const double* __restrict__ rhoi, const float* __restrict__ A1,
         const float* __restrict__ A2, const float* __restrict__ A3,
         const float* __restrict__ phi, const DevParams* __restrict__ P, Geom g,
-        int acc, int seg) {
-  conv_x_line<NS, kXFew>(rhs, Q, rhoi, A1, A2, A3, phi, P, g, acc, seg);
+        int acc, int seg, unsigned nseg) {
+  conv_x_line<NS, kXFew, kXFew>(rhs, Q, rhoi, A1, A2, A3, phi, P, g, acc, seg, nseg);
 }
 
 template <int NS>
@@ -174,8 +184,8 @@ __global__ void __launch_bounds__(kXThreads)
         const double* __restrict__ rhoi, const float* __restrict__ A1,
         const float* __restrict__ A2, const float* __restrict__ A3,
         const float* __restrict__ phi, const DevParams* __restrict__ P, Geom g,
-        int acc, int seg) {
-  conv_x_line<NS, kXMost>(rhs, Q, rhoi, A1, A2, A3, phi, P, g, acc, seg);
+        int acc, int seg, unsigned nseg) {
+  conv_x_line<NS, kXMost, 0>(rhs, Q, rhoi, A1, A2, A3, phi, P, g, acc, seg, nseg);
 }
 
 template <int NS>
@@ -185,8 +195,8 @@ __global__ void __launch_bounds__(kXThreads)
         const double* __restrict__ rhoi, const float* __restrict__ A1,
         const float* __restrict__ A2, const float* __restrict__ A3,
         const float* __restrict__ phi, const DevParams* __restrict__ P, Geom g,
-        int acc, int seg) {
-  conv_x_line<NS, kXShort>(rhs, Q, rhoi, A1, A2, A3, phi, P, g, acc, seg);
+        int acc, int seg, unsigned nseg) {
+  conv_x_line<NS, kXShort, 0>(rhs, Q, rhoi, A1, A2, A3, phi, P, g, acc, seg, nseg);
 }
 
 // ---------------------------------------------------------------------------
@@ -474,13 +484,14 @@ template <int MOST>
 __device__ __forceinline__ void visc_x_line(
     float* __restrict__ rhs, const double* __restrict__ Q, FMet M,
     const float* __restrict__ J, const float* __restrict__ lam,
-    const float* __restrict__ mu, Geom g, int seg) {
+    const float* __restrict__ mu, Geom g, int seg, unsigned nseg) {
+  static_assert(MOST + 4 <= kXThreads, "a thread to a staged point");
   constexpr int NE = MOST + 2;  // cells -1 .. nc
   constexpr int NQ = MOST + 4;  // cells -2 .. nc + 1
   __shared__ float sm[12][NE];    // metrics, J, mu, lambda
   __shared__ float sq[2][NQ], sy[2][NE], sz[2][NE];
   __shared__ float sf[4][MOST + 1];
-  const XSegment x = x_segment(g, seg);
+  const XSegment x = x_segment(g, seg, nseg);
   const int nc = x.nc;
   const int t = threadIdx.x;
   const long NP = g.NP, ty = g.Nxt, tz = (long)g.Nxt * g.Nyt;
@@ -585,24 +596,24 @@ __global__ void __launch_bounds__(kXThreads)
     k_sw_visc_x(
         float* __restrict__ rhs, const double* __restrict__ Q, FMet M,
         const float* __restrict__ J, const float* __restrict__ lam,
-        const float* __restrict__ mu, Geom g, int seg) {
-  visc_x_line<kXFew>(rhs, Q, M, J, lam, mu, g, seg);
+        const float* __restrict__ mu, Geom g, int seg, unsigned nseg) {
+  visc_x_line<kXFew>(rhs, Q, M, J, lam, mu, g, seg, nseg);
 }
 
 __global__ void __launch_bounds__(kXThreads)
     k_sw_visc_x_long(
         float* __restrict__ rhs, const double* __restrict__ Q, FMet M,
         const float* __restrict__ J, const float* __restrict__ lam,
-        const float* __restrict__ mu, Geom g, int seg) {
-  visc_x_line<kXMost>(rhs, Q, M, J, lam, mu, g, seg);
+        const float* __restrict__ mu, Geom g, int seg, unsigned nseg) {
+  visc_x_line<kXMost>(rhs, Q, M, J, lam, mu, g, seg, nseg);
 }
 
 __global__ void __launch_bounds__(kXThreads)
     k_sw_visc_x_short(
         float* __restrict__ rhs, const double* __restrict__ Q, FMet M,
         const float* __restrict__ J, const float* __restrict__ lam,
-        const float* __restrict__ mu, Geom g, int seg) {
-  visc_x_line<kXShort>(rhs, Q, M, J, lam, mu, g, seg);
+        const float* __restrict__ mu, Geom g, int seg, unsigned nseg) {
+  visc_x_line<kXShort>(rhs, Q, M, J, lam, mu, g, seg, nseg);
 }
 
 // x-line block of the species-diffusion sweep with each cell's inputs read
@@ -622,7 +633,9 @@ template <int NS, int MOST>
 __device__ __forceinline__ void spec_x_line(
     float* __restrict__ rhs, const double* __restrict__ Q,
     const float* __restrict__ Yi, FMet M, const float* __restrict__ J,
-    const float* __restrict__ D, const DevParams* __restrict__ P, Geom g, int seg) {
+    const float* __restrict__ D, const DevParams* __restrict__ P, Geom g, int seg,
+    unsigned nseg) {
+  static_assert(MOST + 4 <= kXThreads, "a thread to a staged point");
   constexpr int NE = MOST + 2;  // cells -1 .. nc
   constexpr int NY = MOST + 4;  // cells -2 .. nc + 1
   __shared__ float sy[2][NY], scy[2][NE], scz[2][NE], sd[2][NE];
@@ -632,7 +645,7 @@ __device__ __forceinline__ void spec_x_line(
   } sh;
   auto& sm = sh.m;
   auto& sf = sh.f;
-  const XSegment x = x_segment(g, seg);
+  const XSegment x = x_segment(g, seg, nseg);
   const int nc = x.nc;
   const int t = threadIdx.x;
   const long NP = g.NP, ty = g.Nxt, tz = (long)g.Nxt * g.Nyt;
@@ -744,8 +757,9 @@ __global__ void __launch_bounds__(kXThreads) __attribute__((amdgpu_waves_per_eu(
     k_sw_spec_x(
         float* __restrict__ rhs, const double* __restrict__ Q,
         const float* __restrict__ Yi, FMet M, const float* __restrict__ J,
-        const float* __restrict__ D, const DevParams* __restrict__ P, Geom g, int seg) {
-  spec_x_line<NS, kXFew>(rhs, Q, Yi, M, J, D, P, g, seg);
+        const float* __restrict__ D, const DevParams* __restrict__ P, Geom g, int seg,
+        unsigned nseg) {
+  spec_x_line<NS, kXFew>(rhs, Q, Yi, M, J, D, P, g, seg, nseg);
 }
 
 template <int NS>
@@ -753,8 +767,9 @@ __global__ void __launch_bounds__(kXThreads) __attribute__((amdgpu_waves_per_eu(
     k_sw_spec_x_long(
         float* __restrict__ rhs, const double* __restrict__ Q,
         const float* __restrict__ Yi, FMet M, const float* __restrict__ J,
-        const float* __restrict__ D, const DevParams* __restrict__ P, Geom g, int seg) {
-  spec_x_line<NS, kXMost>(rhs, Q, Yi, M, J, D, P, g, seg);
+        const float* __restrict__ D, const DevParams* __restrict__ P, Geom g, int seg,
+        unsigned nseg) {
+  spec_x_line<NS, kXMost>(rhs, Q, Yi, M, J, D, P, g, seg, nseg);
 }
 
 template <int NS>
@@ -762,8 +777,9 @@ __global__ void __launch_bounds__(kXThreads) __attribute__((amdgpu_waves_per_eu(
     k_sw_spec_x_short(
         float* __restrict__ rhs, const double* __restrict__ Q,
         const float* __restrict__ Yi, FMet M, const float* __restrict__ J,
-        const float* __restrict__ D, const DevParams* __restrict__ P, Geom g, int seg) {
-  spec_x_line<NS, kXShort>(rhs, Q, Yi, M, J, D, P, g, seg);
+        const float* __restrict__ D, const DevParams* __restrict__ P, Geom g, int seg,
+        unsigned nseg) {
+  spec_x_line<NS, kXShort>(rhs, Q, Yi, M, J, D, P, g, seg, nseg);
 }
 
 // ---------------------------------------------------------------------------
@@ -1084,17 +1100,19 @@ __global__ void __launch_bounds__(kBlock)
 }
 
 // ---- launchers --------------------------------------------------------------
-// Segment length, blocks and threads (a multiple of a wave that holds a
-// segment's cells and `more` staged points) of the x-line kernels.
+// Segments of at most `most` cells of the x-line kernels, their length, the
+// launch's blocks and its threads (a multiple of a wave that holds a segment's
+// cells and `more` staged points).
 struct XLaunch {
   int seg;
-  unsigned blocks, threads;
+  unsigned nseg, blocks, threads;
 };
-static XLaunch x_launch(const Geom& g, int more) {
-  const int nseg = (g.Nx + kXMost - 1) / kXMost;
+static XLaunch x_launch(const Geom& g, int more, int most) {
+  const int n = (g.Nx + most - 1) / most;
   XLaunch l;
-  l.seg = (g.Nx + nseg - 1) / nseg;
-  l.blocks = (unsigned)((g.Nx + l.seg - 1) / l.seg) * g.Ny * g.Nz;
+  l.seg = (g.Nx + n - 1) / n;
+  l.nseg = (unsigned)((g.Nx + l.seg - 1) / l.seg);
+  l.blocks = l.nseg * g.Ny * g.Nz;
   l.threads = (l.seg + more + 63) / 64 * 64;
   return l;
 }
@@ -1106,11 +1124,12 @@ static void conv_ns(f3d_ctx* c, int dir, float* rhs, const double* Q, const doub
                     const float* const* A, const float* phi, int acc, hipStream_t s) {
   const Geom& g = c->g;
   if (dir == 0) {
-    const XLaunch l = x_launch(g, 0);
+    XLaunch l = x_launch(g, 0, g.Nx <= kXMost ? kXMost : kXFew);
+    if (l.seg > kXShort && l.seg <= kXFew) l.threads = kXFew;  // k_sw_conv_x's
     const auto k = l.seg <= kXShort ? k_sw_conv_x_short<NS>
                    : l.seg <= kXFew ? k_sw_conv_x<NS> : k_sw_conv_x_long<NS>;
     hipLaunchKernelGGL(k, dim3(l.blocks), dim3(l.threads), 0, s, rhs, Q, rhoi,
-                       A[0], A[1], A[2], phi, c->dparams, g, acc, l.seg);
+                       A[0], A[1], A[2], phi, c->dparams, g, acc, l.seg, l.nseg);
   } else {
     const int nd = dir == 1 ? g.Ny : g.Nz;
     const unsigned nl = (g.Nx + 63) / 64, nt = dir == 1 ? g.Nz : g.Ny;
@@ -1150,15 +1169,15 @@ static void diff_ns(f3d_ctx* c, int dir, float* rhs, const double* Q, const floa
                     const float* D, hipStream_t s) {
   const Geom& g = c->g;
   if (dir == 0) {
-    const XLaunch l = x_launch(g, 4);
+    const XLaunch l = x_launch(g, 4, kXMost);
     const auto kv = l.seg <= kXShort ? k_sw_visc_x_short
                     : l.seg <= kXFew ? k_sw_visc_x : k_sw_visc_x_long;
     const auto ks = l.seg <= kXShort ? k_sw_spec_x_short<NS>
                     : l.seg <= kXFew ? k_sw_spec_x<NS> : k_sw_spec_x_long<NS>;
     hipLaunchKernelGGL(kv, dim3(l.blocks), dim3(l.threads), 0, s, rhs, Q, M, J, lam, mu,
-                       g, l.seg);
+                       g, l.seg, l.nseg);
     hipLaunchKernelGGL(ks, dim3(l.blocks), dim3(l.threads), 0, s, rhs, Q, Yi, M,
-                       J, D, c->dparams, g, l.seg);
+                       J, D, c->dparams, g, l.seg, l.nseg);
   } else {
     const int nd = dir == 1 ? g.Ny : g.Nz;
     const unsigned nl = (g.Nx + 63) / 64, nt = dir == 1 ? g.Nz : g.Ny;

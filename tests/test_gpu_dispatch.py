@@ -143,3 +143,21 @@ def test_x_line_segments(mech, nx, scheme):
     _cmp(f[0], g[0], "dU", 1e-4)
     _cmp(f[1], g[1], "drho_k", 1e-4)
     _cmp(f[2], g[2], "Q", 1e-5)
+
+
+@pytest.mark.parametrize("mech,nx,scheme", [
+    ("h2_lidryer", 192, None), ("air5", 193, "weno7"), ("h2_lidryer", 512, None),
+    ("air5", 513, None), ("h2_lidryer", 608, "weno7"), ("air5", 769, None)])
+def test_x_lines_of_different_segments(mech, nx, scheme):
+    """Lines that the convective sweep takes in other segments than the
+    diffusive ones (more than 304 cells: at most 256 a segment against 304), and
+    those whose cells end below the convective kernel's fixed 256 threads; the
+    granular stage's bars of test_gpu_sweeps."""
+    import flame3d_amd.abi as abi
+    from test_gpu_sweeps import _cmp, _stage_pair
+    sc = {"recon_kind": abi.RECON_WENO7} if scheme else None
+    print(f"\n[x lines] {mech} nx={nx} {scheme}", flush=True)
+    f, g = _stage_pair(mech, (nx, 4, 5), scheme=sc)
+    _cmp(f[0], g[0], "dU", 1e-4)
+    _cmp(f[1], g[1], "drho_k", 1e-4)
+    _cmp(f[2], g[2], "Q", 1e-5)
