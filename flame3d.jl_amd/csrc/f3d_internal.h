@@ -327,13 +327,15 @@ struct NasaTab {
 };
 
 // a / b for a constant b > 0 of the parameter block with rb = 1 / b rounded:
-// one Newton correction of a rb by its exact remainder, four instructions of
-// full rate instead of a division's eleven.  The result is the rounded
-// quotient unless that lies within 2^-51 ulp of a rounding boundary (or a is
-// so small that the remainder is subnormal).
+// one Newton correction of a rb by its exact remainder (a product and two fused
+// multiply-adds) and the division's own last instruction, which puts back what
+// an infinite a gives (its remainder is not a number): four instructions of
+// full rate instead of a division's eleven.  The result is the rounded quotient
+// unless that lies within 2^-51 ulp of a rounding boundary (or a is so small
+// that the remainder is subnormal).
 __device__ __forceinline__ double div_const(double a, double b, double rb) {
   const double q = a * rb;
-  return fma(fma(-q, b, a), rb, q);
+  return __builtin_amdgcn_div_fixup(fma(fma(-q, b, a), rb, q), b, a);
 }
 
 // InternalEnergy, thermo.jl:219-228, and CV, thermo.jl:194-203 (FP64), at the

@@ -161,3 +161,35 @@ def test_x_lines_of_different_segments(mech, nx, scheme):
     _cmp(f[0], g[0], "dU", 1e-4)
     _cmp(f[1], g[1], "drho_k", 1e-4)
     _cmp(f[2], g[2], "Q", 1e-5)
+
+
+@pytest.mark.parametrize("mech", ["air5", "h2_lidryer"])
+def test_infinite_density(mech):
+    """An infinite partial density leaves what does not depend on it as the
+    oracle has it (its own D_k is a sum over the other species: 0), and an
+    infinite density reads as an infinite pressure: a state that has run away
+    does not turn into a small finite one."""
+    import flame3d_amd.abi as abi
+    import flame3d_amd.mech as mm
+    from oracle import Oracle
+    m = mm.load(mech)
+    shape = (4, 4, 4)
+    _, Q, rhoi = _state(shape, m)
+    ctx, orc = abi.Context(*shape, m, "fp64"), Oracle(*shape, m)
+    U = ctx.zeros(5)
+    Qg, rg = Q.cuda(), rhoi.cuda()
+    ctx.prim2c(U, Qg)
+    rg[1, 7, 6, 5] = float("inf")
+    out = [ctx.zeros(m.Ns), ctx.zeros(), ctx.zeros(), ctx.zeros(m.Ns)]
+    ctx.mixture(Qg, rg, *out)
+    torch.cuda.synchronize()
+    ref = orc.mixture(to_np(Qg), to_np(rg))
+    for got, want in zip(out, ref):
+        assert np.allclose(to_np(got)[5, 6, 7], want[5, 6, 7], rtol=1e-12, atol=0, equal_nan=True)
+    assert float(out[3][1, 7, 6, 5]) == 0.0
+    rg = rhoi.cuda()
+    U[0, 7, 6, 5] = float("inf")
+    ctx.c2prim(U, Qg, rg)
+    torch.cuda.synchronize()
+    assert float(Qg[4, 7, 6, 5]) == float("inf")
+    ctx.close()
