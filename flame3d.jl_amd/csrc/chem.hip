@@ -38,10 +38,6 @@ constexpr int kNewtonMaxSub = 64;
 // 0.90 with 6, 0.88 with 5, 0.87 with 4 (1.23 ms all here); but with 4 a tenth
 // of a flame's cells would go.
 constexpr int kNewtonFirst = 5;
-// Most cells that go: two for each half wave the device holds.  A half wave
-// has a twentieth of the one-thread solve's throughput, so where slow cells
-// are many the rest go on in their threads.
-constexpr int kRowsMost = 4096;
 
 // One backward-Euler solve over h of the reactor (rho_k, T) from (r, T),
 // total energy fixed at E0: Newton on

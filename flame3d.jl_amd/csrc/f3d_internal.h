@@ -104,6 +104,9 @@ struct f3d_ctx {
   int32_t* nn_fbcount = nullptr;  // rejected cells per 64-cell tile, then their offsets
   int32_t* nn_fblist = nullptr;   // rejected cell ids in cell order [Nx*Ny*Nz]
   int32_t* nn_fbtotal = nullptr;  // number of rejected cells, and of those taken a second time
+  // cells taken a second time [kRowsMost]; holds cell numbers only (zeros before
+  // the first): they are used as indices
+  int32_t* nn_later = nullptr;
   float* nn_out = nullptr;        // the network's raw outputs [Ns][Nx*Ny*Nz] for the epilogue
   double* nn_cand = nullptr;      // the epilogue's candidate states [Ns + 3][Nx*Ny*Nz]
   // f3d_nn_timing: events around the last f3d_nn_chem's network kernel, its
@@ -146,6 +149,11 @@ inline int fill_segments(int n0, long cap, long lines, int nd) {
   const int want = n > most ? most : (int)n;
   return want >= 2 * n0 ? want : n0;
 }
+// Most cells of a list pass that go to the half-wave solve (f3d_chem_rows.h):
+// two for each half wave the device holds.  A half wave has a twentieth of the
+// one-thread solve's throughput, so where slow cells are many the rest go on in
+// their threads.
+constexpr int kRowsMost = 4096;
 // Resident blocks of a kernel on the current device (queried once per context
 // and kernel; *slot keeps it).
 template <class K>

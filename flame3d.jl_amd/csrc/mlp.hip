@@ -1020,8 +1020,8 @@ void nn_free(f3d_ctx* c) {
   void** ptrs[] = {(void**)&c->nn_master, (void**)&c->nn_m1, (void**)&c->nn_m2,
                    (void**)&c->nn_Wb, (void**)&c->nn_Wtb, (void**)&c->nn_partial,
                    (void**)&c->nn_cfg, (void**)&c->nn_status, (void**)&c->nn_fbcount,
-                   (void**)&c->nn_fblist, (void**)&c->nn_fbtotal, (void**)&c->nn_out,
-                   (void**)&c->nn_cand};
+                   (void**)&c->nn_fblist, (void**)&c->nn_fbtotal, (void**)&c->nn_later,
+                   (void**)&c->nn_out, (void**)&c->nn_cand};
   for (void** q : ptrs) {
     if (*q) (void)hipFree(*q);
     *q = nullptr;
@@ -1136,6 +1136,7 @@ int f3d_nn_init(f3d_ctx* c, const f3d_nn_config* cfg) {
                hipMalloc(&c->nn_fbcount, sizeof(int32_t) * (ntile + nchunk)) == hipSuccess &&
                hipMalloc(&c->nn_fblist, sizeof(int32_t) * ncell) == hipSuccess &&
                hipMalloc(&c->nn_fbtotal, 2 * sizeof(int32_t)) == hipSuccess &&
+               hipMalloc(&c->nn_later, sizeof(int32_t) * kRowsMost) == hipSuccess &&
                hipMalloc(&c->nn_out, sizeof(float) * ncell * ns) == hipSuccess &&
                hipMalloc(&c->nn_cand, sizeof(double) * ncell * (ns + 3)) == hipSuccess;
     if (!okm) {
@@ -1148,6 +1149,7 @@ int f3d_nn_init(f3d_ctx* c, const f3d_nn_config* cfg) {
     (void)hipMemset(c->nn_m2, 0, sizeof(float) * NN_NPARAM);
     (void)hipMemset(c->nn_Wb, 0, 2 * NN_NPARAM);
     (void)hipMemset(c->nn_Wtb, 0, 2 * NN_NPARAM);
+    (void)hipMemset(c->nn_later, 0, sizeof(int32_t) * kRowsMost);
     c->nn_ready = true;
   }
   c->nn_dt = cfg->dt;
@@ -1340,7 +1342,7 @@ int f3d_nn_chem(f3d_ctx* c, double* U, double* Q, double* rhoi, double dt, int32
   if (timed) (void)hipEventRecord(c->nn_ev[4], s);  // after the read-back
   if (nfb > 0) {
     rc = launch_chem(c, 2, U, Q, rhoi, dt, maxiter, rtol, ttol, nullptr, tag, s, c->nn_fblist,
-                     nfb, reinterpret_cast<int32_t*>(c->nn_out), c->nn_fbtotal + 1);
+                     nfb, c->nn_later, c->nn_fbtotal + 1);
     if (rc) return rc;
   }
   if (timed) {

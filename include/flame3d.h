@@ -303,7 +303,9 @@ int f3d_nn_forward(f3d_ctx* ctx, const float* X, float* Y, int32_t B, hipStream_
  * 3 element balance, 4 positivity, 5 predicted temperature change,
  * 6 backward-Euler residual, 7 thermal explosiveness, 8 chain explosiveness.
  * *n_fallback (host) receives the number of fallback cells; this call
- * synchronizes the stream to size the fallback launch. */
+ * synchronizes the stream to size the fallback launch, which still runs when
+ * it returns.  The lists and predictions of a call live in the context: calls
+ * on one context must follow each other in stream order. */
 int f3d_nn_chem(f3d_ctx* ctx, double* U, double* Q, double* rhoi, double dt, int32_t maxiter,
                 double rtol, double ttol, int8_t* status, int64_t* n_fallback, const int64_t* tag,
                 hipStream_t s);
