@@ -114,6 +114,11 @@ __global__ void __launch_bounds__(kBlock)
 // the sum is known (174 VGPRs, two waves per SIMD).  128^3, 9 species, FP64:
 // 357 -> 195 us (x), 240 us (y, z: 72 % of the L1's access rate), of which the
 // slab order of the lines took the fetched bytes from 1.08 to 0.60 GB.
+// FP32 (x direction of the granular path) keeps each species' velocity until
+// the sum is known: subtracted after the sums over h, the correction leaves the
+// rounding of the sums instead of that of the difference (61x40x37 skewed
+// blocks, H2: error of Fh against FP64 up to 4.0e-7 of its maximum, 3.0e-7 so),
+// and the register count is no limit there.
 template <int NS, typename R, typename MT, int DIR>
 __global__ void __launch_bounds__(kBlock)
     k_spec_viscous(R* __restrict__ Fd, const double* __restrict__ Q, const R* __restrict__ Yi,
@@ -142,7 +147,9 @@ __global__ void __launch_bounds__(kBlock)
   const R rho = ((R)Q[im] + (R)Q[ic]) * R(0.5);
   const R T = ((R)Q[im + 5 * NP] + (R)Q[ic + 5 * NP]) * R(0.5);
   const R n0 = m[3 * DIR], n1 = m[3 * DIR + 1], n2 = m[3 * DIR + 2];
+  constexpr bool kLinear = sizeof(R) == 8;
   R Vn[NS], Yn[NS];
+  R Vk[kLinear ? 1 : NS][3], hi[kLinear ? 1 : NS];
   R sum1 = 0, sum2 = 0, sum3 = 0;  // sum_k V_k
   R fh1 = 0, fh2 = 0, fh3 = 0;     // sum_k V_k h_k
   R yh = 0;                        // sum_k Y_k h_k
@@ -164,10 +171,17 @@ __global__ void __launch_bounds__(kBlock)
     const R Vz = (dY[0] * m[2] + dY[1] * m[5] + dY[2] * m[8]) * Jac * rhoDi;
     const R hk = H.h(P, n);
     Yn[n] = R(0.5) * (y[im] + y[ic]);
-    Vn[n] = Vx * n0 + Vy * n1 + Vz * n2;
     sum1 += Vx;
     sum2 += Vy;
     sum3 += Vz;
+    if constexpr (!kLinear) {
+      Vk[n][0] = Vx;
+      Vk[n][1] = Vy;
+      Vk[n][2] = Vz;
+      hi[n] = hk;
+      continue;
+    }
+    Vn[n] = Vx * n0 + Vy * n1 + Vz * n2;
     fh1 += Vx * hk;
     fh2 += Vy * hk;
     fh3 += Vz * hk;
@@ -181,6 +195,22 @@ __global__ void __launch_bounds__(kBlock)
 #pragma unroll
       for (int k = n - 2; k <= n; ++k) asm volatile("" : "+v"(Vn[k]), "+v"(Yn[k]));
     }
+  }
+  if constexpr (!kLinear) {
+#pragma unroll
+    for (int n = 0; n < NS; ++n) {
+      const R V1 = Vk[n][0] - sum1 * Yn[n];
+      const R V2 = Vk[n][1] - sum2 * Yn[n];
+      const R V3 = Vk[n][2] - sum3 * Yn[n];
+      Fd[f + n * nf] = V1 * n0 + V2 * n1 + V3 * n2;
+      fh1 += V1 * hi[n];
+      fh2 += V2 * hi[n];
+      fh3 += V3 * hi[n];
+    }
+    Fh[f] = fh1;
+    Fh[f + nf] = fh2;
+    Fh[f + 2 * nf] = fh3;
+    return;
   }
   const R sn = sum1 * n0 + sum2 * n1 + sum3 * n2;
 #pragma unroll

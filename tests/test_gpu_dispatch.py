@@ -193,3 +193,28 @@ def test_infinite_density(mech):
     torch.cuda.synchronize()
     assert float(Qg[4, 7, 6, 5]) == float("inf")
     ctx.close()
+
+
+@pytest.mark.parametrize("d", [0, 1, 2])
+def test_single_species_has_no_diffusion_flux(d):
+    """FP32 species faces: V_k - Y_k sum V is formed before it is multiplied by
+    the enthalpy, so one species whose mass fraction at the face is one (0.75 and
+    1.25 in turn along the sweep: a gradient, but a mean of 1) has no flux and
+    carries no enthalpy: zero, not the rounding of two sums."""
+    import flame3d_amd.abi as abi
+    import flame3d_amd.cases as cases
+    m = cases.tgv_gas()
+    shape = (9, 8, 7)
+    grid, Q, rhoi = _state(shape, m)
+    ctx = abi.Context(*shape, m, "fp32")
+    Q = Q.cuda()
+    n = torch.arange(Q.shape[3 - d], device="cuda") % 2
+    Y = (0.75 + 0.5 * n).float().reshape([-1 if 2 - d == k else 1 for k in range(3)])
+    Y = Y.expand(Q.shape[1:]).contiguous()[None]
+    D = ctx.rzeros(1) + 1e-4 * (1 + torch.rand(Q.shape[1:], device="cuda"))
+    Fd, Fh = ctx.face_zeros(d, 1) + 1, ctx.face_zeros(d, 3) + 1
+    ctx.spec_viscous_flux(d, Fd, Q, Y.contiguous(), [x.cuda() for x in grid.metrics],
+                          grid.J.cuda(), D, Fh)
+    torch.cuda.synchronize()
+    assert int((Fd != 0).sum()) == 0 and int((Fh != 0).sum()) == 0
+    ctx.close()
