@@ -183,7 +183,7 @@ __global__ void __launch_bounds__(chem_block(MODE)) __attribute__((amdgpu_waves_
            int maxiter, double rtol, double ttol, int32_t* __restrict__ iters,
            const int64_t* __restrict__ tag, const DevParams* __restrict__ P, Geom g, int bug,
            const int32_t* __restrict__ list, long nwork, int32_t* __restrict__ later,
-           int32_t* __restrict__ nlater) {
+           int32_t* __restrict__ nlater, int most) {
   __shared__ NasaTab<NS> N;
   N.fill(P);
   // one thread per interior cell, or per entry of an ordered cell list (the
@@ -265,11 +265,17 @@ __global__ void __launch_bounds__(chem_block(MODE)) __attribute__((amdgpu_waves_
                              it);
       if (first && !ok) {  // left to k_newton_rows, from the start, or begun again here
         const int slot = atomicAdd(nlater, 1);
-        if (slot < kRowsMost) {
+        if (slot < most) {
           later[slot] = (int32_t)id;
           return;
         }
         first = false;
+        // a solve that had all its iterations or left the admissible set would
+        // only fail again
+        bool failed = maxiter <= kNewtonFirst || !(T > T_lo && T < T_hi);
+#pragma unroll
+        for (int n = 0; n < NS; ++n) failed = failed || !(r[n] > -rho_tot);
+        if (failed) nsub *= 2;
         continue;
       }
       if (!ok) nsub *= 2;
@@ -296,13 +302,16 @@ static void chem_k(f3d_ctx* c, int mode, double* U, double* Q, double* rhoi, dou
   const int bug = c->bug_compat & 1;
   if (mode == 0)
     hipLaunchKernelGGL((k_chem<NS, 0, K>), dim3(nblocks(n)), dim3(kBlock), 0, s, U, Q, rhoi, dt,
-                       maxiter, rtol, ttol, iters, tag, c->dparams, c->g, bug, list, n, nullptr, nullptr);
+                       maxiter, rtol, ttol, iters, tag, c->dparams, c->g, bug, list, n, nullptr,
+                       nullptr, 0);
   else if (mode == 1)
     hipLaunchKernelGGL((k_chem<NS, 1, K>), dim3(nblocks(n)), dim3(kBlock), 0, s, U, Q, rhoi, dt,
-                       maxiter, rtol, ttol, iters, tag, c->dparams, c->g, bug, list, n, nullptr, nullptr);
+                       maxiter, rtol, ttol, iters, tag, c->dparams, c->g, bug, list, n, nullptr,
+                       nullptr, 0);
   else
     hipLaunchKernelGGL((k_chem<NS, 2, K>), dim3(nblocks(n, chem_block(2))), dim3(chem_block(2)),
-                       0, s, U, Q, rhoi, dt, maxiter, rtol, ttol, iters, tag, c->dparams, c->g, bug, list, n, later, nlater);
+                       0, s, U, Q, rhoi, dt, maxiter, rtol, ttol, iters, tag, c->dparams, c->g, bug,
+                       list, n, later, nlater, rows_most(n));
 }
 
 // the list pass's slow cells: as many waves as the device holds stride over them
@@ -310,11 +319,12 @@ template <class T>
 static void launch_rows(f3d_ctx* c, double* U, double* Q, double* rhoi, double dt, int maxiter,
                         double rtol, double ttol, hipStream_t s, long nlist,
                         const int32_t* later, const int32_t* nlater) {
-  const long most = std::min(nlist, (long)kRowsMost);
+  const int cap = rows_most(nlist);
+  const long most = std::min(nlist, (long)cap);
   const long nb = std::min(resident_blocks(&k_newton_rows<T>, 64, &c->rows_blocks),
                            (most + kRowCells - 1) / kRowCells);
   hipLaunchKernelGGL((k_newton_rows<T>), dim3((unsigned)nb), dim3(64), 0, s, U, Q, rhoi, dt,
-                     maxiter, rtol, ttol, c->dparams, c->g, kNewtonMaxSub, later, nlater, kRowsMost);
+                     maxiter, rtol, ttol, c->dparams, c->g, kNewtonMaxSub, later, nlater, cap);
 }
 
 // the compiled-in tables of the context's mechanism when it is one of the
@@ -353,6 +363,7 @@ int launch_chem(f3d_ctx* c, int mode, double* U, double* Q, double* rhoi, double
     set_error("bug_compat coeffs_lo[n,6] read needs Ns >= 6 (it reads past the array for Ns < 6)");
     return F3D_ERR_ARG;
   }
+  if (rows_most(nlist) == 0) later = nullptr;
   switch (c->g.Ns) {
     case 5: chem_ns<5>(c, mode, U, Q, rhoi, dt, maxiter, rtol, ttol, iters, tag, s, list, nlist, later, nlater); break;
     case 9: chem_ns<9>(c, mode, U, Q, rhoi, dt, maxiter, rtol, ttol, iters, tag, s, list, nlist, later, nlater); break;

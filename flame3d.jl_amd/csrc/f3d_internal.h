@@ -149,11 +149,20 @@ inline int fill_segments(int n0, long cap, long lines, int nd) {
   const int want = n > most ? most : (int)n;
   return want >= 2 * n0 ? want : n0;
 }
-// Most cells of a list pass that go to the half-wave solve (f3d_chem_rows.h):
-// two for each half wave the device holds.  A half wave has a twentieth of the
-// one-thread solve's throughput, so where slow cells are many the rest go on in
-// their threads.
-constexpr int kRowsMost = 4096;
+// Most cells of a list of n that go to the half-wave solve (f3d_chem_rows.h): two
+// for each half wave the device holds, or one in 128.  A half wave has a
+// twentieth of the one-thread solve's throughput, so where slow cells are many
+// the rest go on in their threads, and each of the two passes then takes as long
+// as its slowest cell: the list has to hold what a flow has of them.  A pass
+// over more than 2^21 cells takes longer than its slowest cell anyway; none go.
+// Surrogate step of H2/O2 reactors (1 in 230 listed cells is slow) in ms with
+// none going / at most 4096 / this rule:
+//   0.15 million listed  1.38 / 0.91 / 0.90     0.70  2.46 / 3.12 / 2.12
+//   1.21                 3.44 / 4.36 / 3.22     2.84  6.45 / 7.79 / 6.45
+constexpr int kRowsMost = 16384;
+inline int rows_most(long n) {
+  return n > 128L * kRowsMost ? 0 : n > 128L * 4096 ? (int)(n / 128) : 4096;
+}
 // Resident blocks of a kernel on the current device (queried once per context
 // and kernel; *slot keeps it).
 template <class K>

@@ -218,3 +218,40 @@ def test_single_species_has_no_diffusion_flux(d):
     torch.cuda.synchronize()
     assert int((Fd != 0).sum()) == 0 and int((Fh != 0).sum()) == 0
     ctx.close()
+
+
+@pytest.mark.parametrize("shape,stretch,maxiter,slow_over", [
+    ((48, 40, 36), 5.0, 3, 4096),        # all of a solve's iterations, more cells than may go
+    ((112, 104, 96), 1.0, 50, None),     # a list of which one cell in 128 may go, and fewer do
+    ((112, 104, 96), 5.0, 50, 8192),     # ... and more than that are slow
+    ((144, 136, 136), 1.0, 50, None)])   # a list so long that no cell goes
+def test_slow_cells_of_long_lists(shape, stretch, maxiter, slow_over):
+    """Every rejected cell equals the Newton mode's bit for bit, whether the
+    half-wave solve takes it, takes it on from a full list (from its beginning,
+    or with two substeps at once where the first step failed) or takes none."""
+    import flame3d_amd.abi as abi
+    import flame3d_amd.cases as cases
+    import flame3d_amd.mech as mm
+    import flame3d_amd.surrogate as sur
+    m = mm.load("h2_lidryer")
+    print(f"\n[long list] {shape} dt x {stretch} maxiter {maxiter}", flush=True)
+    Q, r = cases.chem_cells(shape, m, seed=7, dev="cuda")
+    dt = stretch * sur.DT
+    U = torch.zeros((5,) + tuple(Q.shape[1:]), dtype=torch.float64, device="cuda")
+    ctx = abi.Context(*shape, m, "fp64")
+    sur.attach(ctx, chain_max=1e-30, dt=dt)
+    Un, Qn, rn = U.clone(), Q.clone(), r.clone()
+    it = torch.zeros(shape[::-1], dtype=torch.int32, device="cuda")
+    ctx.chem_newton(Un, Qn, rn, dt, maxiter, iters=it)
+    st = torch.zeros(shape[::-1], dtype=torch.int8, device="cuda")
+    n = int(ctx.nn_chem(U, Q, r, dt, maxiter, status=st))
+    torch.cuda.synchronize()
+    back = st >= 2
+    slow = int((back & ((it > min(5, maxiter)) | (it < 0))).sum())
+    print(f"[long list] {n} rejected, {slow} of them slow", flush=True)
+    assert n == int(back.sum()) and n > st.numel() // 2
+    if slow_over:
+        assert slow > slow_over
+    for got, ref in ((U, Un), (Q, Qn), (r, rn)):
+        assert torch.equal(sur.interior(got)[back.flatten()], sur.interior(ref)[back.flatten()])
+    ctx.close()

@@ -27,5 +27,9 @@ def test_slow_cells_list_holds_cell_numbers_only():
     assert any(re.search(rf"hipMemset\(c->{lst}, 0, sizeof\(int32_t\) \* kRowsMost\)", u)
                for u in uses)
     assert not any("hipLaunchKernelGGL" in u for u in uses)
-    # its one writer stores cell numbers, at slots of the allocation
-    assert re.search(r"if \(slot < kRowsMost\) \{\s*later\[slot\] = \(int32_t\)id;", chem)
+    # its one writer stores cell numbers, at slots of the allocation: rows_most(n)
+    # of a list of n, at most n / 128 with n <= 128 kRowsMost, or 4096
+    assert re.search(r"if \(slot < most\) \{\s*later\[slot\] = \(int32_t\)id;", chem)
+    assert re.search(r"list, n, later, nlater, rows_most\(n\)\)", chem)
+    assert "return n > 128L * kRowsMost ? 0 : n > 128L * 4096 ? (int)(n / 128) : 4096;" in internal
+    assert int(re.search(r"constexpr int kRowsMost = (\d+);", internal).group(1)) >= 4096
