@@ -307,8 +307,9 @@ struct NasaTab {
   double emin[NS], emax[NS];  // e_k W_k / Ru at min_temp, max_temp
   double as[NS];            // (a1(low) - 1) Ru / W_k
 
-  // by every thread of the block, before any of them leaves the kernel
-  __device__ void fill(const DevParams* __restrict__ P) {
+  // by every thread of the block, before any of them leaves the kernel;
+  // fill_fits: without what only e -> T reads (emin, emax, as)
+  __device__ void fill_fits(const DevParams* __restrict__ P) {
     for (int i = threadIdx.x; i < 2 * NS; i += blockDim.x) {
       const int n = i >> 1;
       const double* c = (i & 1) ? P->hi[n] : P->lo[n];
@@ -324,6 +325,9 @@ struct NasaTab {
       q.c6 = c[6];
     }
     __syncthreads();
+  }
+  __device__ void fill(const DevParams* __restrict__ P) {
+    fill_fits(P);
     for (int n = threadIdx.x; n < NS; n += blockDim.x) {
       emin[n] = energy_poly(n, P->min_temp, P->sep[n]);
       emax[n] = energy_poly(n, P->max_temp, P->sep[n]);

@@ -705,7 +705,9 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))
   const long id = gid();  // a wave holds the 64 cells of one tile
   const long NP = g.NP;
   int code = (id < ncell) ? status[id] : 0;
-  if (__syncthreads_or(code == 1)) N.fill(P);
+  const bool res_on = C->res_tol > 0.0f || C->res_T_tol > 0.0f;
+  const bool rates = res_on || C->chi_max > 0.0f || C->chain_max > 0.0f;
+  if (rates && __syncthreads_or(code == 1)) N.fill_fits(P);
   if (code == 1) {
     const int a = (int)(id % g.Nx);
     const int t = (int)(id / g.Nx);
@@ -718,8 +720,7 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))
     const double rhoc = fmax(Q[p], kEps);
     // 5. backward-Euler residual at (rho', T'): its largest species entry,
     //    and the temperature error its formation energies imply
-    const bool res_on = C->res_tol > 0.0f || C->res_T_tol > 0.0f;
-    if (res_on || C->chi_max > 0.0f || C->chain_max > 0.0f) {
+    if (rates) {
       double sc[NS], wdot[NS], Adum[NS][NS], Mc[3][3];
 #pragma unroll
       for (int n = 0; n < NS; ++n) sc[n] = rn[n] * P->cmw[n];
@@ -953,11 +954,15 @@ static int nn_partials(f3d_ctx* c, long tiles) {
   return F3D_OK;
 }
 
-// The gate kernel's instance: constant carriers with the compiled-in tables
-// when the configuration names the carriers the shipped networks gate on (H,
-// O, OH of the hydrogen mechanism, O of air), else the run-time reaction loop:
-// with constant tables, run-time carriers put three tests on every species of
-// every unrolled reaction (180 KB of code, half of it scalar).
+// The gate kernel's instance: the compiled-in tables with constant carriers when
+// the configuration names those the shipped networks gate on (H, O, OH of the
+// hydrogen mechanism, O of air): run-time carriers put three tests on every
+// species of every unrolled reaction (180 KB of code, half of it scalar).  For
+// the hydrogen mechanism that is still faster than the run-time reaction loop,
+// for the air mechanism's few reactions it is not.  Prediction and gate of a
+// 192x128x128 H2/air mixing layer: 0.63 ms with the shipped carriers, 1.33 with
+// H and OH (1.45 in the loop), 1.11 with H alone (1.30); of 128x96x64 air
+// reactors with O2 and O 123 us (124 in the loop), with three carriers 142 (134).
 static bool nn_carriers(const f3d_ctx* c, int a, int b, int d) {
   return c->nn_chain[0] == a && c->nn_chain[1] == b && c->nn_chain[2] == d;
 }
@@ -1307,6 +1312,8 @@ int f3d_nn_chem(f3d_ctx* c, double* U, double* Q, double* rhoi, double dt, int32
     launch_pred<9>(c, Q, rhoi, st, s);
     if (c->kin_table == F3D_KIN_H2_LIDRYER && nn_carriers(c, 3, 4, 5))
       launch_gate<9, KinCT<MechH2LiDryer>>(c, U, Q, rhoi, dt, st, s, CarrierCT<3, 4, 5>());
+    else if (c->kin_table == F3D_KIN_H2_LIDRYER)
+      launch_gate<9, KinCT<MechH2LiDryer>>(c, U, Q, rhoi, dt, st, s, nn_carriers_rt(c));
     else
       launch_gate<9, KinRT>(c, U, Q, rhoi, dt, st, s, nn_carriers_rt(c));
   } else {

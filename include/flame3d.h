@@ -243,7 +243,8 @@ typedef struct {
                             root while a near-root with a tiny residual exists);
                             <= 0: off */
   int32_t chain_species; /* bitmask of the (at most 3) chain-carrier species, bit k =
-                            species k (H2/O2: H, O, OH) */
+                            species k (H2/O2: H, O, OH; with these, or O of air, the
+                            gate has constants and is faster than with others) */
   float boxcox_lambda;
   int32_t label_mode;    /* outputs: 0 dY_k; 1 d BoxCox(Y_k) (post_predict form,
                             Y' = (lambda (BoxCox(Y) + out) + 1)^(1/lambda));

@@ -626,3 +626,80 @@ def test_train_on_integrator_data():
     print(f"  held-out mse {l0:.3e} -> {l1:.3e}", flush=True)
     assert l1 < 0.35 * l0  # 30 epochs on 15k samples: a fourfold drop
     ctx.close()
+
+
+@pytest.mark.parametrize("mech,chain,cmax,tables", [
+    ("h2_lidryer", ("H", "OH"), 0.02, True), ("h2_lidryer", ("H", "OH"), 0.02, False),
+    ("h2_lidryer", ("H2O", "H", "OH"), 0.1, True), ("h2_lidryer", ("H", "O", "OH"), 0.1, False),
+    ("h2_lidryer", ("H2O", "OH", "HO2"), 0.01, True),
+    ("air5", ("N", "O"), 2e-4, True), ("air5", ("N", "O"), 2e-4, False),
+    ("air5", ("N", "NO", "O"), 2e-4, True), ("air5", ("O",), 1e-4, False)])
+def test_nn_chem_chain_gate_of_other_carriers(mech, chain, cmax, tables):
+    """test_nn_chem_chain_gate for carriers that the shipped networks do not
+    gate on and (tables False) for a mechanism that is not a compiled-in one (a
+    rate constant moved by 1e-7 of itself): reactors with traces of every
+    species, identity prediction, only the chain gate on; judged with
+    the oracle's analytic Jacobian (mass action and [M], the falloff factor held
+    fixed, as the gate has it), cells within 1e-3 of the threshold left out."""
+    import dataclasses
+    import flame3d_amd.cases as cases
+    import flame3d_amd.mech as mm
+    abi = _abi()
+    from oracle import Oracle
+    size = (9, 8, 7)
+    m = mm.load(mech)
+    if not tables:
+        A = np.array(m.Arr, copy=True)
+        A[0, 0] *= 1.0 + 1e-7
+        m = dataclasses.replace(m, Arr=A)
+    h2 = mech == "h2_lidryer"
+    dt = 1e-7 if h2 else 6e-9
+    Q, r = (cases.chem_cells if h2 else cases.chem_cells_air)(size, m, seed=44)
+    g = torch.Generator().manual_seed(5)
+    Y = r / Q[0] + 10.0 ** (-6.0 + 5.0 * torch.rand(r.shape, generator=g, dtype=torch.float64))
+    z = torch.zeros_like(Q[0])
+    Q, r = cases.state_from_TPY(m, Q[5], Q[4], Y / Y.sum(0), z, z, z)
+    U = cases.prim2c(Q).cuda().contiguous()
+    Q, r = Q.cuda().contiguous(), r.cuda().contiguous()
+    ctx = abi.Context(*size, m, "fp64")
+    assert (ctx.kinetics_source() != abi.KIN_RUNTIME) == tables
+    cfg = abi.NNConfig()
+    for k in range(m.Ns + 2):
+        cfg.in_std[k] = 1.0
+    for k in range(m.Ns):
+        cfg.out_std[k] = 1.0
+    idx = [m.index(x) for x in chain]
+    cfg.d_max, cfg.elem_tol, cfg.neg_tol, cfg.res_tol = 1e30, 1e30, 1.0, 0.0
+    cfg.chain_max, cfg.chain_species = cmax, sum(1 << k for k in idx)
+    cfg.boxcox_lambda, cfg.dt = 0.1, dt
+    ctx.nn_init(cfg)
+    ctx.nn_set_params(np.zeros(12512, np.float32))  # identity prediction dY = 0
+    Qn, rn, Un = Q.clone(), r.clone(), U.clone()
+    ctx.chem_newton(Un, Qn, rn, dt, 50, 1e-10, 1e-6)
+    q0, r0 = _interior(Q), _interior(r)
+    st = torch.zeros(size[::-1], dtype=torch.int8, device="cuda")
+    nfb = ctx.nn_chem(U, Q, r, dt, 50, 1e-10, 1e-6, status=st)
+    torch.cuda.synchronize()
+    s = st.cpu().numpy().reshape(-1)
+    assert nfb == int((s >= 2).sum()) and 0 < nfb < s.size
+    assert set(np.unique(s).tolist()) <= {1, 8}  # only the chain gate is active
+    q1, r1, qn, rnn = _interior(Q), _interior(r), _interior(Qn), _interior(rn)
+    rej = s == 8
+    assert np.array_equal(q1[rej], qn[rej]) and np.array_equal(r1[rej], rnn[rej])
+    orc = Oracle(*size, m)
+    mw = np.asarray(m.mw)
+    checked = 0
+    for c in range(0, s.size, 3):
+        rho = q0[c, 0]
+        rr = np.maximum(r0[c], 0)
+        rr = rr * (rho / rr.sum())
+        T = orc.get_T_from(q0[c, 6], rr, q0[c, 5])
+        sc = rr / mw * 1e-6
+        J = orc.production_rate(sc, T, full_jac=True)[1]
+        lam = np.linalg.eigvals(dt * J[np.ix_(idx, idx)]).real.max()
+        if abs(lam / cmax - 1) < 1e-3:
+            continue
+        assert (s[c] == 1) == (lam < cmax), (c, lam, s[c])
+        checked += 1
+    assert checked > s.size // 4
+    ctx.close()
