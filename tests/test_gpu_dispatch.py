@@ -255,3 +255,33 @@ def test_slow_cells_of_long_lists(shape, stretch, maxiter, slow_over):
     for got, ref in ((U, Un), (Q, Qn), (r, rn)):
         assert torch.equal(sur.interior(got)[back.flatten()], sur.interior(ref)[back.flatten()])
     ctx.close()
+
+
+@pytest.mark.parametrize("a", [0, 1, 2, 3])
+@pytest.mark.parametrize("b", [0, 1, 2, 3])
+def test_fill_all_pairs(a, b):
+    """All 16 ordered pairs of fill kinds of a direction's two faces, in each
+    direction, on the smallest extents (4): with both faces in one launch, in
+    turn, or one of them kept; equal bit for bit."""
+    import flame3d_amd.abi as abi
+    import flame3d_amd.mech as mm
+    from oracle import Oracle
+    m = mm.load("air5")
+    shape = (4, 4, 4)
+    _, Q, rhoi = _state(shape, m)
+    orc, ctx = Oracle(*shape, m), abi.Context(*shape, m, "fp64")
+    inQ = [1.2, 300.0, 1.0, -2.0, 1.0e5, 310.0, 2.0e5]
+    inr = list(np.linspace(0.1, 0.2, m.Ns))
+    for d in range(3):
+        kinds = [2, 1, 1, 2, 3, 0]
+        kinds[2 * d:2 * d + 2] = [a, b]
+        Qo, ro = to_np(Q), to_np(rhoi)
+        Uo = orc.prim2c(Qo)
+        Qg, rg, Ug = Q.cuda(), rhoi.cuda(), to_torch(Uo)
+        orc.fill(kinds, Qo, Uo, ro, inQ, inr)
+        ctx.set_boundary(kinds, inQ, inr)
+        ctx.fill(Qg, Ug, rg)
+        torch.cuda.synchronize()
+        for got, ref in ((Qg, Qo), (Ug, Uo), (rg, ro)):
+            assert np.array_equal(to_np(got), ref), kinds
+    ctx.close()
