@@ -39,15 +39,7 @@ constexpr int kNewtonMaxSub = 64;
 // of a flame's cells would go.
 constexpr int kNewtonFirst = 5;
 
-// One backward-Euler solve over h of the reactor (rho_k, T) from (r, T),
-// total energy fixed at E0: Newton on
-//   F_k = rho_k - rs_k - h W_k wdot_k(rho, T) = 0,  F_E = E(rho, T) - E0 = 0
-// with the exact mass-action Jacobian (+ third-body terms) and the analytic
-// temperature derivative of the rates.  Constant quotients (1e-6/W_n,
-// W_n/W_l, Ru/W_n, 1/W_n, the reverse rates' 1/RsT, the pivots' reciprocals)
-// are multiplied where the reference's point-implicit step divides.  Returns false when the iterate leaves the admissible set
-// (non-finite, T outside [T_lo, T_hi], rho_k < -rho_tot) or maxiter
-// iterations pass without convergence; `it` counts the iterations taken.
+// the parameter block by scalar loads
 typedef const __attribute__((address_space(4))) DevParams ConstParams;
 
 // Per-lane values that an iteration needs now and then live in LDS (the
@@ -66,6 +58,16 @@ struct GibbsLds {
   __device__ double h(int m) const { return L.h[m][lane]; }
 };
 
+// One backward-Euler solve over h of the reactor (rho_k, T) from (r, T),
+// total energy fixed at E0: Newton on
+//   F_k = rho_k - rs_k - h W_k wdot_k(rho, T) = 0,  F_E = E(rho, T) - E0 = 0
+// with the exact mass-action Jacobian (+ third-body terms) and the analytic
+// temperature derivative of the rates.  Constant quotients (1e-6/W_n,
+// W_n/W_l, Ru/W_n, 1/W_n, the reverse rates' 1/RsT, the pivots' reciprocals)
+// are multiplied where the reference's point-implicit step divides.  Returns
+// false when the iterate leaves the admissible set (non-finite, T outside
+// [T_lo, T_hi], rho_k < -rho_tot) or maxiter iterations pass without
+// convergence; `it` counts the iterations taken.
 template <int NS, class K>
 __device__ inline bool be_solve(const NasaTab<NS>& N, NewtonLds<NS>& L, int lane,
                                 const DevParams* __restrict__ P0, double (&r)[NS], double& T,

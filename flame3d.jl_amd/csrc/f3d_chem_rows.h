@@ -495,9 +495,11 @@ __device__ inline bool be_rows(const NasaTab<T::NS>& N, RowsLds<T>& L, int grp, 
     }
     // gauss_solve<N1, true, kInert>: a row stays in its lane, pos is its place
     // after the exchanges (rows that were pivots go on being updated, unread).
-    // The pivot is the entry of the largest upper word; equal upper words (and
-    // entries that are not numbers) take the comparison in full and then, as
-    // the exchanges do, the first place.
+    // The pivot is the entry of the largest upper word; equal upper words take
+    // the comparison in full and then, as the exchanges do, the first place.
+    // (An entry that is not a number has the largest upper word and is taken,
+    // where the exchanges would pass it over; with either the update is not a
+    // number and the solve fails.)
     int pos = l < N1 ? l : 99;
     row_eliminate<T, 0>(L, grp, l, pos, a, b);
     if (pos == N1 - 1) {

@@ -138,11 +138,12 @@ inline int small_block(long n) { return n <= 1024 * 64 ? 64 : kBlock; }
 // Segments per line of a march over nd cells or faces: n0, or more where a
 // launch of n0 `lines` blocks leaves half of the device's resident block slots
 // (cap) empty.  A march is a chain of dependent steps, so on a block too small
-// to fill the chip its time is the longest chain, and shorter segments (4 at
-// least, below which the priming rows are most of the work) run side by side
-// instead: the FP32 right-hand side of 97x61x43 cells 603 -> 265 us.  Up to
-// half full the longer segments' fewer priming rows win (256^3 viscous sweep,
-// 5 instead of 4 segments: 1 % slower).
+// to fill the chip its time is the longest chain, and shorter segments (at most
+// one for every four cells: below that the priming rows are most of the work;
+// the callers' equal lengths, rounded up, can leave a line's last one shorter or
+// empty) run side by side instead: the FP32 right-hand side of 97x61x43 cells
+// 603 -> 265 us.  Up to half full the longer segments' fewer priming rows win
+// (256^3 viscous sweep, 5 instead of 4 segments: 1 % slower).
 inline int fill_segments(int n0, long cap, long lines, int nd) {
   const long n = cap / (lines < 1 ? 1 : lines);
   const int most = nd / 4 < 1 ? 1 : nd / 4;

@@ -262,8 +262,11 @@ __global__ void __launch_bounds__(64)
 // fluxes of its points in LDS (dynamic: a short line's block takes less, so
 // more of them are resident).  Lines shorter than 129 cells leave threads for
 // two to four groups of variables side by side.  The line's last face is
-// shared out over the block's threads, one variable each.  128^3, 9 species:
-// 195 us, against 182 us (splits) + 370 us (reconstruction) in four launches.
+// shared out over the block's threads, one variable each.  128^3, 9 species: 139
+// us on the initial mixing layer and 173 on average over a step's stages (more
+// faces take WENO), against 182 us (splits) + 370 us (reconstruction) in four
+// launches; 256^3, where 61 KB a block leave two of them to a compute unit: 1.27
+// ms and 2.08.
 constexpr int kFuseSeg = 256;
 template <int NS>
 __global__ void __launch_bounds__(kFuseSeg)

@@ -384,7 +384,8 @@ int f3d_time_step(f3d_ctx* ctx, double* U, double* Un, double* rhoi, double* rho
 int f3d_nan_check(f3d_ctx* ctx, const double* U, int32_t* flag, hipStream_t s);
 /* Device pointer of a context-owned intermediate after f3d_rk3_stage, by
  * name ("Yi", "lambda", "mu", "D", "phi", "Fx", "Fy", "Fz", "Fvx", ...,
- * "Fhz"); NULL if unknown. */
+ * "Fhz"; "Fp", "Fm", "Fp_i", "Fm_i": the split fluxes of the last direction,
+ * z, which a fused float stage does not form); NULL if unknown. */
 void* f3d_workspace(f3d_ctx* ctx, const char* name);
 
 #ifdef __cplusplus
