@@ -349,15 +349,22 @@ struct NasaTab {
 };
 
 // a / b for a constant b > 0 of the parameter block with rb = 1 / b rounded:
-// one Newton correction of a rb by its exact remainder (a product and two fused
-// multiply-adds) and the division's own last instruction, which puts back what
-// an infinite a gives (its remainder is not a number): four instructions of
-// full rate instead of a division's eleven.  The result is the rounded quotient
-// unless that lies within 2^-51 ulp of a rounding boundary (or a is so small
-// that the remainder is subnormal).
+// one Newton correction of a rb by its exact remainder, a product and two fused
+// multiply-adds of full rate instead of a division's eleven instructions.  The
+// result is the rounded quotient unless that lies within 2^-51 ulp of a rounding
+// boundary (or a is so small that the remainder is subnormal); an infinite a,
+// whose remainder is not a number, gives NaN.
 __device__ __forceinline__ double div_const(double a, double b, double rb) {
   const double q = a * rb;
-  return __builtin_amdgcn_div_fixup(fma(fma(-q, b, a), rb, q), b, a);
+  return fma(fma(-q, b, a), rb, q);
+}
+// the same with the division's own last instruction, which puts back what an
+// infinite a gives: for what is formed once per call.  (In the e -> T updates an
+// infinite density leaves nothing but NaN with true divisions as well: get_T_start
+// has returned, or its start is NaN.  There it would cost 3 % of the
+// point-implicit air step.)
+__device__ __forceinline__ double div_const_any(double a, double b, double rb) {
+  return __builtin_amdgcn_div_fixup(div_const(a, b, rb), b, a);
 }
 
 // InternalEnergy, thermo.jl:219-228, and CV, thermo.jl:194-203 (FP64), at the
@@ -412,7 +419,7 @@ __device__ inline double pmixture(const DevParams* P, double T, const double* rh
   double YOW = 0;
 #pragma unroll
   for (int n = 0; n < NS; ++n)
-    YOW += RCP ? rhoi[n] * P->rmw[n] : div_const(rhoi[n], P->mw[n], P->rmw[n]);
+    YOW += RCP ? rhoi[n] * P->rmw[n] : div_const_any(rhoi[n], P->mw[n], P->rmw[n]);
   return P->Ru * T * YOW;
 }
 
@@ -425,8 +432,8 @@ __device__ inline bool get_T_start(const NasaTab<NS>& N, const DevParams* P, dou
   double emin = 0, emax = 0, As = 0;
 #pragma unroll
   for (int n = 0; n < NS; ++n) {
-    emin += div_const(rhoi[n] * N.emin[n], P->mw[n], P->rmw[n]);
-    emax += div_const(rhoi[n] * N.emax[n], P->mw[n], P->rmw[n]);
+    emin += div_const_any(rhoi[n] * N.emin[n], P->mw[n], P->rmw[n]);
+    emax += div_const_any(rhoi[n] * N.emax[n], P->mw[n], P->rmw[n]);
     As += N.as[n] * rhoi[n];
   }
   emin *= P->Ru;

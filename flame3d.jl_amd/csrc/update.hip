@@ -197,7 +197,7 @@ __global__ void __launch_bounds__(kBlock)
     Y[n] = fmax((R)rhoi[p + (long)n * NP] * rinv, R(0));
     Yi[p + (long)n * NP] = Y[n];
     if constexpr (sizeof(R) == 8)
-      X[n] = div_const(Y[n], P->mw[n], P->rmw[n]);
+      X[n] = div_const_any(Y[n], P->mw[n], P->rmw[n]);
     else
       X[n] = Y[n] / PT<R>::mw(P, n);
     YOW += X[n];
