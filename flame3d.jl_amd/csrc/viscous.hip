@@ -39,8 +39,11 @@ struct Metrics {
 // waves it saves registers and waits in between): 128^3, 153-168 us per launch
 // to 132-150 us, and 13.8 to 4.9 us on a 24x16x12 block.
 // The y direction takes its lines y by y, so that the next line's stencil is
-// this one's moved by a point (200x100x100: 131 us, 141 in slab order, 132 with
-// four waves of the earlier form); the others in slab order.
+// this one's moved by a point (200x100x100: 131 us, 141 in slab order), up to
+// planes of 65536 points, beyond which the stencil's z neighbours have left the
+// L2 when they come round again (512x256x256: 2.46 ms, 2.20 in slab order;
+// 256x256x256 1.12, 1.11); the others in slab order.
+constexpr int kPlaneMost = 65536;
 template <typename R, typename MT, int dir>
 __global__ void __launch_bounds__(kBlock)
     __attribute__((amdgpu_waves_per_eu(sizeof(R) == 8 ? 2 : 1, sizeof(R) == 8 ? 2 : 8)))
@@ -54,7 +57,7 @@ __global__ void __launch_bounds__(kBlock)
   const int a = (int)(id % nx);
   const int tt = (int)(id / nx);
   int b, c;
-  if (dir == 1) {
+  if (dir == 1 && g.Nxt * g.Nyt <= kPlaneMost) {
     b = tt % ny;
     c = tt / ny;
   } else {

@@ -285,3 +285,25 @@ def test_fill_all_pairs(a, b):
         for got, ref in ((Qg, Qo), (Ug, Uo), (rg, ro)):
             assert np.array_equal(to_np(got), ref), kinds
     ctx.close()
+
+
+@pytest.mark.parametrize("shape", [(248, 248, 4), (249, 248, 5)])
+def test_viscous_faces_at_the_plane_limit(shape):
+    """FP64 viscous faces on the largest x-y plane that the y direction takes y
+    by y (65536 points) and on one that it takes in slabs: 1e-12 normwise."""
+    import flame3d_amd.abi as abi
+    import flame3d_amd.mech as mm
+    from oracle import Oracle
+    m = mm.load("air5")
+    grid, Q, rhoi = _state(shape, m)
+    M, J = [to_np(x) for x in grid.metrics], to_np(grid.J)
+    ctx, orc = abi.Context(*shape, m, "fp64"), Oracle(*shape, m)
+    Qg, Mg, Jg = Q.cuda(), [x.cuda() for x in grid.metrics], grid.J.cuda()
+    lam, mu = ctx.zeros() + 0.05, ctx.zeros() + 2e-5
+    for d in range(3):
+        Fv, Fh = ctx.face_zeros(d, 4), ctx.face_zeros(d, 3)
+        ctx.viscous_flux(d, Fv, Qg, Mg, Jg, lam, mu, Fh)
+        torch.cuda.synchronize()
+        ref = orc.viscous_flux(d, to_np(Q), M, J, to_np(lam), to_np(mu), to_np(Fh))
+        assert rel_err(to_np(Fv), ref) < 1e-12, d
+    ctx.close()
